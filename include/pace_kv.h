@@ -115,6 +115,23 @@ int pace_kv_move(const void* const* src_layers, int64_t src_pool_pages,
                  int32_t* err_count, void* stream);
 
 /*
+ * MOVE THROUGH A BUFFER: the bytes of PACK into `buffer` followed by UNPACK
+ * out of it, in chunks of buffer_layers layers (the buffer holds buffer_layers
+ * layers of buffer_layer_stride bytes; with fewer than num_layers, it keeps
+ * each slot's last chunk).  Each page is read once and written to the buffer
+ * and to its destination by the same launch; pools (or a buffer) that share
+ * memory are packed and unpacked in two launches per chunk, so a destination
+ * page may be a source page of the same chunk.  err_count counts as the two
+ * calls do.
+ */
+int pace_kv_move_buffered(const void* const* src_layers, int64_t src_pool_pages,
+                          const int32_t* src_ids, void* buffer,
+                          int64_t buffer_layer_stride, int buffer_layers,
+                          void* const* dst_layers, int64_t dst_pool_pages,
+                          const int32_t* dst_ids, int num_layers, int64_t n_pages,
+                          int64_t page_bytes, int32_t* err_count, void* stream);
+
+/*
  * SWAP OUT / SWAP IN between a device pool and a host-resident pool of pages
  * in pinned memory (hipHostMalloc / torch pin_memory), in one kernel that
  * reads or writes the host pages across PCIe directly (no staging buffer):
@@ -399,9 +416,8 @@ int pace_kv_promoter_destroy(pace_kv_promoter* promoter);
 /*
  * One-call promotion of a batch: pace_kv_plan, one host-to-device copy of
  * both id lists on `stream`, then the page movement: with buffer == NULL a
- * fused pace_kv_move; otherwise pace_kv_pack into `buffer` followed by
- * pace_kv_unpack, in chunks of buffer_layers layers (the buffer holds
- * buffer_layers layers of buffer_layer_stride bytes).  out_dst_tables is as in
+ * fused pace_kv_move; otherwise pace_kv_move_buffered through `buffer` (which
+ * holds buffer_layers layers of buffer_layer_stride bytes).  out_dst_tables is as in
  * pace_kv_plan.  On failure no destination page stays allocated.
  *
  * Replaces KVhelper.get_kv_cache + BaseWorker._insert_kv_cache for requests

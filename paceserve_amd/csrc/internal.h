@@ -41,20 +41,36 @@ struct Side {
 // finds them in the memory-side cache.
 enum class StorePolicy { kStream, kPack };
 
+// A second destination of a copy with ids on both sides: page j of layer l
+// also goes to base + l * layer_stride + j * page_bytes.
+struct Tee {
+  char* base;
+  int64_t layer_stride;
+};
+
 // Validates arguments and enqueues the copy dst[l][dst_id(j)] = src[l][src_id(j)]
 // for l < num_layers, j < n_pages on `stream`, in launches of at most
 // PACE_KV_MAX_LAYERS_PER_LAUNCH layers.  host_src_ids / host_dst_ids (host
 // arrays, n_pages <= PACE_KV_INLINE_IDS) replace the sides' device ids and
-// travel in the kernel arguments.
-
+// travel in the kernel arguments.  With a tee the pools and its buffer must
+// not share memory.
 int launch_page_copy(const Side& src, const Side& dst, int num_layers,
                      int64_t n_pages, int64_t page_bytes, int32_t* err_count,
                      hipStream_t stream, const int32_t* host_src_ids = nullptr,
                      const int32_t* host_dst_ids = nullptr,
-                     StorePolicy policy = StorePolicy::kStream);
+                     StorePolicy policy = StorePolicy::kStream, const Tee* tee = nullptr);
+
+// src -> buffer -> dst in chunks of buffer_layers layers: the bytes of a pack
+// into `buffer` and an unpack out of it, which stays filled.  One launch per
+// chunk reads each page once and writes it to both, unless source, buffer and
+// destination share memory.  Ids as in launch_page_copy; the caller has
+// checked page_bytes, buffer_layers >= 1 and the buffer's stride.
+int buffered_copy(const Side& src, const Side& dst, char* buffer, int64_t buffer_layer_stride, int buffer_layers,
+                  int num_layers, int64_t n_pages, int64_t page_bytes, int32_t* err_count, hipStream_t stream,
+                  const int32_t* host_src_ids = nullptr, const int32_t* host_dst_ids = nullptr);
 
 // Builds the layer table of a contiguous buffer [num_layers][layer_stride].
 void buffer_layers(const void* base, int64_t layer_stride, int num_layers,
-                   const char** out);
+                      const char** out);
 
 }  // namespace pace_kv

@@ -28,6 +28,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "internal.h"
@@ -60,7 +61,14 @@ struct CopyParams {
   uint32_t page_vecs;      // page_bytes / 16
   uint32_t rows_per_page;  // ceil(page_bytes / kRowBytes)
   uint32_t rows_log2;      // log2(rows_per_page) when that is a power of two
+  char* tee;               // Kind::kTee: page j of layer l also goes to tee + l * tee_stride + j * page_bytes
+  int64_t tee_stride;
 };
+
+// What a launch copies: kStream (unpack, move, swap), kPack (into a transfer
+// buffer that an unpack reads next), kTee (a move that also leaves the pages
+// in a transfer buffer).
+enum Kind { kStream = 0, kPack = 1, kTee = 2 };
 
 // Page ids carried in the kernel arguments (small promotions): no device id
 // array, so no upload has to precede the launch.
@@ -88,18 +96,46 @@ __device__ __forceinline__ uint32_t page_of(const int32_t* ids, uint32_t j) {
 // asm, so the asm carries them (s_nop 1: two wait states).  Without them a
 // variant that computed its next address into the stored registers wrote
 // wrong data.
-template <bool PACK>
+template <bool CACHED>
 __device__ __forceinline__ void store_vec(const u32x4 v, u32x4* d) {
-  if (PACK) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(d), "v"(v) : "memory");
+  if (CACHED) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(d), "v"(v) : "memory");
   else asm volatile("global_store_dwordx4 %0, %1, off nt sc1\n\ts_nop 1" : : "v"(d), "v"(v) : "memory");
+}
+
+// The tee's copy of one vector: pool page sp to page j of the transfer buffer
+// and to pool page dp, from one read.  The same bytes and the same counts as a
+// pack followed by an unpack, including a source id outside its pool, where
+// the pack leaves the buffer's page as it was and the unpack copies that.
+//
+// Bound by HBM, and by its writes: 3 bytes of traffic per payload byte, two of
+// them written, against the 4 of a pack and an unpack.  Measured on MI355X
+// against those two launches: 512 MiB of 64 KiB pages 259 us (6.2 TB/s) against
+// 300-310; 2.8 GB of 8 KiB pages, 80 layers, 1.47 ms against 1.79.  Of the
+// shapes and policies tried, one wave per 1 KiB row with streaming stores and
+// plain loads is the fastest: cacheable buffer stores cost 0.5%, cacheable
+// stores on both sides 4-7%, nontemporal loads 0.5-1%, the destination store
+// first 0.2-1%; 128 threads are 0.5% faster on 512 MiB and 2% slower on 2.8 GB,
+// 256 and 512 threads slower on both.
+__device__ __forceinline__ void tee_row(const CopyParams& p, uint32_t j, uint32_t layer, uint32_t row,
+                                        uint32_t vec, uint32_t sp, uint32_t dp) {
+  u32x4* buf = reinterpret_cast<u32x4*>(p.tee + layer * p.tee_stride + static_cast<int64_t>(j) * p.page_bytes) + vec;
+  const bool src_ok = sp < p.src_pool_pages, dst_ok = dp < p.dst_pool_pages;
+  if (!(src_ok && dst_ok) && row == 0 && threadIdx.x == 0 && p.err != nullptr)
+    atomicAdd(p.err, static_cast<int>(!src_ok) + static_cast<int>(!dst_ok));
+  const u32x4* s = src_ok ? reinterpret_cast<const u32x4*>(p.src[layer] + static_cast<int64_t>(sp) * p.page_bytes) + vec
+                          : buf;
+  const u32x4 v = *s;
+  if (src_ok) store_vec<false>(v, buf);
+  if (dst_ok)
+    store_vec<false>(v, reinterpret_cast<u32x4*>(p.dst[layer] + static_cast<int64_t>(dp) * p.page_bytes) + vec);
 }
 
 // The copy of one 1 KiB row: item blockIdx.x (page j, row r of it) of layer
 // blockIdx.y; the grid is exactly (rows x pages) x layers.  POW2: the page has
 // a power-of-two number of rows.  sids / dids are the sides' page ids (device
 // or kernel-argument arrays), nullptr for a contiguous side.  Loads are
-// always nontemporal; PACK selects the pack's store policy (store_vec).
-template <bool GUARD, bool PACK, bool POW2>
+// nontemporal but in a tee; KIND selects the store policy (store_vec) and the tee.
+template <bool GUARD, Kind KIND, bool POW2>
 __device__ __forceinline__ void copy_row(const CopyParams& p, const int32_t* sids,
                                          const int32_t* dids) {
   const uint32_t x = blockIdx.x;
@@ -119,11 +155,15 @@ __device__ __forceinline__ void copy_row(const CopyParams& p, const int32_t* sid
       if (row == 0 && threadIdx.x == 0 && p.err != nullptr) atomicAdd(p.err, 1);
       return;
     }
-    store_vec<PACK>(v, reinterpret_cast<u32x4*>(p.dst[layer] + static_cast<int64_t>(dp) * p.page_bytes) + vec);
+    store_vec<KIND == kPack>(v, reinterpret_cast<u32x4*>(p.dst[layer] + static_cast<int64_t>(dp) * p.page_bytes) + vec);
     return;
   }
   const uint32_t sp = static_cast<uint32_t>(sids[j]);
   const uint32_t dp = page_of(dids, j);
+  if (KIND == kTee) {
+    tee_row(p, j, layer, row, vec, sp, dp);
+    return;
+  }
   // Negative ids wrap to large unsigned values and fail the same test.
   if (sp >= p.src_pool_pages || dp >= p.dst_pool_pages) {
     if (row == 0 && threadIdx.x == 0 && p.err != nullptr) atomicAdd(p.err, 1);
@@ -131,29 +171,29 @@ __device__ __forceinline__ void copy_row(const CopyParams& p, const int32_t* sid
   }
   const u32x4 v = __builtin_nontemporal_load(
       reinterpret_cast<const u32x4*>(p.src[layer] + static_cast<int64_t>(sp) * p.page_bytes) + vec);
-  store_vec<PACK>(v, reinterpret_cast<u32x4*>(p.dst[layer] + static_cast<int64_t>(dp) * p.page_bytes) + vec);
+  store_vec<KIND == kPack>(v, reinterpret_cast<u32x4*>(p.dst[layer] + static_cast<int64_t>(dp) * p.page_bytes) + vec);
 }
 
 // GUARD: page_bytes is not a multiple of kRowBytes, so the last row of a page
 // is partial.
-template <bool GUARD, bool PACK, bool POW2>
+template <bool GUARD, Kind KIND, bool POW2>
 __global__ __launch_bounds__(kThreads) void page_copy_kernel(const CopyParams p) {
-  copy_row<GUARD, PACK, POW2>(p, p.src_ids, p.dst_ids);
+  copy_row<GUARD, KIND, POW2>(p, p.src_ids, p.dst_ids);
 }
 
 // Same copy with the ids in the kernel arguments.  A side whose ids are not
 // inline (the contiguous buffer of a pack or unpack) indexes pages by
 // position.
-template <bool GUARD, bool PACK, bool POW2, bool SRC_INLINE, bool DST_INLINE>
+template <bool GUARD, Kind KIND, bool POW2, bool SRC_INLINE, bool DST_INLINE>
 __global__ __launch_bounds__(kThreads) void page_copy_inline_kernel(const CopyParamsInline p) {
-  copy_row<GUARD, PACK, POW2>(p.base, SRC_INLINE ? p.src_ids : nullptr,
+  copy_row<GUARD, KIND, POW2>(p.base, SRC_INLINE ? p.src_ids : nullptr,
                               DST_INLINE ? p.dst_ids : nullptr);
 }
 
-template <bool GUARD, bool PACK, bool POW2>
+template <bool GUARD, Kind KIND, bool POW2>
 hipError_t launch_t(const CopyParams& p, dim3 grid, hipStream_t stream) {
   void* args[] = {const_cast<CopyParams*>(&p)};
-  return hipLaunchKernel(reinterpret_cast<const void*>(&page_copy_kernel<GUARD, PACK, POW2>), grid,
+  return hipLaunchKernel(reinterpret_cast<const void*>(&page_copy_kernel<GUARD, KIND, POW2>), grid,
                          dim3(kThreads), args, 0, stream);
 }
 
@@ -161,37 +201,41 @@ hipError_t launch_t(const CopyParams& p, dim3 grid, hipStream_t stream) {
 // only (unpack).
 enum InlineSides { kBothInline = 0, kSrcInline = 1, kDstInline = 2 };
 
-template <bool GUARD, bool PACK, bool POW2, int SIDES>
+template <bool GUARD, Kind KIND, bool POW2, int SIDES>
 hipError_t launch_inline_t(const CopyParamsInline& p, dim3 grid, hipStream_t stream) {
   void* args[] = {const_cast<CopyParamsInline*>(&p)};
   constexpr bool kS = SIDES != kDstInline, kD = SIDES != kSrcInline;
   return hipLaunchKernel(
-      reinterpret_cast<const void*>(&page_copy_inline_kernel<GUARD, PACK, POW2, kS, kD>), grid,
+      reinterpret_cast<const void*>(&page_copy_inline_kernel<GUARD, KIND, POW2, kS, kD>), grid,
       dim3(kThreads), args, 0, stream);
 }
 
 using LaunchFn = hipError_t (*)(const CopyParams&, dim3, hipStream_t);
 using LaunchInlineFn = hipError_t (*)(const CopyParamsInline&, dim3, hipStream_t);
 
-// Instances indexed [GUARD][PACK][POW2] (and [SIDES] for inline ids).
-constexpr LaunchFn kLaunch[2][2][2] = {
-    {{launch_t<false, false, false>, launch_t<false, false, true>},
-     {launch_t<false, true, false>, launch_t<false, true, true>}},
-    {{launch_t<true, false, false>, launch_t<true, false, true>},
-     {launch_t<true, true, false>, launch_t<true, true, true>}}};
+// Instances indexed [GUARD][KIND][POW2] (and [SIDES] for inline ids; a tee
+// has ids on both sides).
+constexpr LaunchFn kLaunch[2][3][2] = {
+    {{launch_t<false, kStream, false>, launch_t<false, kStream, true>},
+     {launch_t<false, kPack, false>, launch_t<false, kPack, true>},
+     {launch_t<false, kTee, false>, launch_t<false, kTee, true>}},
+    {{launch_t<true, kStream, false>, launch_t<true, kStream, true>},
+     {launch_t<true, kPack, false>, launch_t<true, kPack, true>},
+     {launch_t<true, kTee, false>, launch_t<true, kTee, true>}}};
 
-template <bool GUARD, bool PACK, bool POW2>
-constexpr LaunchInlineFn kInlineSides[3] = {launch_inline_t<GUARD, PACK, POW2, kBothInline>,
-                                            launch_inline_t<GUARD, PACK, POW2, kSrcInline>,
-                                            launch_inline_t<GUARD, PACK, POW2, kDstInline>};
+template <bool GUARD, Kind KIND, bool POW2>
+constexpr LaunchInlineFn kInlineSides[3] = {launch_inline_t<GUARD, KIND, POW2, kBothInline>,
+                                            launch_inline_t<GUARD, KIND, POW2, kSrcInline>,
+                                            launch_inline_t<GUARD, KIND, POW2, kDstInline>};
 
-LaunchInlineFn launch_inline_fn(bool guard, bool pack, bool pow2, int sides) {
-  if (guard) {
-    if (pack) return pow2 ? kInlineSides<true, true, true>[sides] : kInlineSides<true, true, false>[sides];
-    return pow2 ? kInlineSides<true, false, true>[sides] : kInlineSides<true, false, false>[sides];
+template <Kind KIND>
+LaunchInlineFn launch_inline_fn(bool guard, bool pow2, int sides) {
+  if (KIND == kTee) {
+    if (guard) return pow2 ? launch_inline_t<true, KIND, true, kBothInline> : launch_inline_t<true, KIND, false, kBothInline>;
+    return pow2 ? launch_inline_t<false, KIND, true, kBothInline> : launch_inline_t<false, KIND, false, kBothInline>;
   }
-  if (pack) return pow2 ? kInlineSides<false, true, true>[sides] : kInlineSides<false, true, false>[sides];
-  return pow2 ? kInlineSides<false, false, true>[sides] : kInlineSides<false, false, false>[sides];
+  if (guard) return pow2 ? kInlineSides<true, KIND, true>[sides] : kInlineSides<true, KIND, false>[sides];
+  return pow2 ? kInlineSides<false, KIND, true>[sides] : kInlineSides<false, KIND, false>[sides];
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -230,7 +274,7 @@ void buffer_layers(const void* base, int64_t layer_stride, int num_layers, const
 int launch_page_copy(const Side& src, const Side& dst, int num_layers, int64_t n_pages,
                      int64_t page_bytes, int32_t* err_count, hipStream_t stream,
                      const int32_t* host_src_ids, const int32_t* host_dst_ids,
-                     StorePolicy policy) {
+                     StorePolicy policy, const Tee* tee) {
   if (num_layers < 0) return fail(PACE_KV_EINVAL, "num_layers must be >= 0 (got %d)", num_layers);
   if (n_pages < 0) return fail(PACE_KV_EINVAL, "n_pages must be >= 0 (got %lld)", (long long)n_pages);
   if (page_bytes <= 0 || page_bytes % kVecBytes != 0)
@@ -249,6 +293,8 @@ int launch_page_copy(const Side& src, const Side& dst, int num_layers, int64_t n
   if (rc) return rc;
   rc = check_layers(dst.layers, num_layers, "destination");
   if (rc) return rc;
+  if (tee != nullptr && (!src_indexed || !dst_indexed || !aligned16(tee->base) || tee->layer_stride % kVecBytes != 0))
+    return fail(PACE_KV_EINVAL, "tee: needs page ids on both sides and a 16-byte aligned buffer");
   const bool inline_ids = host_src_ids != nullptr || host_dst_ids != nullptr;
   // The inline kernels index a side without inline ids by position.
   if (inline_ids && ((host_src_ids == nullptr && src.ids != nullptr) ||
@@ -295,20 +341,91 @@ int launch_page_copy(const Side& src, const Side& dst, int num_layers, int64_t n
       p.page_vecs = static_cast<uint32_t>(page_bytes / kVecBytes);
       p.rows_per_page = static_cast<uint32_t>(rows_per_page);
       p.rows_log2 = rows_log2;
+      if (tee != nullptr) {
+        p.tee = tee->base + l0 * tee->layer_stride + j0 * page_bytes;
+        p.tee_stride = tee->layer_stride;
+      }
       const dim3 grid(static_cast<uint32_t>(rows_per_page * nj), static_cast<uint32_t>(nl));
-      const bool pack = policy == StorePolicy::kPack;
+      const Kind kind = tee != nullptr ? kTee : (policy == StorePolicy::kPack ? kPack : kStream);
       if (inline_ids) {
         CopyParamsInline q;
         q.base = p;
         if (host_src_ids) memcpy(q.src_ids, host_src_ids + j0, nj * sizeof(int32_t));
         if (host_dst_ids) memcpy(q.dst_ids, host_dst_ids + j0, nj * sizeof(int32_t));
         const int sides = host_src_ids && host_dst_ids ? kBothInline : (host_src_ids ? kSrcInline : kDstInline);
-        rc = hip_status(launch_inline_fn(guard, pack, pow2, sides)(q, grid, stream), "page copy launch");
+        const LaunchInlineFn fn = kind == kTee    ? launch_inline_fn<kTee>(guard, pow2, sides)
+                                  : kind == kPack ? launch_inline_fn<kPack>(guard, pow2, sides)
+                                                  : launch_inline_fn<kStream>(guard, pow2, sides);
+        rc = hip_status(fn(q, grid, stream), "page copy launch");
       } else {
-        rc = hip_status(kLaunch[guard][pack][pow2](p, grid, stream), "page copy launch");
+        rc = hip_status(kLaunch[guard][kind][pow2](p, grid, stream), "page copy launch");
       }
       if (rc) return rc;
     }
+  }
+  return PACE_KV_OK;
+}
+
+namespace {
+
+// Whether no byte of any [a[i], a[i] + a_bytes) lies in any [b[k], b[k] + b_bytes).
+bool disjoint(const char* const* a, int64_t a_bytes, const char* const* b, int64_t b_bytes, int n) {
+  const auto hull = [n](const char* const* t) { return std::minmax_element(t, t + n); };
+  const auto ha = hull(a), hb = hull(b);
+  // Pools allocated one after the other, the usual case: all of one side
+  // lies below all of the other.
+  if (*ha.second + a_bytes <= *hb.first || *hb.second + b_bytes <= *ha.first) return true;
+  std::vector<const char*> sa(a, a + n), sb(b, b + n);
+  std::sort(sa.begin(), sa.end());
+  std::sort(sb.begin(), sb.end());
+  for (int i = 0, k = 0; i < n && k < n;) {
+    if (sa[i] + a_bytes <= sb[k]) ++i;
+    else if (sb[k] + b_bytes <= sa[i]) ++k;
+    else return false;
+  }
+  return true;
+}
+
+}  // namespace
+
+int buffered_copy(const Side& src, const Side& dst, char* buffer, int64_t buffer_layer_stride, int buffer_layers,
+                  int num_layers, int64_t n_pages, int64_t page_bytes, int32_t* err_count, hipStream_t stream,
+                  const int32_t* host_src_ids, const int32_t* host_dst_ids) {
+  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
+  PACE_KV_TRY(check_layers(src.layers, num_layers, "source"));
+  PACE_KV_TRY(check_layers(dst.layers, num_layers, "destination"));
+  const int nb = buffer_layers < num_layers ? buffer_layers : num_layers;
+  // A pack reads every source page before the unpack writes the first
+  // destination page, so the two steps also serve pools that share memory (and
+  // a buffer inside a pool); the tee does not, and needs all three apart.
+  bool tee = page_bytes > 0 && src.pool_pages >= 0 && dst.pool_pages >= 0 &&
+             src.pool_pages <= INT64_MAX / 4 / page_bytes && dst.pool_pages <= INT64_MAX / 4 / page_bytes;
+  if (tee) {
+    const int64_t sb = src.pool_pages * page_bytes, db = dst.pool_pages * page_bytes;
+    const char* const lo = buffer;
+    const char* const hi = buffer + (nb - 1) * buffer_layer_stride + n_pages * page_bytes;
+    tee = disjoint(src.layers, sb, dst.layers, db, num_layers);
+    for (int l = 0; l < num_layers && tee; ++l)
+      tee = (src.layers[l] + sb <= lo || hi <= src.layers[l]) && (dst.layers[l] + db <= lo || hi <= dst.layers[l]);
+  }
+  std::vector<const char*> buf;
+  if (!tee) {
+    buf.resize(nb);
+    pace_kv::buffer_layers(buffer, buffer_layer_stride, nb, buf.data());
+  }
+  for (int l0 = 0; l0 < num_layers; l0 += nb) {
+    const int nl = num_layers - l0 < nb ? num_layers - l0 : nb;
+    const Side s{src.layers + l0, src.ids, src.pool_pages}, d{dst.layers + l0, dst.ids, dst.pool_pages};
+    if (tee) {
+      const Tee t{buffer, buffer_layer_stride};
+      PACE_KV_TRY(launch_page_copy(s, d, nl, n_pages, page_bytes, err_count, stream, host_src_ids, host_dst_ids,
+                                   StorePolicy::kStream, &t));
+      continue;
+    }
+    const Side b{buf.data(), nullptr, n_pages};
+    PACE_KV_TRY(launch_page_copy(s, b, nl, n_pages, page_bytes, err_count, stream, host_src_ids, nullptr,
+                                 StorePolicy::kPack));
+    PACE_KV_TRY(launch_page_copy(b, d, nl, n_pages, page_bytes, err_count, stream, nullptr, host_dst_ids));
   }
   return PACE_KV_OK;
 }
@@ -461,6 +578,26 @@ int pace_kv_move(const void* const* src_layers, int64_t src_pool_pages, const in
   Side dst{reinterpret_cast<const char* const*>(dst_layers), dst_ids, dst_pool_pages};
   return pace_kv::launch_page_copy(src, dst, num_layers, n_pages, page_bytes, err_count,
                                    static_cast<hipStream_t>(stream));
+}
+
+int pace_kv_move_buffered(const void* const* src_layers, int64_t src_pool_pages, const int32_t* src_ids,
+                          void* buffer, int64_t buffer_layer_stride, int buffer_layers,
+                          void* const* dst_layers, int64_t dst_pool_pages, const int32_t* dst_ids,
+                          int num_layers, int64_t n_pages, int64_t page_bytes, int32_t* err_count,
+                          void* stream) {
+  if (num_layers < 0 || n_pages < 0) return fail(PACE_KV_EINVAL, "move_buffered: negative size");
+  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
+  if (src_ids == nullptr || dst_ids == nullptr || buffer == nullptr)
+    return fail(PACE_KV_EINVAL, "move_buffered: NULL page ids or buffer");
+  if (buffer_layers <= 0) return fail(PACE_KV_EINVAL, "move_buffered: buffer_layers must be >= 1");
+  if (page_bytes <= 0 || page_bytes % 16 != 0)
+    return fail(PACE_KV_EINVAL, "page_bytes must be a positive multiple of 16 (got %lld)", (long long)page_bytes);
+  if (n_pages > INT64_MAX / page_bytes || buffer_layer_stride < n_pages * page_bytes || buffer_layer_stride % 16 != 0)
+    return fail(PACE_KV_ERANGE, "move_buffered: buffer_layer_stride must be >= n_pages*page_bytes and a multiple of 16");
+  Side src{reinterpret_cast<const char* const*>(src_layers), src_ids, src_pool_pages};
+  Side dst{reinterpret_cast<const char* const*>(dst_layers), dst_ids, dst_pool_pages};
+  return pace_kv::buffered_copy(src, dst, static_cast<char*>(buffer), buffer_layer_stride, buffer_layers, num_layers,
+                                n_pages, page_bytes, err_count, static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

@@ -172,19 +172,9 @@ int promote_inline(pace_kv_promoter* pr, pace_kv_allocator* dst_alloc,
                                      Side{dst_tab, nullptr, dst_pool_pages}, num_layers, n,
                                      page_bytes, err_count, stream, src_ids, dst_ids);
     } else {
-      std::vector<const char*> buf(buffer_layers);
-      pace_kv::buffer_layers(buffer, buffer_layer_stride, buffer_layers, buf.data());
-      for (int l0 = 0; l0 < num_layers && rc == PACE_KV_OK; l0 += buffer_layers) {
-        const int nl = num_layers - l0 < buffer_layers ? num_layers - l0 : buffer_layers;
-        rc = pace_kv::launch_page_copy(Side{src_tab + l0, nullptr, src_pool_pages},
-                                       Side{buf.data(), nullptr, n}, nl, n, page_bytes, err_count,
-                                       stream, src_ids, nullptr,
-                                       pace_kv::StorePolicy::kPack);
-        if (rc == PACE_KV_OK)
-          rc = pace_kv::launch_page_copy(Side{buf.data(), nullptr, n},
-                                         Side{dst_tab + l0, nullptr, dst_pool_pages}, nl, n,
-                                         page_bytes, err_count, stream, nullptr, dst_ids);
-      }
+      rc = pace_kv::buffered_copy(Side{src_tab, nullptr, src_pool_pages}, Side{dst_tab, nullptr, dst_pool_pages},
+                                  static_cast<char*>(buffer), buffer_layer_stride, buffer_layers, num_layers, n,
+                                  page_bytes, err_count, stream, src_ids, dst_ids);
     }
   }
   if (rc) {
@@ -383,14 +373,8 @@ int pace_kv_promote(pace_kv_promoter* pr, pace_kv_allocator* dst_alloc,
     rc = pace_kv_move(src_layers, src_pool_pages, dev_ids, dst_layers, dst_pool_pages, dev_ids + n,
                       num_layers, n, page_bytes, err_count, stream);
   } else {
-    for (int l0 = 0; l0 < num_layers && rc == PACE_KV_OK; l0 += buffer_layers) {
-      const int nl = num_layers - l0 < buffer_layers ? num_layers - l0 : buffer_layers;
-      rc = pace_kv_pack(src_layers + l0, nl, src_pool_pages, dev_ids, n, page_bytes, buffer,
-                        buffer_layer_stride, err_count, stream);
-      if (rc == PACE_KV_OK)
-        rc = pace_kv_unpack(buffer, buffer_layer_stride, dst_layers + l0, nl, dst_pool_pages,
-                            dev_ids + n, n, page_bytes, err_count, stream);
-    }
+    rc = pace_kv_move_buffered(src_layers, src_pool_pages, dev_ids, buffer, buffer_layer_stride, buffer_layers,
+                               dst_layers, dst_pool_pages, dev_ids + n, num_layers, n, page_bytes, err_count, stream);
   }
   // Record even on failure: the slot's next user waits on this event.
   const int rc2 = hip_status(hipEventRecord(pr->done[s], stream), "promoter record");

@@ -210,6 +210,9 @@ class KVMigrator:
         elif mode == "buffer":
             k = layers_per_chunk or self.chunk_layers(n)
             buf = self._buffer(min(k, L), n)
+            if dst_ids.numel() == n:
+                ops.move_buffered(self.src, src_ids, self.dst, dst_ids, buf)
+                return
             for lb in range(0, L, k):
                 le = min(L, lb + k)
                 ops.pack(self.src, src_ids, buf[: le - lb], layer_begin=lb, layer_end=le)

@@ -242,6 +242,27 @@ def move(src, src_ids: IdsLike, dst, dst_ids: IdsLike, *, layer_begin: int = 0,
         d_ids.data_ptr(), le - lb, n, sp.page_bytes, _err_ptr(err), _stream_handle(sp.device)))
 
 
+def move_buffered(src, src_ids: IdsLike, dst, dst_ids: IdsLike, buffer: torch.Tensor, *,
+                  err: Optional[torch.Tensor] = None) -> None:
+    """pack into `buffer` ([k, n, *page_shape]) and unpack out of it, k layers
+    at a time: the same bytes in buffer and destination, each page read once.
+    dst_ids must be distinct, as for unpack."""
+    sp, dp = as_pool(src), as_pool(dst)
+    if not sp.compatible(dp) or sp.num_layers != dp.num_layers:
+        raise ValueError("source and destination pools differ in layout, layers, dtype or device")
+    s_ids = device_ids(src_ids, sp.device)
+    d_ids = device_ids(dst_ids, dp.device, distinct=True)
+    n = s_ids.numel()
+    if n != d_ids.numel():
+        raise ValueError(f"{n} source ids but {d_ids.numel()} destination ids")
+    if n == 0:
+        return
+    stride = _check_buffer(buffer, sp, 1, n, "move_buffered")
+    _native.check(_native.load().pace_kv_move_buffered(
+        sp.table(), sp.num_pages, s_ids.data_ptr(), buffer.data_ptr(), stride, buffer.shape[0], dp.table(),
+        dp.num_pages, d_ids.data_ptr(), sp.num_layers, n, sp.page_bytes, _err_ptr(err), _stream_handle(sp.device)))
+
+
 def _swap_args(dev: PagedPool, host: PagedPool, dev_ids: IdsLike, host_ids: IdsLike, into_host: bool):
     if not host.host or dev.host:
         raise ValueError("swap needs one device pool and one host pool")
