@@ -14,14 +14,28 @@
 // pace_kv_append_indptr derives them in the same launch from append_indptr,
 // kv_indptr and kv_last_page_len, so a layer's append is one launch.
 //
-// One wave64 workgroup copies one token's K or V row (or a 16 KiB chunk of a
-// longer row): every lane loads its vectors of the row, then stores them,
-// with the page copy's device-scope write-through store.  Measured on MI355X
-// (Llama-3-8B rows of 2 KiB, 16 x 1024 tokens): 20.6 us per launch against
-// 23.3-24.5 us for a wave per 1 KiB half row with nontemporal stores, and
-// 22.3 us for the half-row waves with these stores; nontemporal
-// write-through stores ran at 23.9 us.  Every index is checked: a token whose
-// request, page slot or page id is out of range is skipped and counted.
+// One wave64 workgroup carries 1 KiB of the key rows and the same 1 KiB of the
+// value rows, one 16-byte vector of each per lane, stored with the page copy's
+// device-scope write-through store.  A token's two rows go to the same slot of
+// the two halves of a page, so they share one chain of index loads.  Rows of
+// whole KiB give a wave one token, whose indices are scalar; other rows are
+// taken end to end, vector after vector, so that every lane carries one and a
+// wave holds several tokens (or the end of one and the start of the next).
+//
+// Bound by HBM from some 16 MiB up, and below by the launch and by the chain
+// of two to four dependent index loads.  Measured on MI355X per launch in a
+// graph, fused form, against one wave per K or V row (or 16 KiB of it):
+//   256-byte rows, 16384 tokens               4.35 us, before 8.1
+//   384-byte rows, about 8500 tokens          5.2 us, before 8.4
+//   2 KiB rows, about 8500 tokens             15.5 us, before 17.0
+//   2 KiB rows, 256 tokens of a decode step   2.4 us, before 2.9
+//   8 KiB rows, 8190 tokens                   46 us, before 50 (the other form)
+// Slower are launches of few tokens with rows that are not whole KiB, which
+// take 3 us: 2-3% at 270 tokens of 256 or 384 bytes.
+// Waves that end with a row (idle lanes, scalar indices) never measured
+// faster than rows end to end, not in decode either, and up to 40% slower at
+// 16384 tokens.  Every index is checked: a token whose request, page slot or
+// page id is out of range is skipped and counted.
 #include "internal.h"
 
 namespace pace_kv {
@@ -29,8 +43,17 @@ namespace {
 
 constexpr int kThreads = 64;
 constexpr int kVecBytes = 16;
-// Longest row one wave carries: 16 vectors of 16 bytes per lane.
-constexpr int kMaxVecsPerLane = 16;
+// Workgroups per launch: grid * 64 threads stays within the 32-bit limit; a
+// longer batch uses more launches.
+constexpr int64_t kMaxGroupsPerLaunch = int64_t(1) << 25;
+
+// Appends of at most this many key bytes load their rows with plain loads,
+// larger ones nontemporally.  Measured on MI355X, 2 KiB rows: 512 KiB of keys
+// 2.4 us plain, 2.6 nontemporal; 1 MiB the same either way; 2 MiB 3.8 against
+// 4.05 and 32 MiB 24.0 against 23.1.
+constexpr int64_t kCachedLoadBytes = int64_t(1) << 20;
+// Blocks of 64 append_indptr entries that one round of the search loads.
+constexpr int kSearchBlocks = 4;
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
@@ -51,9 +74,12 @@ struct AppendParams {
   uint32_t batch_size;
   uint32_t num_pages;
   uint32_t page_size;
-  uint32_t chunks_per_row;   // ceil(row_vecs / (V * 64))
-  uint32_t total_items;      // nnz * 2 * chunks_per_row
+  int32_t page_log2;         // log2(page_size), or -1 when it is no power of two
   uint32_t row_vecs;         // row_bytes / 16
+  uint32_t row_div;          // waves (rows of whole KiB) or lanes per row
+  uint32_t div_mul, div_shift1, div_shift2;  // division by row_div (over_row)
+  uint32_t first_token;      // of this launch
+  uint32_t total_items;      // lanes of this launch: its tokens * row_vecs
   uint32_t guess_own_request;  // fused form, nnz <= batch_size: try request i for token i first
 };
 
@@ -63,127 +89,189 @@ __device__ __forceinline__ void store_row_vec(u32x4* d, const u32x4 v) {
   asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(d), "v"(v) : "memory");
 }
 
-// Request of token i in the fused form: the largest b < batch_size with
-// append_indptr[b] <= i, found by the whole wave at once: each lane loads
-// one entry of each block of 64 (four blocks per round, loaded before any is
-// tested, so up to 256 requests cost one load latency), and the entries that
-// pass are counted; -1 if none.
-__device__ __forceinline__ int32_t request_of(const AppendParams& p, int32_t i) {
-  constexpr int kBlocks = 4;
-  uint32_t count = 0;
-  for (uint32_t base = 0; base < p.batch_size; base += kBlocks * kThreads) {
-    int32_t x[kBlocks];
+// The search for a token's request in the fused form, the largest
+// b < batch_size with append_indptr[b] <= token: the whole wave searches at
+// once, each lane loading one entry of each block of 64 (four blocks per round,
+// loaded before any is tested, so up to 256 requests cost one load latency),
+// and the entries that pass are counted.
+__device__ __forceinline__ void search_load(const AppendParams& p, uint32_t base, int32_t* x) {
 #pragma unroll
-    for (int k = 0; k < kBlocks; ++k) {
-      const uint32_t e = base + k * kThreads + threadIdx.x;
-      x[k] = e < p.batch_size ? p.append_indptr[e] : INT32_MAX;
-    }
-#pragma unroll
-    for (int k = 0; k < kBlocks; ++k) count += __popcll(__ballot(x[k] <= i));
+  for (int k = 0; k < kSearchBlocks; ++k) {
+    x[k] = INT32_MAX;
+    if (k > 0 && base + k * kThreads >= p.batch_size) continue;
+    const uint32_t e = base + k * kThreads + threadIdx.x;
+    if (e < p.batch_size) x[k] = p.append_indptr[e];
   }
-  return static_cast<int32_t>(count) - 1;
 }
 
-// Page and slot of token i, or false when any index is out of range.
-template <bool FUSED>
-__device__ __forceinline__ bool locate(const AppendParams& p, uint32_t i, uint32_t* page, uint32_t* slot) {
+// How many of the entries x, summed over the wave, are at most t.
+__device__ __forceinline__ uint32_t search_count(const int32_t* x, int32_t t) {
+  uint32_t n = 0;
+#pragma unroll
+  for (int k = 0; k < kSearchBlocks; ++k) n += __popcll(__ballot(x[k] <= t));
+  return n;
+}
+
+// What the first round of index loads gives: the guessed request's offsets in
+// the fused form, the token's request and position in the other.
+struct FirstRound {
+  int32_t a0, a1, k0, k1, len;
+  int32_t b, pos;
+  bool guessed;
+  int32_t x[kSearchBlocks];  // the search's first round, where there is no guess
+};
+
+__device__ __forceinline__ void request_offsets(const AppendParams& p, uint32_t b, FirstRound* f) {
+  f->a0 = p.append_indptr[b];
+  f->a1 = p.append_indptr[b + 1];
+  f->k0 = p.kv_indptr[b];
+  f->k1 = p.kv_indptr[b + 1];
+  f->len = p.kv_last_page_len[b];
+}
+
+template <bool FUSED, bool UNIFORM>
+__device__ __forceinline__ FirstRound first_round(const AppendParams& p, uint32_t i) {
+  FirstRound f = {};
+  if (!FUSED) {
+    f.b = p.batch_indices[i];
+    f.pos = p.positions[i];
+  } else if (p.guess_own_request) {  // i < nnz <= batch_size
+    // A decode batch (no more tokens than requests) usually appends one
+    // token per request: guess that token i is request i's and load every
+    // index that places it in one round.
+    f.guessed = true;
+    request_offsets(p, i, &f);
+  } else if (UNIFORM) {
+    search_load(p, 0, f.x);
+  }
+  return f;
+}
+
+// Page and slot of the lane's token, or false when any index is out of range.
+template <bool FUSED, bool UNIFORM>
+__device__ __forceinline__ bool locate(const AppendParams& p, FirstRound f, uint32_t first_i, uint32_t last_i,
+                                       uint32_t i, uint32_t* page, uint32_t* slot) {
   int32_t pos;
   int64_t first, last;
   if (FUSED) {
     const int32_t t = static_cast<int32_t>(i);
-    int32_t a0 = 0, a1 = 0, k0 = 0, k1 = 0, len = 0;
-    bool found = false;
-    if (p.guess_own_request && i < p.batch_size) {
-      // A decode batch (no more tokens than requests) usually appends one
-      // token per request: guess that token i is request i's and load every
-      // index that places it in one round.  The guess holds exactly when
-      // append_indptr[i] <= i < append_indptr[i+1], which is when the
-      // search below finds request i.
-      a0 = p.append_indptr[i];
-      a1 = p.append_indptr[i + 1];
-      k0 = p.kv_indptr[i];
-      k1 = p.kv_indptr[i + 1];
-      len = p.kv_last_page_len[i];
-      found = a0 <= t && t < a1;
+    // The guess holds exactly when append_indptr[i] <= i < append_indptr[i+1],
+    // which is when the search finds request i.
+    const bool found = f.guessed && f.a0 <= t && t < f.a1;
+    if (UNIFORM ? !found : __ballot(!found) != 0) {
+      const int32_t t0 = static_cast<int32_t>(first_i), t1 = static_cast<int32_t>(last_i);
+      if (!UNIFORM || f.guessed) search_load(p, 0, f.x);
+      uint32_t lo = search_count(f.x, t0), hi = UNIFORM ? 0 : search_count(f.x, t1);
+      for (uint32_t base = kSearchBlocks * kThreads; base < p.batch_size; base += kSearchBlocks * kThreads) {
+        search_load(p, base, f.x);
+        lo += search_count(f.x, t0);
+        if (!UNIFORM) hi += search_count(f.x, t1);
+      }
+      if (UNIFORM) hi = lo;
+      // A wave of several requests: the entries between its first and its
+      // last token's are loaded once more and counted for each token.  (Counting
+      // the entries still held instead measured the same or 1% slower.)
+      uint32_t count = lo;
+      for (uint32_t base = lo; base < hi; base += kThreads) {
+        const uint32_t e = base + threadIdx.x;
+        const int32_t x = e < hi ? p.append_indptr[e] : INT32_MAX;
+        for (int32_t k = t0 + 1; k <= t1; ++k) {
+          const uint32_t n = __popcll(__ballot(x <= k));
+          if (t == k) count += n;
+        }
+      }
+      if (!found) {
+        if (count == 0) return false;
+        // Request count - 1 < batch_size: its offsets are loaded in one round,
+        // before the range check; by scalar loads where the wave has one
+        // request.
+        if (lo == hi) request_offsets(p, __builtin_amdgcn_readfirstlane(lo) - 1, &f);
+        else request_offsets(p, count - 1, &f);
+        if (t >= f.a1) return false;
+      }
     }
-    if (!found) {
-      const int32_t b = request_of(p, t);
-      if (b < 0) return false;
-      // b < batch_size: every offset of request b is loaded in one round,
-      // before the range check.
-      a0 = p.append_indptr[b];
-      a1 = p.append_indptr[b + 1];
-      k0 = p.kv_indptr[b];
-      k1 = p.kv_indptr[b + 1];
-      len = p.kv_last_page_len[b];
-      if (t >= a1) return false;
-    }
-    const int32_t pages = k1 - k0;
-    const int32_t seq_len = (pages > 1 ? pages - 1 : 0) * static_cast<int32_t>(p.page_size) + len;
-    pos = seq_len - (a1 - a0) + (t - a0);
-    first = k0;
-    last = k1;
+    const int32_t pages = f.k1 - f.k0;
+    const int32_t seq_len = (pages > 1 ? pages - 1 : 0) * static_cast<int32_t>(p.page_size) + f.len;
+    pos = seq_len - (f.a1 - f.a0) + (t - f.a0);
+    first = f.k0;
+    last = f.k1;
   } else {
-    const int32_t b = p.batch_indices[i];
-    pos = p.positions[i];
-    if (b < 0 || static_cast<uint32_t>(b) >= p.batch_size) return false;
-    first = p.kv_indptr[b];
-    last = p.kv_indptr[b + 1];
+    pos = f.pos;
+    if (f.b < 0 || static_cast<uint32_t>(f.b) >= p.batch_size) return false;
+    first = p.kv_indptr[f.b];
+    last = p.kv_indptr[f.b + 1];
   }
   if (pos < 0) return false;
-  const int64_t it = first + pos / static_cast<int32_t>(p.page_size);
+  const uint32_t upos = static_cast<uint32_t>(pos);
+  const uint32_t nth = p.page_log2 >= 0 ? upos >> p.page_log2 : upos / p.page_size;
+  const int64_t it = first + nth;
   if (first < 0 || it >= last || it >= p.num_indices) return false;
   *page = static_cast<uint32_t>(p.kv_indices[it]);
   if (*page >= p.num_pages) return false;
-  *slot = static_cast<uint32_t>(pos) % p.page_size;
+  *slot = upos - nth * p.page_size;
   return true;
 }
 
-// V: vectors per lane (the row, or its chunk, is V * 64 vectors); GUARD: the
-// row is not a multiple of that; MULTI: rows longer than one chunk.
-template <int V, bool GUARD, bool MULTI, bool FUSED>
+// n / row_div by the multiply-and-shift form for a divisor known ahead
+// (Granlund and Montgomery, "Division by invariant integers using
+// multiplication", figure 4.1), exact for every n.
+__device__ __forceinline__ uint32_t over_row(const AppendParams& p, uint32_t n) {
+  const uint32_t q = __umulhi(p.div_mul, n);
+  return (q + ((n - q) >> p.div_shift1)) >> p.div_shift2;
+}
+
+template <bool NT>
+__device__ __forceinline__ u32x4 load_vec(const u32x4* s) {
+  return NT ? __builtin_nontemporal_load(s) : *s;
+}
+
+// UNIFORM: rows of whole KiB, so that a wave holds one token and its index
+// loads are scalar.
+template <bool FUSED, bool UNIFORM, bool NT>
 __global__ __launch_bounds__(kThreads) void append_kernel(const AppendParams p) {
-  const uint32_t item = blockIdx.x;
-  if (item >= p.total_items) return;
-  uint32_t i, kv, chunk;
-  if (MULTI) {
-    const uint32_t per_token = 2 * p.chunks_per_row;
-    i = item / per_token;
-    const uint32_t rem = item - i * per_token;
-    kv = rem / p.chunks_per_row;
-    chunk = rem - kv * p.chunks_per_row;
+  uint32_t i, vec, first_i, last_i;
+  bool live = true;
+  if (UNIFORM) {
+    const uint32_t t = over_row(p, blockIdx.x);
+    vec = (blockIdx.x - t * p.row_div) * kThreads + threadIdx.x;
+    i = first_i = last_i = p.first_token + t;
   } else {
-    i = item >> 1;
-    kv = item & 1;
-    chunk = 0;
+    uint32_t g = blockIdx.x * kThreads + threadIdx.x;
+    live = g < p.total_items;
+    if (!live) g = p.total_items - 1;  // the lane stays for the wave's search
+    const uint32_t t = over_row(p, g);
+    vec = g - t * p.row_div;
+    i = p.first_token + t;
+    first_i = __builtin_amdgcn_readlane(i, 0);
+    last_i = __builtin_amdgcn_readlane(i, kThreads - 1);
   }
-  // The row's loads depend on the token alone (always in range): they are
+  FirstRound f;
+  if (!UNIFORM) {
+    // Per-lane index loads share the row loads' counter, which counts in
+    // order: the first round goes ahead of them.
+    f = first_round<FUSED, false>(p, i);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // The rows' loads depend on the token alone (always in range): they are
   // issued before the index loads that place it, so their latencies overlap.
-  const u32x4* src = reinterpret_cast<const u32x4*>((kv ? p.value : p.key) + static_cast<int64_t>(i) * p.token_stride);
-  const uint32_t first_vec = chunk * (V * kThreads) + threadIdx.x;
-  u32x4 v[V];
-#pragma unroll
-  for (int c = 0; c < V; ++c) {
-    const uint32_t vec = first_vec + c * kThreads;
-    if (!GUARD || vec < p.row_vecs) v[c] = __builtin_nontemporal_load(src + vec);
-  }
+  const int64_t at = static_cast<int64_t>(i) * p.token_stride;
+  const u32x4 k = load_vec<NT>(reinterpret_cast<const u32x4*>(p.key + at) + vec);
+  const u32x4 v = load_vec<NT>(reinterpret_cast<const u32x4*>(p.value + at) + vec);
   // Without this barrier the compiler sinks the row loads below the index
   // loads (into the block that stores the row), and the two latencies add up
   // again (measured: 1 us of a 20.8 us prefill launch).
   __builtin_amdgcn_sched_barrier(0);
+  if (UNIFORM) f = first_round<FUSED, true>(p, i);
   uint32_t page = 0, slot = 0;
-  if (!locate<FUSED>(p, i, &page, &slot)) {
-    if (kv == 0 && chunk == 0 && threadIdx.x == 0 && p.err != nullptr) atomicAdd(p.err, 1);
+  if (!locate<FUSED, UNIFORM>(p, f, first_i, last_i, i, &page, &slot)) {
+    if (live && vec == 0 && p.err != nullptr) atomicAdd(p.err, 1);
     return;
   }
-  const int64_t page_bytes = 2 * static_cast<int64_t>(p.page_size) * p.row_bytes;
-  u32x4* dst = reinterpret_cast<u32x4*>(p.cache + static_cast<int64_t>(page) * page_bytes +
-                                        (static_cast<int64_t>(kv) * p.page_size + slot) * p.row_bytes);
-#pragma unroll
-  for (int c = 0; c < V; ++c) {
-    const uint32_t vec = first_vec + c * kThreads;
-    if (!GUARD || vec < p.row_vecs) store_row_vec(dst + vec, v[c]);
-  }
+  if (!live) return;
+  const int64_t half = static_cast<int64_t>(p.page_size) * p.row_bytes;
+  char* row = p.cache + 2 * half * page + static_cast<int64_t>(slot) * p.row_bytes;
+  store_row_vec(reinterpret_cast<u32x4*>(row) + vec, k);
+  store_row_vec(reinterpret_cast<u32x4*>(row + half) + vec, v);
 }
 
 // One thread per appended token: finds its request by binary search over
@@ -217,22 +305,19 @@ __global__ __launch_bounds__(256) void positions_kernel(const int32_t* __restric
 namespace pace_kv {
 namespace {
 
-template <int V, bool GUARD, bool MULTI, bool FUSED>
-const void* kernel_of() {
-  return reinterpret_cast<const void*>(&append_kernel<V, GUARD, MULTI, FUSED>);
+int32_t exact_log2(int64_t n) {
+  return (n & (n - 1)) == 0 ? static_cast<int32_t>(__builtin_ctzll(static_cast<uint64_t>(n))) : -1;
+}
+
+template <bool FUSED, bool UNIFORM>
+const void* kernel_of(bool nt) {
+  return nt ? reinterpret_cast<const void*>(&append_kernel<FUSED, UNIFORM, true>)
+            : reinterpret_cast<const void*>(&append_kernel<FUSED, UNIFORM, false>);
 }
 
 template <bool FUSED>
-const void* pick_kernel(int v, bool guard, bool multi) {
-  switch (v) {
-    case 1: return guard ? kernel_of<1, true, false, FUSED>() : kernel_of<1, false, false, FUSED>();
-    case 2: return guard ? kernel_of<2, true, false, FUSED>() : kernel_of<2, false, false, FUSED>();
-    case 4: return guard ? kernel_of<4, true, false, FUSED>() : kernel_of<4, false, false, FUSED>();
-    case 8: return guard ? kernel_of<8, true, false, FUSED>() : kernel_of<8, false, false, FUSED>();
-    default:
-      if (multi) return guard ? kernel_of<16, true, true, FUSED>() : kernel_of<16, false, true, FUSED>();
-      return guard ? kernel_of<16, true, false, FUSED>() : kernel_of<16, false, false, FUSED>();
-  }
+const void* pick_kernel(bool uniform, bool nt) {
+  return uniform ? kernel_of<FUSED, true>(nt) : kernel_of<FUSED, false>(nt);
 }
 
 // Checks the arguments both forms share, sizes the grid and launches.
@@ -253,12 +338,10 @@ int launch_append(AppendParams& p, int64_t nnz, int batch_size, int64_t num_page
     return fail(PACE_KV_EINVAL, "append: keys, values and cache must be 16-byte aligned");
   if (num_pages > INT32_MAX) return fail(PACE_KV_ERANGE, "append: too many pages");
   const int64_t row_vecs = row_bytes / kVecBytes;
-  const int64_t per_lane = (row_vecs + kThreads - 1) / kThreads;
-  int v = 1;
-  while (v < per_lane && v < kMaxVecsPerLane) v *= 2;
-  const int64_t chunk_vecs = static_cast<int64_t>(v) * kThreads;
-  const int64_t chunks = (row_vecs + chunk_vecs - 1) / chunk_vecs;
-  if (nnz > INT32_MAX || nnz * 2 * chunks >= (int64_t(1) << 25))
+  // The most one call takes: 2^24 rows per side, a row longer than 16 KiB
+  // counting once per 16 KiB.
+  const int64_t pieces = (row_bytes + (16 << 10) - 1) / (16 << 10);
+  if (nnz > INT32_MAX || nnz * 2 * pieces >= (int64_t(1) << 25))
     return fail(PACE_KV_ERANGE, "append: too many tokens for one launch (%lld)", (long long)nnz);
   p.token_stride = token_stride_bytes;
   p.num_indices = num_indices;
@@ -266,14 +349,31 @@ int launch_append(AppendParams& p, int64_t nnz, int batch_size, int64_t num_page
   p.batch_size = static_cast<uint32_t>(batch_size);
   p.num_pages = static_cast<uint32_t>(num_pages);
   p.page_size = static_cast<uint32_t>(page_size);
-  p.chunks_per_row = static_cast<uint32_t>(chunks);
-  p.total_items = static_cast<uint32_t>(nnz * 2 * chunks);
+  p.page_log2 = exact_log2(page_size);
   p.row_vecs = static_cast<uint32_t>(row_vecs);
   p.guess_own_request = fused && nnz <= batch_size ? 1u : 0u;
-  const bool guard = row_vecs % chunk_vecs != 0;
-  const void* fn = fused ? pick_kernel<true>(v, guard, chunks > 1) : pick_kernel<false>(v, guard, chunks > 1);
-  void* args[] = {&p};
-  return hip_status(hipLaunchKernel(fn, dim3(p.total_items), dim3(kThreads), args, 0, stream), "append launch");
+  const bool uniform = row_vecs % kThreads == 0;
+  const bool nt = nnz * row_bytes > kCachedLoadBytes;
+  const int64_t waves_per_row = (row_vecs + kThreads - 1) / kThreads;
+  p.row_div = static_cast<uint32_t>(uniform ? waves_per_row : row_vecs);
+  uint32_t log2_up = 0;
+  while ((uint64_t(1) << log2_up) < p.row_div) ++log2_up;
+  p.div_mul = static_cast<uint32_t>((((uint64_t(1) << log2_up) - p.row_div) << 32) / p.row_div + 1);
+  p.div_shift1 = log2_up > 0 ? 1 : 0;
+  p.div_shift2 = log2_up > 0 ? log2_up - 1 : 0;
+  const void* fn = fused ? pick_kernel<true>(uniform, nt) : pick_kernel<false>(uniform, nt);
+  const int64_t max_tokens = kMaxGroupsPerLaunch / waves_per_row;
+  if (max_tokens < 1) return fail(PACE_KV_ERANGE, "append: row bytes too large (%lld)", (long long)row_bytes);
+  for (int64_t t0 = 0; t0 < nnz; t0 += max_tokens) {
+    const int64_t n = nnz - t0 < max_tokens ? nnz - t0 : max_tokens;
+    const int64_t groups = (n * row_vecs + kThreads - 1) / kThreads;
+    p.first_token = static_cast<uint32_t>(t0);
+    p.total_items = static_cast<uint32_t>(n * row_vecs);
+    void* args[] = {&p};
+    PACE_KV_TRY(hip_status(hipLaunchKernel(fn, dim3(static_cast<uint32_t>(groups)),
+                                           dim3(kThreads), args, 0, stream), "append launch"));
+  }
+  return PACE_KV_OK;
 }
 
 }  // namespace
