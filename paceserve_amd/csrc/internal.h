@@ -23,6 +23,27 @@ int fail(int code, const char* fmt, ...);
 // and records its message; returns 0 for hipSuccess.
 int hip_status(hipError_t err, const char* what);
 
+// Division by a divisor known on the host, by the multiply-and-shift form
+// (Granlund and Montgomery, "Division by invariant integers using
+// multiplication", figure 4.1), exact for every 32-bit n and divisor >= 1.
+struct FastDiv {
+  uint32_t mul, shift1, shift2;
+};
+
+inline FastDiv fast_div(uint32_t divisor) {
+  uint32_t log2_up = 0;
+  while ((uint64_t(1) << log2_up) < divisor) ++log2_up;
+  return FastDiv{static_cast<uint32_t>((((uint64_t(1) << log2_up) - divisor) << 32) / divisor + 1),
+                 log2_up > 0 ? 1u : 0u, log2_up > 0 ? log2_up - 1 : 0u};
+}
+
+#ifdef __HIP__
+__device__ __forceinline__ uint32_t over(const FastDiv& d, uint32_t n) {
+  const uint32_t q = __umulhi(d.mul, n);
+  return (q + ((n - q) >> d.shift1)) >> d.shift2;
+}
+#endif
+
 // One side of a page copy: per-layer base pointers plus an optional device
 // page-id array (NULL means page j of layer l is at base[l] + j*page_bytes,
 // which is how the contiguous transfer buffer is addressed).

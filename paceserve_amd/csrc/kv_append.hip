@@ -77,7 +77,7 @@ struct AppendParams {
   int32_t page_log2;         // log2(page_size), or -1 when it is no power of two
   uint32_t row_vecs;         // row_bytes / 16
   uint32_t row_div;          // waves (rows of whole KiB) or lanes per row
-  uint32_t div_mul, div_shift1, div_shift2;  // division by row_div (over_row)
+  FastDiv by_row;            // division by row_div
   uint32_t first_token;      // of this launch
   uint32_t total_items;      // lanes of this launch: its tokens * row_vecs
   uint32_t guess_own_request;  // fused form, nnz <= batch_size: try request i for token i first
@@ -212,14 +212,6 @@ __device__ __forceinline__ bool locate(const AppendParams& p, FirstRound f, uint
   return true;
 }
 
-// n / row_div by the multiply-and-shift form for a divisor known ahead
-// (Granlund and Montgomery, "Division by invariant integers using
-// multiplication", figure 4.1), exact for every n.
-__device__ __forceinline__ uint32_t over_row(const AppendParams& p, uint32_t n) {
-  const uint32_t q = __umulhi(p.div_mul, n);
-  return (q + ((n - q) >> p.div_shift1)) >> p.div_shift2;
-}
-
 template <bool NT>
 __device__ __forceinline__ u32x4 load_vec(const u32x4* s) {
   return NT ? __builtin_nontemporal_load(s) : *s;
@@ -232,14 +224,14 @@ __global__ __launch_bounds__(kThreads) void append_kernel(const AppendParams p) 
   uint32_t i, vec, first_i, last_i;
   bool live = true;
   if (UNIFORM) {
-    const uint32_t t = over_row(p, blockIdx.x);
+    const uint32_t t = over(p.by_row, blockIdx.x);
     vec = (blockIdx.x - t * p.row_div) * kThreads + threadIdx.x;
     i = first_i = last_i = p.first_token + t;
   } else {
     uint32_t g = blockIdx.x * kThreads + threadIdx.x;
     live = g < p.total_items;
     if (!live) g = p.total_items - 1;  // the lane stays for the wave's search
-    const uint32_t t = over_row(p, g);
+    const uint32_t t = over(p.by_row, g);
     vec = g - t * p.row_div;
     i = p.first_token + t;
     first_i = __builtin_amdgcn_readlane(i, 0);
@@ -356,11 +348,7 @@ int launch_append(AppendParams& p, int64_t nnz, int batch_size, int64_t num_page
   const bool nt = nnz * row_bytes > kCachedLoadBytes;
   const int64_t waves_per_row = (row_vecs + kThreads - 1) / kThreads;
   p.row_div = static_cast<uint32_t>(uniform ? waves_per_row : row_vecs);
-  uint32_t log2_up = 0;
-  while ((uint64_t(1) << log2_up) < p.row_div) ++log2_up;
-  p.div_mul = static_cast<uint32_t>((((uint64_t(1) << log2_up) - p.row_div) << 32) / p.row_div + 1);
-  p.div_shift1 = log2_up > 0 ? 1 : 0;
-  p.div_shift2 = log2_up > 0 ? log2_up - 1 : 0;
+  p.by_row = fast_div(p.row_div);
   const void* fn = fused ? pick_kernel<true>(uniform, nt) : pick_kernel<false>(uniform, nt);
   const int64_t max_tokens = kMaxGroupsPerLaunch / waves_per_row;
   if (max_tokens < 1) return fail(PACE_KV_ERANGE, "append: row bytes too large (%lld)", (long long)row_bytes);

@@ -18,7 +18,8 @@
 // (unpack) or write (pack) adjacent rows of the transfer buffer and adjacent
 // rows of each pool page.  A wave splits blockIdx.x into page and row with a
 // shift when a page has a power-of-two number of rows (every common KV page),
-// else with one division.  An unpack wave issues its buffer load before its
+// else with one division; pages that are no whole number of rows are taken end
+// to end (enum Shape).  An unpack wave issues its buffer load before its
 // destination page id arrives.  Measured on MI355X, this fine grain keeps
 // the chip's in-flight accesses within a narrow address window and copies at
 // ~6.6 TB/s, against ~5.6-5.9 TB/s for 8-32 KiB per workgroup, persistent
@@ -59,8 +60,11 @@ struct CopyParams {
   uint32_t src_pool_pages;
   uint32_t dst_pool_pages;
   uint32_t page_vecs;      // page_bytes / 16
-  uint32_t rows_per_page;  // ceil(page_bytes / kRowBytes)
+  uint32_t rows_per_page;  // page_bytes / kRowBytes (pages of whole rows)
   uint32_t rows_log2;      // log2(rows_per_page) when that is a power of two
+  FastDiv by_page;         // pages end to end: division by page_vecs
+  uint32_t n_pages;        // of this launch, per layer
+  uint32_t total_vecs;     // n_pages * page_vecs
   char* tee;               // Kind::kTee: page j of layer l also goes to tee + l * tee_stride + j * page_bytes
   int64_t tee_stride;
 };
@@ -70,6 +74,29 @@ struct CopyParams {
 // in a transfer buffer).
 enum Kind { kStream = 0, kPack = 1, kTee = 2 };
 
+// How a launch splits a layer's pages over its waves.  Pages of a power-of-two
+// number of 1 KiB rows (kPow2) or of another whole number (kRows): one row per
+// wave.  Other pages are taken end to end, vector after vector, so that every
+// lane carries a vector and a wave may hold several pages, or the end of one
+// and the start of the next: each lane loads its own page's ids (kLaneFlat), or
+// the wave loads the at most kSpan ids per side that its lanes choose from by
+// scalar loads (kSpanFlat, ids on both sides and pages of at least kSpanVecs
+// vectors).
+// Measured on MI355X, 32 layers, 150 MiB, against waves that end with a page:
+//   move    160 B 210 -> 103 us, 256 B 132 -> 52, 512 B 67.4 -> 50.3, 1280 B
+//           57 -> 50, 1536 B 53.7 -> 49.8, the same from 2560 B on
+//   pack    160 B 210 -> 60, 512 B 67 -> 46, 1280 B 54.5 -> 46.3, 1536 B and
+//           more the same or up to 2% faster
+//   unpack  160 B 210 -> 85, 512 B 67.5 -> 48.9, 1280 B 56.4 -> 48.8
+// and on 8 MiB in a graph 512 B 5.3 -> 4.0 us; launches of 0.5 to 2 MiB, about
+// 2.1 us, are up to 0.1 us faster or slower (a move of 0.5 MiB 0.15 slower).
+// A move by lanes' own ids is 3-4% slower than by scalar ids (its id loads go
+// ahead of the page's in one chain); a pack or unpack by scalar ids is 4-8%
+// slower at 150 MiB (the contiguous side needs no id).
+enum Shape { kPow2 = 0, kRows = 1, kSpanFlat = 2, kLaneFlat = 3 };
+constexpr int kSpan = 3;
+constexpr int kSpanVecs = kThreads / (kSpan - 1);
+
 // Page ids carried in the kernel arguments (small promotions): no device id
 // array, so no upload has to precede the launch.
 struct CopyParamsInline {
@@ -78,8 +105,15 @@ struct CopyParamsInline {
   int32_t dst_ids[PACE_KV_INLINE_IDS];
 };
 
-__device__ __forceinline__ uint32_t page_of(const int32_t* ids, uint32_t j) {
-  return ids ? static_cast<uint32_t>(ids[j]) : j;
+// The page id of position j; in kSpanFlat j lies `nth` < kSpan pages after j0,
+// the wave's first, and the ids of all of them are loaded by scalar loads.
+template <Shape SHAPE>
+__device__ __forceinline__ uint32_t page_of(const CopyParams& p, const int32_t* ids, uint32_t j, uint32_t j0,
+                                            uint32_t nth) {
+  if (SHAPE != kSpanFlat) return static_cast<uint32_t>(ids[j]);
+  const uint32_t last = p.n_pages - 1;
+  const int32_t a = ids[j0], b = ids[min(j0 + 1, last)], c = ids[min(j0 + 2, last)];
+  return static_cast<uint32_t>(nth == 0 ? a : nth == 1 ? b : c);
 }
 
 // Stores carry the device-scope bit (sc1): an XCD's L2 is not coherent with
@@ -116,11 +150,11 @@ __device__ __forceinline__ void store_vec(const u32x4 v, u32x4* d) {
 // stores on both sides 4-7%, nontemporal loads 0.5-1%, the destination store
 // first 0.2-1%; 128 threads are 0.5% faster on 512 MiB and 2% slower on 2.8 GB,
 // 256 and 512 threads slower on both.
-__device__ __forceinline__ void tee_row(const CopyParams& p, uint32_t j, uint32_t layer, uint32_t row,
-                                        uint32_t vec, uint32_t sp, uint32_t dp) {
+__device__ __forceinline__ void tee_row(const CopyParams& p, uint32_t j, uint32_t layer, uint32_t vec,
+                                        uint32_t sp, uint32_t dp) {
   u32x4* buf = reinterpret_cast<u32x4*>(p.tee + layer * p.tee_stride + static_cast<int64_t>(j) * p.page_bytes) + vec;
   const bool src_ok = sp < p.src_pool_pages, dst_ok = dp < p.dst_pool_pages;
-  if (!(src_ok && dst_ok) && row == 0 && threadIdx.x == 0 && p.err != nullptr)
+  if (!(src_ok && dst_ok) && vec == 0 && p.err != nullptr)
     atomicAdd(p.err, static_cast<int>(!src_ok) + static_cast<int>(!dst_ok));
   const u32x4* s = src_ok ? reinterpret_cast<const u32x4*>(p.src[layer] + static_cast<int64_t>(sp) * p.page_bytes) + vec
                           : buf;
@@ -130,43 +164,59 @@ __device__ __forceinline__ void tee_row(const CopyParams& p, uint32_t j, uint32_
     store_vec<false>(v, reinterpret_cast<u32x4*>(p.dst[layer] + static_cast<int64_t>(dp) * p.page_bytes) + vec);
 }
 
-// The copy of one 1 KiB row: item blockIdx.x (page j, row r of it) of layer
-// blockIdx.y; the grid is exactly (rows x pages) x layers.  POW2: the page has
-// a power-of-two number of rows.  sids / dids are the sides' page ids (device
-// or kernel-argument arrays), nullptr for a contiguous side.  Loads are
-// nontemporal but in a tee; KIND selects the store policy (store_vec) and the tee.
-template <bool GUARD, Kind KIND, bool POW2>
+// The copy of one 1 KiB row: item blockIdx.x of layer blockIdx.y.  For pages
+// of whole rows (kPow2, kRows) that is row r of page j, the grid is exactly
+// (rows x pages) x layers and every index is scalar; else it is the next
+// 64 vectors of the layer's pages.  sids / dids are the
+// sides' page ids (device or kernel-argument arrays), nullptr for a contiguous
+// side.  Loads are nontemporal but in a tee; KIND selects the store policy
+// (store_vec) and the tee.
+template <Shape SHAPE, Kind KIND>
 __device__ __forceinline__ void copy_row(const CopyParams& p, const int32_t* sids,
                                          const int32_t* dids) {
   const uint32_t x = blockIdx.x;
-  const uint32_t j = POW2 ? x >> p.rows_log2 : x / p.rows_per_page;
-  const uint32_t row = POW2 ? x & (p.rows_per_page - 1) : x - j * p.rows_per_page;
   const uint32_t layer = blockIdx.y;
-  const uint32_t vec = row * kThreads + threadIdx.x;
-  // Lane 0 of row 0 is never guarded out, so a skipped tile is still counted.
-  if (GUARD && vec >= p.page_vecs) return;
-  if (sids == nullptr) {
+  uint32_t j, vec, j0 = 0, nth = 0;
+  if (SHAPE == kLaneFlat) {
+    const uint32_t g = x * kThreads + threadIdx.x;
+    if (g >= p.total_vecs) return;
+    j = over(p.by_page, g);
+    vec = g - j * p.page_vecs;
+  } else if (SHAPE == kSpanFlat) {
+    const uint32_t g0 = x * kThreads;
+    if (g0 + threadIdx.x >= p.total_vecs) return;
+    j0 = over(p.by_page, g0);
+    vec = g0 - j0 * p.page_vecs + threadIdx.x;
+    nth = (vec >= p.page_vecs ? 1 : 0) + (vec >= 2 * p.page_vecs ? 1 : 0);
+    j = j0 + nth;
+    vec -= nth * p.page_vecs;
+  } else {
+    j = SHAPE == kPow2 ? x >> p.rows_log2 : x / p.rows_per_page;
+    const uint32_t row = SHAPE == kPow2 ? x & (p.rows_per_page - 1) : x - j * p.rows_per_page;
+    vec = row * kThreads + threadIdx.x;
+  }
+  if (SHAPE != kSpanFlat && sids == nullptr) {
     // Contiguous source (unpack): page j of the buffer is always in bounds,
     // so the load is issued before the destination id is known.
     const u32x4 v = __builtin_nontemporal_load(
         reinterpret_cast<const u32x4*>(p.src[layer] + static_cast<int64_t>(j) * p.page_bytes) + vec);
-    const uint32_t dp = page_of(dids, j);
+    const uint32_t dp = dids ? static_cast<uint32_t>(dids[j]) : j;
     if (dp >= p.dst_pool_pages) {
-      if (row == 0 && threadIdx.x == 0 && p.err != nullptr) atomicAdd(p.err, 1);
+      if (vec == 0 && p.err != nullptr) atomicAdd(p.err, 1);
       return;
     }
     store_vec<KIND == kPack>(v, reinterpret_cast<u32x4*>(p.dst[layer] + static_cast<int64_t>(dp) * p.page_bytes) + vec);
     return;
   }
-  const uint32_t sp = static_cast<uint32_t>(sids[j]);
-  const uint32_t dp = page_of(dids, j);
+  const uint32_t sp = page_of<SHAPE>(p, sids, j, j0, nth);
+  const uint32_t dp = SHAPE == kSpanFlat || dids ? page_of<SHAPE>(p, dids, j, j0, nth) : j;
   if (KIND == kTee) {
-    tee_row(p, j, layer, row, vec, sp, dp);
+    tee_row(p, j, layer, vec, sp, dp);
     return;
   }
   // Negative ids wrap to large unsigned values and fail the same test.
   if (sp >= p.src_pool_pages || dp >= p.dst_pool_pages) {
-    if (row == 0 && threadIdx.x == 0 && p.err != nullptr) atomicAdd(p.err, 1);
+    if (vec == 0 && p.err != nullptr) atomicAdd(p.err, 1);
     return;
   }
   const u32x4 v = __builtin_nontemporal_load(
@@ -174,68 +224,71 @@ __device__ __forceinline__ void copy_row(const CopyParams& p, const int32_t* sid
   store_vec<KIND == kPack>(v, reinterpret_cast<u32x4*>(p.dst[layer] + static_cast<int64_t>(dp) * p.page_bytes) + vec);
 }
 
-// GUARD: page_bytes is not a multiple of kRowBytes, so the last row of a page
-// is partial.
-template <bool GUARD, Kind KIND, bool POW2>
+template <Shape SHAPE, Kind KIND>
 __global__ __launch_bounds__(kThreads) void page_copy_kernel(const CopyParams p) {
-  copy_row<GUARD, KIND, POW2>(p, p.src_ids, p.dst_ids);
+  copy_row<SHAPE, KIND>(p, p.src_ids, p.dst_ids);
 }
 
 // Same copy with the ids in the kernel arguments.  A side whose ids are not
 // inline (the contiguous buffer of a pack or unpack) indexes pages by
 // position.
-template <bool GUARD, Kind KIND, bool POW2, bool SRC_INLINE, bool DST_INLINE>
+template <Shape SHAPE, Kind KIND, bool SRC_INLINE, bool DST_INLINE>
 __global__ __launch_bounds__(kThreads) void page_copy_inline_kernel(const CopyParamsInline p) {
-  copy_row<GUARD, KIND, POW2>(p.base, SRC_INLINE ? p.src_ids : nullptr,
-                              DST_INLINE ? p.dst_ids : nullptr);
-}
-
-template <bool GUARD, Kind KIND, bool POW2>
-hipError_t launch_t(const CopyParams& p, dim3 grid, hipStream_t stream) {
-  void* args[] = {const_cast<CopyParams*>(&p)};
-  return hipLaunchKernel(reinterpret_cast<const void*>(&page_copy_kernel<GUARD, KIND, POW2>), grid,
-                         dim3(kThreads), args, 0, stream);
+  copy_row<SHAPE, KIND>(p.base, SRC_INLINE ? p.src_ids : nullptr, DST_INLINE ? p.dst_ids : nullptr);
 }
 
 // Inline ids on both sides (move), the source only (pack) or the destination
 // only (unpack).
 enum InlineSides { kBothInline = 0, kSrcInline = 1, kDstInline = 2 };
 
-template <bool GUARD, Kind KIND, bool POW2, int SIDES>
-hipError_t launch_inline_t(const CopyParamsInline& p, dim3 grid, hipStream_t stream) {
-  void* args[] = {const_cast<CopyParamsInline*>(&p)};
-  constexpr bool kS = SIDES != kDstInline, kD = SIDES != kSrcInline;
-  return hipLaunchKernel(
-      reinterpret_cast<const void*>(&page_copy_inline_kernel<GUARD, KIND, POW2, kS, kD>), grid,
-      dim3(kThreads), args, 0, stream);
+template <Shape SHAPE>
+const void* kernel_of(Kind kind) {
+  switch (kind) {
+    case kPack: return reinterpret_cast<const void*>(&page_copy_kernel<SHAPE, kPack>);
+    case kTee: return reinterpret_cast<const void*>(&page_copy_kernel<SHAPE, kTee>);
+    default: return reinterpret_cast<const void*>(&page_copy_kernel<SHAPE, kStream>);
+  }
 }
 
-using LaunchFn = hipError_t (*)(const CopyParams&, dim3, hipStream_t);
-using LaunchInlineFn = hipError_t (*)(const CopyParamsInline&, dim3, hipStream_t);
-
-// Instances indexed [GUARD][KIND][POW2] (and [SIDES] for inline ids; a tee
-// has ids on both sides).
-constexpr LaunchFn kLaunch[2][3][2] = {
-    {{launch_t<false, kStream, false>, launch_t<false, kStream, true>},
-     {launch_t<false, kPack, false>, launch_t<false, kPack, true>},
-     {launch_t<false, kTee, false>, launch_t<false, kTee, true>}},
-    {{launch_t<true, kStream, false>, launch_t<true, kStream, true>},
-     {launch_t<true, kPack, false>, launch_t<true, kPack, true>},
-     {launch_t<true, kTee, false>, launch_t<true, kTee, true>}}};
-
-template <bool GUARD, Kind KIND, bool POW2>
-constexpr LaunchInlineFn kInlineSides[3] = {launch_inline_t<GUARD, KIND, POW2, kBothInline>,
-                                            launch_inline_t<GUARD, KIND, POW2, kSrcInline>,
-                                            launch_inline_t<GUARD, KIND, POW2, kDstInline>};
-
-template <Kind KIND>
-LaunchInlineFn launch_inline_fn(bool guard, bool pow2, int sides) {
-  if (KIND == kTee) {
-    if (guard) return pow2 ? launch_inline_t<true, KIND, true, kBothInline> : launch_inline_t<true, KIND, false, kBothInline>;
-    return pow2 ? launch_inline_t<false, KIND, true, kBothInline> : launch_inline_t<false, KIND, false, kBothInline>;
+template <Shape SHAPE, Kind KIND>
+const void* inline_kernel_of(InlineSides sides) {
+  switch (sides) {
+    case kSrcInline: return reinterpret_cast<const void*>(&page_copy_inline_kernel<SHAPE, KIND, true, false>);
+    case kDstInline: return reinterpret_cast<const void*>(&page_copy_inline_kernel<SHAPE, KIND, false, true>);
+    default: return reinterpret_cast<const void*>(&page_copy_inline_kernel<SHAPE, KIND, true, true>);
   }
-  if (guard) return pow2 ? kInlineSides<true, KIND, true>[sides] : kInlineSides<true, KIND, false>[sides];
-  return pow2 ? kInlineSides<false, KIND, true>[sides] : kInlineSides<false, KIND, false>[sides];
+}
+
+template <Shape SHAPE>
+const void* inline_kernel_of(Kind kind, InlineSides sides) {
+  switch (kind) {
+    case kPack: return inline_kernel_of<SHAPE, kPack>(sides);
+    // a tee has ids on both sides
+    case kTee: return reinterpret_cast<const void*>(&page_copy_inline_kernel<SHAPE, kTee, true, true>);
+    default: return inline_kernel_of<SHAPE, kStream>(sides);
+  }
+}
+
+const void* pick_kernel(Shape shape, Kind kind) {
+  switch (shape) {
+    case kPow2: return kernel_of<kPow2>(kind);
+    case kRows: return kernel_of<kRows>(kind);
+    case kSpanFlat:  // a move or a tee
+      return kind == kTee ? reinterpret_cast<const void*>(&page_copy_kernel<kSpanFlat, kTee>)
+                          : reinterpret_cast<const void*>(&page_copy_kernel<kSpanFlat, kStream>);
+    default: return kernel_of<kLaneFlat>(kind);
+  }
+}
+
+const void* pick_inline_kernel(Shape shape, Kind kind, InlineSides sides) {
+  switch (shape) {
+    case kPow2: return inline_kernel_of<kPow2>(kind, sides);
+    case kRows: return inline_kernel_of<kRows>(kind, sides);
+    case kSpanFlat:
+      return kind == kTee ? reinterpret_cast<const void*>(&page_copy_inline_kernel<kSpanFlat, kTee, true, true>)
+                          : reinterpret_cast<const void*>(&page_copy_inline_kernel<kSpanFlat, kStream, true, true>);
+    default: return inline_kernel_of<kLaneFlat>(kind, sides);
+  }
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -308,7 +361,6 @@ int launch_page_copy(const Side& src, const Side& dst, int num_layers, int64_t n
   if (dst.ids != nullptr && (reinterpret_cast<uintptr_t>(dst.ids) & 3u))
     return fail(PACE_KV_EINVAL, "destination page ids are not 4-byte aligned");
 
-  const bool guard = page_bytes % kRowBytes != 0;
   const int64_t rows_per_page = (page_bytes + kRowBytes - 1) / kRowBytes;
 
   const auto clamp_pool = [](int64_t pages) -> uint32_t {
@@ -317,7 +369,11 @@ int launch_page_copy(const Side& src, const Side& dst, int num_layers, int64_t n
 
   uint32_t rows_log2 = 0;
   while ((int64_t(1) << rows_log2) < rows_per_page) ++rows_log2;
-  const bool pow2 = (int64_t(1) << rows_log2) == rows_per_page;
+  const bool whole_rows = page_bytes % kRowBytes == 0;
+  const bool span = page_bytes >= kSpanVecs * kVecBytes && src_indexed && dst_indexed && policy == StorePolicy::kStream;
+  const Shape shape = whole_rows ? ((int64_t(1) << rows_log2) == rows_per_page ? kPow2 : kRows)
+                      : span     ? kSpanFlat
+                                 : kLaneFlat;
 
   for (int l0 = 0; l0 < num_layers; l0 += kMaxLayers) {
     const int nl = num_layers - l0 < kMaxLayers ? num_layers - l0 : kMaxLayers;
@@ -341,24 +397,30 @@ int launch_page_copy(const Side& src, const Side& dst, int num_layers, int64_t n
       p.page_vecs = static_cast<uint32_t>(page_bytes / kVecBytes);
       p.rows_per_page = static_cast<uint32_t>(rows_per_page);
       p.rows_log2 = rows_log2;
+      p.by_page = fast_div(p.page_vecs);
+      p.n_pages = static_cast<uint32_t>(nj);
+      p.total_vecs = static_cast<uint32_t>(nj * p.page_vecs);  // < 2^25 * 64: see max_pages
       if (tee != nullptr) {
         p.tee = tee->base + l0 * tee->layer_stride + j0 * page_bytes;
         p.tee_stride = tee->layer_stride;
       }
-      const dim3 grid(static_cast<uint32_t>(rows_per_page * nj), static_cast<uint32_t>(nl));
+      const int64_t groups = whole_rows ? rows_per_page * nj : (nj * p.page_vecs + kThreads - 1) / kThreads;
+      const dim3 grid(static_cast<uint32_t>(groups), static_cast<uint32_t>(nl));
       const Kind kind = tee != nullptr ? kTee : (policy == StorePolicy::kPack ? kPack : kStream);
       if (inline_ids) {
         CopyParamsInline q;
         q.base = p;
         if (host_src_ids) memcpy(q.src_ids, host_src_ids + j0, nj * sizeof(int32_t));
         if (host_dst_ids) memcpy(q.dst_ids, host_dst_ids + j0, nj * sizeof(int32_t));
-        const int sides = host_src_ids && host_dst_ids ? kBothInline : (host_src_ids ? kSrcInline : kDstInline);
-        const LaunchInlineFn fn = kind == kTee    ? launch_inline_fn<kTee>(guard, pow2, sides)
-                                  : kind == kPack ? launch_inline_fn<kPack>(guard, pow2, sides)
-                                                  : launch_inline_fn<kStream>(guard, pow2, sides);
-        rc = hip_status(fn(q, grid, stream), "page copy launch");
+        const InlineSides sides =
+            host_src_ids && host_dst_ids ? kBothInline : (host_src_ids ? kSrcInline : kDstInline);
+        void* args[] = {&q};
+        rc = hip_status(hipLaunchKernel(pick_inline_kernel(shape, kind, sides), grid, dim3(kThreads), args, 0, stream),
+                        "page copy launch");
       } else {
-        rc = hip_status(kLaunch[guard][kind][pow2](p, grid, stream), "page copy launch");
+        void* args[] = {&p};
+        rc = hip_status(hipLaunchKernel(pick_kernel(shape, kind), grid, dim3(kThreads), args, 0, stream),
+                        "page copy launch");
       }
       if (rc) return rc;
     }

@@ -1,0 +1,83 @@
+"""Pages that are no whole number of 1 KiB rows are copied end to end: pack,
+unpack, move and promotion of pages around the sizes where the split changes
+(32 vectors: 512 bytes) and where a wave holds one, two or many pages, with
+page counts that leave a last wave of one vector, part of it or all of it."""
+import pytest
+import torch
+
+from paceserve_amd.core.block_manager import NativeBlockAllocator
+from paceserve_amd.kv_transfer import ops
+from paceserve_amd.kv_transfer.migrate import KVMigrator
+
+pytestmark = pytest.mark.gpu
+PAGE_BYTES = [32, 64, 480, 496, 512, 544, 1008, 1056, 1536, 3104]
+
+
+def pool(layers, pages, page_bytes, gen, dev):
+    shape = (layers, pages, 2, 1, 1, page_bytes // 2)
+    whole = torch.randint(0, 120, shape, dtype=torch.uint8, generator=gen).to(dev)
+    return whole, list(whole.view(torch.float8_e4m3fn))
+
+
+def ids_of(n, pages, gen, bad):
+    t = torch.randperm(pages, generator=gen)[:n]
+    if bad:
+        t[0], t[n // 2], t[n - 1] = -1, pages, -2 ** 31
+    return t.tolist()
+
+
+def in_pool(ids, pages):
+    return [j for j, p in enumerate(ids) if 0 <= p < pages]
+
+
+@pytest.mark.parametrize("bad", [False, True])
+@pytest.mark.parametrize("n", [1, 2, 33, 1025])
+@pytest.mark.parametrize("page_bytes", PAGE_BYTES)
+def test_pack_unpack_move(gpu, page_bytes, n, bad):
+    L, N = 3, n + 5
+    gen = torch.Generator().manual_seed(page_bytes * 2048 + n)
+    (src, src_l), (dst, dst_l) = pool(L, N, page_bytes, gen, gpu), pool(L, N, page_bytes, gen, gpu)
+    s_ids, d_ids = ids_of(n, N, gen, bad), ids_of(n, N, gen, bad)
+    dev = [torch.tensor(t, dtype=torch.int32, device=gpu) for t in (s_ids, d_ids)]
+    err = torch.zeros(1, dtype=torch.int32, device=gpu)
+    before = dst.cpu()
+
+    buf = torch.zeros((L, n) + tuple(src.shape[2:]), dtype=torch.uint8, device=gpu).view(torch.float8_e4m3fn)
+    ops.pack(src_l, dev[0], buf, err=err)
+    want = torch.zeros((L, n) + tuple(src.shape[2:]), dtype=torch.uint8)
+    ok = in_pool(s_ids, N)
+    want[:, ok] = src.cpu()[:, [s_ids[j] for j in ok]]
+    assert torch.equal(buf.view(torch.uint8).cpu(), want)
+    skipped = n - len(ok)
+    assert int(err.item()) == L * skipped
+
+    ops.unpack(buf, dst_l, dev[1], err=err)
+    ok = in_pool(d_ids, N)
+    want_dst = before.clone()
+    want_dst[:, [d_ids[j] for j in ok]] = want[:, ok]
+    assert torch.equal(dst.cpu(), want_dst)
+    assert int(err.item()) == L * (skipped + n - len(ok))
+
+    dst.copy_(before)
+    err.zero_()
+    ops.move(src_l, dev[0], dst_l, dev[1], err=err)
+    ok = [j for j in in_pool(s_ids, N) if 0 <= d_ids[j] < N]
+    want_dst = before.clone()
+    want_dst[:, [d_ids[j] for j in ok]] = src.cpu()[:, [s_ids[j] for j in ok]]
+    assert torch.equal(dst.cpu(), want_dst)
+    assert int(err.item()) == L * (n - len(ok))
+
+
+@pytest.mark.parametrize("mode", ["fused", "buffer"])
+@pytest.mark.parametrize("n", [1, 33, 512, 513])     # up to 512 ids travel in the kernel arguments
+@pytest.mark.parametrize("page_bytes", PAGE_BYTES)
+def test_promotion(gpu, page_bytes, n, mode):
+    L, N = 3, n + 5
+    gen = torch.Generator().manual_seed(page_bytes * 2048 + n)
+    (src, src_l), (dst, dst_l) = pool(L, N, page_bytes, gen, gpu), pool(L, N, page_bytes, gen, gpu)
+    before = dst.cpu()
+    s_ids, free = ids_of(n, N, gen, False), torch.randperm(N, generator=gen).tolist()
+    plan = KVMigrator(src_l, dst_l, NativeBlockAllocator(1, N, free)).promote([s_ids], mode=mode)
+    want = before.clone()
+    want[:, plan.dst_ids] = src.cpu()[:, s_ids]
+    assert torch.equal(dst.cpu(), want)
