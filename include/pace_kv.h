@@ -187,8 +187,10 @@ int pace_kv_stager_destroy(pace_kv_stager* stager);
  * asynchronous DMA; pageable memory works but the runtime stages it.
  * When the call returns, `stream` is ordered after the last copy enqueued,
  * also when it fails part-way.  A call of one chunk
- * (layers_per_chunk >= num_layers) packs and copies on `stream`, the copy by
- * a 16-wave kernel when host_out is pinned memory the device addresses.
+ * (layers_per_chunk >= num_layers) runs on `stream`: one kernel gathers the
+ * pages into host_out when that is pinned memory the device addresses, on a
+ * 16-byte boundary (a page whose id is out of range stays as it was), else a
+ * pack and a copy.
  *
  * Replaces the gather + pageable device-to-host copy loop of
  * KVhelper.get_kv_cache (paceserve/kv_transfer/kv_utils.py:44-47).
@@ -203,8 +205,9 @@ int pace_kv_pack_to_host(pace_kv_stager* stager,
 /*
  * Unpack from host memory: the mirror of pace_kv_pack_to_host.  Chunk c is
  * copied host-to-device on the H2D side stream while chunk c-1 is unpacked on
- * `stream`; a call of one chunk copies and unpacks on `stream`.  When the
- * call returns, `stream` is ordered after every copy it enqueued, also when
+ * `stream`; a call of one chunk runs on `stream`: one kernel scatters host_in's
+ * pages when that is pinned memory the device addresses, on a 16-byte
+ * boundary, else a copy and an unpack.  When the call returns, `stream` is ordered after every copy it enqueued, also when
  * it fails part-way.
  *
  * Replaces the pageable host-to-device copy + scatter loop of
@@ -269,7 +272,9 @@ int pace_kv_pack_to_host_noalloc(const void* const* src_layers, int num_layers,
  * overlap however the runtime maps these streams onto its hardware queues.
  * Calls on one stager run their packs and unpacks in call order, whichever
  * `stream` each names.  A call of one chunk has nothing to overlap and runs
- * its four stages on `stream`, after the stager's earlier calls.
+ * its stages on `stream`, after the stager's earlier calls: with pinned memory
+ * the device addresses, on a 16-byte boundary, the two kernels of the one-way
+ * calls, else pack, two copies and unpack.
  * host_buf holds host_bytes of host memory used as a ring of chunk-sized
  * regions (host_bytes >= one chunk; pass the full payload to keep a complete
  * host copy, as the reference's KVobj does).

@@ -44,13 +44,16 @@ __device__ __forceinline__ uint32_t over(const FastDiv& d, uint32_t n) {
 }
 #endif
 
-// One side of a page copy: per-layer base pointers plus an optional device
-// page-id array (NULL means page j of layer l is at base[l] + j*page_bytes,
-// which is how the contiguous transfer buffer is addressed).
+// One side of a page copy: per-layer base pointers plus optional page ids, in
+// a device array or (n_pages <= PACE_KV_INLINE_IDS) in a host array whose ids
+// travel in the kernel arguments.  Without either, page j of layer l is at
+// base[l] + j*page_bytes, which is how the contiguous transfer buffer is
+// addressed.
 struct Side {
   const char* const* layers;  // host array, num_layers entries
   const int32_t* ids;         // device array of n_pages ids, or nullptr
   int64_t pool_pages;         // ids must lie in [0, pool_pages)
+  const int32_t* host_ids = nullptr;
 };
 
 // Most page ids per side that a launch carries in its kernel arguments.
@@ -71,15 +74,11 @@ struct Tee {
 
 // Validates arguments and enqueues the copy dst[l][dst_id(j)] = src[l][src_id(j)]
 // for l < num_layers, j < n_pages on `stream`, in launches of at most
-// PACE_KV_MAX_LAYERS_PER_LAUNCH layers.  host_src_ids / host_dst_ids (host
-// arrays, n_pages <= PACE_KV_INLINE_IDS) replace the sides' device ids and
-// travel in the kernel arguments.  With a tee the pools and its buffer must
-// not share memory.
+// PACE_KV_MAX_LAYERS_PER_LAUNCH layers.  With a tee the pools and its buffer
+// must not share memory.
 int launch_page_copy(const Side& src, const Side& dst, int num_layers,
                      int64_t n_pages, int64_t page_bytes, int32_t* err_count,
-                     hipStream_t stream, const int32_t* host_src_ids = nullptr,
-                     const int32_t* host_dst_ids = nullptr,
-                     StorePolicy policy = StorePolicy::kStream, const Tee* tee = nullptr);
+                     hipStream_t stream, StorePolicy policy = StorePolicy::kStream, const Tee* tee = nullptr);
 
 // src -> buffer -> dst in chunks of buffer_layers layers: the bytes of a pack
 // into `buffer` and an unpack out of it, which stays filled.  One launch per
@@ -87,8 +86,15 @@ int launch_page_copy(const Side& src, const Side& dst, int num_layers,
 // destination share memory.  Ids as in launch_page_copy; the caller has
 // checked page_bytes, buffer_layers >= 1 and the buffer's stride.
 int buffered_copy(const Side& src, const Side& dst, char* buffer, int64_t buffer_layer_stride, int buffer_layers,
-                  int num_layers, int64_t n_pages, int64_t page_bytes, int32_t* err_count, hipStream_t stream,
-                  const int32_t* host_src_ids = nullptr, const int32_t* host_dst_ids = nullptr);
+                  int num_layers, int64_t n_pages, int64_t page_bytes, int32_t* err_count, hipStream_t stream);
+
+// Copies pages between a pool and `host`, pinned memory that the device
+// addresses at this pointer, laid out [num_layers][n_pages][page_bytes]: out of
+// the pool (to_host) or into it, in one launch per PACE_KV_MAX_LAYERS_PER_LAUNCH
+// layers.  The arguments are checked as launch_page_copy checks them; a page
+// whose id is outside the pool is left as it was, on either side, and counted.
+int launch_host_leg(const Side& pool, char* host, bool to_host, int num_layers, int64_t n_pages, int64_t page_bytes,
+                    int32_t* err_count, hipStream_t stream);
 
 // Builds the layer table of a contiguous buffer [num_layers][layer_stride].
 void buffer_layers(const void* base, int64_t layer_stride, int num_layers,

@@ -770,9 +770,8 @@ int pack_pages(const void* const* src_layers, int nl, int64_t pool_pages, const 
   std::vector<const char*> buf(static_cast<size_t>(nl));
   pace_kv::buffer_layers(out, stride, nl, buf.data());
   return pace_kv::launch_page_copy(
-      pace_kv::Side{reinterpret_cast<const char* const*>(src_layers), nullptr, pool_pages},
-      pace_kv::Side{buf.data(), nullptr, nj}, nl, nj, page_bytes, err, stream, ids.ptr + j0, nullptr,
-      pace_kv::StorePolicy::kPack);
+      pace_kv::Side{reinterpret_cast<const char* const*>(src_layers), nullptr, pool_pages, ids.ptr + j0},
+      pace_kv::Side{buf.data(), nullptr, nj}, nl, nj, page_bytes, err, stream, pace_kv::StorePolicy::kPack);
 }
 
 // unpack of in[l][j - j0] into pages [j0, j0 + nj) of layers [0, nl), as
@@ -785,8 +784,8 @@ int unpack_pages(const char* in, int64_t stride, void* const* dst_layers, int nl
   pace_kv::buffer_layers(in, stride, nl, buf.data());
   return pace_kv::launch_page_copy(pace_kv::Side{buf.data(), nullptr, nj},
                                    pace_kv::Side{reinterpret_cast<const char* const*>(dst_layers), nullptr,
-                                                 pool_pages},
-                                   nl, nj, page_bytes, err, stream, nullptr, ids.ptr + j0);
+                                                 pool_pages, ids.ptr + j0},
+                                   nl, nj, page_bytes, err, stream);
 }
 
 // ------------------------------------------------------------ device ring

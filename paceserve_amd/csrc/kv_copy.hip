@@ -269,6 +269,115 @@ const void* inline_kernel_of(Kind kind, InlineSides sides) {
   }
 }
 
+// Pages between a pool and pinned host memory, without a device buffer between
+// them.
+//
+// Bound by the link (56-57 GB/s per direction), so what counts is to keep
+// enough of it in flight with few waves: the rest of the chip stays free for
+// whatever other streams run, and more waves slow the other direction's
+// traffic.  Each lane keeps UNROLL vectors in flight and loads the next round's
+// ids behind them.  Measured on MI355X at 14 and 56 MiB, by workgroups of 256:
+//   out, 16 vectors   4: 54.5 and 56.2 GB/s, 6 to 12 within 2% either way
+//   in, 8 vectors     8: 33, 16: 55.4 and 56.8, 24 to 64: 54 to 56.5;
+//                     16 vectors the same or slower
+// Beside host-to-device DMA copies 4 workgroups out keep 48.6 GB/s per
+// direction, 32 workgroups 44; a read stream by waves beside a write stream
+// falls to 28, so only short copies read the host this way.
+constexpr int kHostThreads = 256;
+constexpr int kOutGroups = 4, kOutUnroll = 16;
+constexpr int kInGroups = 16, kInUnroll = 8;
+
+struct HostLegParams {
+  char* layers[kMaxLayers];
+  u32x4* host;             // [layers][n_pages][page_vecs]
+  const int32_t* ids;      // device array; unused by the inline kernel
+  int32_t* err;
+  int64_t page_bytes;
+  uint32_t pool_pages;
+  uint32_t page_vecs;
+  uint32_t n_pages;
+  uint32_t total_vecs;
+  FastDiv by_page;         // division by page_vecs
+  FastDiv by_count;        // division by n_pages
+};
+
+struct HostLegParamsInline {
+  HostLegParams base;
+  int32_t ids[PACE_KV_INLINE_IDS];
+};
+
+// What a lane needs to know of the UNROLL vectors of one round.
+template <int UNROLL>
+struct HostRound {
+  uint32_t k[UNROLL], vec[UNROLL], id[UNROLL];
+  char* base[UNROLL];
+};
+
+template <int UNROLL>
+__device__ __forceinline__ void next_round(const HostLegParams& p, const int32_t* ids, uint32_t i, uint32_t stride,
+                                           HostRound<UNROLL>* r) {
+#pragma unroll
+  for (int u = 0; u < UNROLL; ++u) {
+    r->k[u] = min(i + u * stride, p.total_vecs - 1);
+    const uint32_t at = over(p.by_page, r->k[u]);
+    r->vec[u] = r->k[u] - at * p.page_vecs;
+    const uint32_t layer = over(p.by_count, at);
+    r->base[u] = p.layers[layer];
+    r->id[u] = static_cast<uint32_t>(ids[at - layer * p.n_pages]);
+  }
+}
+
+// The loads of a round are free of branches, so that all of a lane's are in
+// flight together: a vector past the end repeats the last one's and a page id
+// out of range reads the host side, and neither is stored.  The next round's
+// ids are loaded behind this round's vectors.
+template <bool TO_HOST, int UNROLL>
+__device__ __forceinline__ void host_leg(const HostLegParams& p, const int32_t* ids) {
+  const uint32_t stride = gridDim.x * kHostThreads;
+  uint32_t i = blockIdx.x * kHostThreads + threadIdx.x;
+  HostRound<UNROLL> r;
+  next_round(p, ids, i, stride, &r);
+  for (; i < p.total_vecs; i += UNROLL * stride) {
+    u32x4* pool[UNROLL];
+    u32x4 v[UNROLL];
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      pool[u] = reinterpret_cast<u32x4*>(r.base[u] + static_cast<int64_t>(r.id[u]) * p.page_bytes) + r.vec[u];
+      const u32x4* from = p.host + r.k[u];
+      if (TO_HOST) {
+        // The compiler must not see what the choice is between: it would put
+        // the address, and the loads it needs, behind a branch per vector.
+        uint64_t in_pool = reinterpret_cast<uint64_t>(pool[u]), on_host = reinterpret_cast<uint64_t>(from);
+        asm("" : "+v"(in_pool), "+v"(on_host));
+        from = reinterpret_cast<const u32x4*>(r.id[u] < p.pool_pages ? in_pool : on_host);
+      }
+      v[u] = __builtin_nontemporal_load(reinterpret_cast<const __attribute__((address_space(1))) u32x4*>(
+          reinterpret_cast<uint64_t>(from)));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    HostRound<UNROLL> ahead;
+    next_round(p, ids, i + UNROLL * stride, stride, &ahead);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      if (i + u * stride >= p.total_vecs) continue;
+      if (r.id[u] < p.pool_pages) store_vec<false>(v[u], TO_HOST ? p.host + r.k[u] : pool[u]);
+      else if (r.vec[u] == 0 && p.err != nullptr) atomicAdd(p.err, 1);
+    }
+    r = ahead;
+  }
+}
+
+template <bool TO_HOST>
+__global__ __launch_bounds__(kHostThreads) void host_leg_kernel(const HostLegParams p) {
+  host_leg<TO_HOST, TO_HOST ? kOutUnroll : kInUnroll>(p, p.ids);
+}
+
+template <bool TO_HOST>
+__global__ __launch_bounds__(kHostThreads) void host_leg_inline_kernel(const HostLegParamsInline p) {
+  host_leg<TO_HOST, TO_HOST ? kOutUnroll : kInUnroll>(p.base, p.ids);
+}
+
 const void* pick_kernel(Shape shape, Kind kind) {
   switch (shape) {
     case kPow2: return kernel_of<kPow2>(kind);
@@ -325,9 +434,9 @@ void buffer_layers(const void* base, int64_t layer_stride, int num_layers, const
 }
 
 int launch_page_copy(const Side& src, const Side& dst, int num_layers, int64_t n_pages,
-                     int64_t page_bytes, int32_t* err_count, hipStream_t stream,
-                     const int32_t* host_src_ids, const int32_t* host_dst_ids,
-                     StorePolicy policy, const Tee* tee) {
+                     int64_t page_bytes, int32_t* err_count, hipStream_t stream, StorePolicy policy,
+                     const Tee* tee) {
+  const int32_t *const host_src_ids = src.host_ids, *const host_dst_ids = dst.host_ids;
   if (num_layers < 0) return fail(PACE_KV_EINVAL, "num_layers must be >= 0 (got %d)", num_layers);
   if (n_pages < 0) return fail(PACE_KV_EINVAL, "n_pages must be >= 0 (got %lld)", (long long)n_pages);
   if (page_bytes <= 0 || page_bytes % kVecBytes != 0)
@@ -450,9 +559,59 @@ bool disjoint(const char* const* a, int64_t a_bytes, const char* const* b, int64
 
 }  // namespace
 
+int launch_host_leg(const Side& pool, char* host, bool to_host, int num_layers, int64_t n_pages, int64_t page_bytes,
+                    int32_t* err_count, hipStream_t stream) {
+  if (num_layers < 0 || n_pages < 0 || pool.pool_pages < 0) return fail(PACE_KV_EINVAL, "host leg: negative size");
+  if (page_bytes <= 0 || page_bytes % kVecBytes != 0)
+    return fail(PACE_KV_EINVAL, "page_bytes must be a positive multiple of 16 (got %lld)", (long long)page_bytes);
+  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
+  if (host == nullptr || !aligned16(host)) return fail(PACE_KV_EINVAL, "host buffer is NULL or not 16-byte aligned");
+  PACE_KV_TRY(check_layers(pool.layers, num_layers, to_host ? "source" : "destination"));
+  if (pool.ids == nullptr && pool.host_ids == nullptr) return fail(PACE_KV_EINVAL, "host leg: NULL page_ids");
+  if (reinterpret_cast<uintptr_t>(pool.ids) & 3u) return fail(PACE_KV_EINVAL, "page ids are not 4-byte aligned");
+  if (pool.host_ids != nullptr && n_pages > PACE_KV_INLINE_IDS)
+    return fail(PACE_KV_ERANGE, "more than %d pages cannot travel in the kernel arguments", PACE_KV_INLINE_IDS);
+  constexpr int64_t kMaxVecs = int64_t(1) << 31;  // of one launch: 32-bit indexes, with room for a round past the end
+  const int64_t page_vecs = page_bytes / kVecBytes;
+  if (n_pages > kMaxVecs / page_vecs) return fail(PACE_KV_ERANGE, "host leg: a layer of more than 32 GiB");
+  const int64_t fit = kMaxVecs / (n_pages * page_vecs);
+  const int step = static_cast<int>(std::min<int64_t>({fit, kMaxLayers, num_layers}));
+  for (int l0 = 0; l0 < num_layers; l0 += step) {
+    const int nl = std::min(step, num_layers - l0);
+    HostLegParamsInline q;
+    memset(&q.base, 0, sizeof(q.base));
+    HostLegParams& p = q.base;
+    for (int l = 0; l < nl; ++l) p.layers[l] = const_cast<char*>(pool.layers[l0 + l]);
+    p.host = reinterpret_cast<u32x4*>(host + l0 * n_pages * page_bytes);
+    p.ids = pool.ids;
+    p.err = err_count;
+    p.page_bytes = page_bytes;
+    p.pool_pages = static_cast<uint32_t>(std::min<int64_t>(pool.pool_pages, INT32_MAX));
+    p.page_vecs = static_cast<uint32_t>(page_vecs);
+    p.n_pages = static_cast<uint32_t>(n_pages);
+    p.total_vecs = static_cast<uint32_t>(nl * n_pages * page_vecs);
+    p.by_page = fast_div(p.page_vecs);
+    p.by_count = fast_div(p.n_pages);
+    const int64_t most = (p.total_vecs + kHostThreads - 1) / kHostThreads;
+    const dim3 grid(static_cast<uint32_t>(std::min<int64_t>(to_host ? kOutGroups : kInGroups, most)));
+    const void* fn;
+    void* args[] = {&q};
+    if (pool.host_ids != nullptr) {
+      memcpy(q.ids, pool.host_ids, n_pages * sizeof(int32_t));
+      fn = to_host ? reinterpret_cast<const void*>(&host_leg_inline_kernel<true>)
+                   : reinterpret_cast<const void*>(&host_leg_inline_kernel<false>);
+    } else {
+      fn = to_host ? reinterpret_cast<const void*>(&host_leg_kernel<true>)
+                   : reinterpret_cast<const void*>(&host_leg_kernel<false>);
+      args[0] = &p;
+    }
+    PACE_KV_TRY(hip_status(hipLaunchKernel(fn, grid, dim3(kHostThreads), args, 0, stream), "host leg launch"));
+  }
+  return PACE_KV_OK;
+}
+
 int buffered_copy(const Side& src, const Side& dst, char* buffer, int64_t buffer_layer_stride, int buffer_layers,
-                  int num_layers, int64_t n_pages, int64_t page_bytes, int32_t* err_count, hipStream_t stream,
-                  const int32_t* host_src_ids, const int32_t* host_dst_ids) {
+                  int num_layers, int64_t n_pages, int64_t page_bytes, int32_t* err_count, hipStream_t stream) {
   if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
   PACE_KV_TRY(check_layers(src.layers, num_layers, "source"));
   PACE_KV_TRY(check_layers(dst.layers, num_layers, "destination"));
@@ -477,17 +636,16 @@ int buffered_copy(const Side& src, const Side& dst, char* buffer, int64_t buffer
   }
   for (int l0 = 0; l0 < num_layers; l0 += nb) {
     const int nl = num_layers - l0 < nb ? num_layers - l0 : nb;
-    const Side s{src.layers + l0, src.ids, src.pool_pages}, d{dst.layers + l0, dst.ids, dst.pool_pages};
+    const Side s{src.layers + l0, src.ids, src.pool_pages, src.host_ids};
+    const Side d{dst.layers + l0, dst.ids, dst.pool_pages, dst.host_ids};
     if (tee) {
       const Tee t{buffer, buffer_layer_stride};
-      PACE_KV_TRY(launch_page_copy(s, d, nl, n_pages, page_bytes, err_count, stream, host_src_ids, host_dst_ids,
-                                   StorePolicy::kStream, &t));
+      PACE_KV_TRY(launch_page_copy(s, d, nl, n_pages, page_bytes, err_count, stream, StorePolicy::kStream, &t));
       continue;
     }
     const Side b{buf.data(), nullptr, n_pages};
-    PACE_KV_TRY(launch_page_copy(s, b, nl, n_pages, page_bytes, err_count, stream, host_src_ids, nullptr,
-                                 StorePolicy::kPack));
-    PACE_KV_TRY(launch_page_copy(b, d, nl, n_pages, page_bytes, err_count, stream, nullptr, host_dst_ids));
+    PACE_KV_TRY(launch_page_copy(s, b, nl, n_pages, page_bytes, err_count, stream, StorePolicy::kPack));
+    PACE_KV_TRY(launch_page_copy(b, d, nl, n_pages, page_bytes, err_count, stream));
   }
   return PACE_KV_OK;
 }
@@ -586,8 +744,7 @@ int pace_kv_pack(const void* const* src_layers, int num_layers, int64_t pool_pag
   Side src{reinterpret_cast<const char* const*>(src_layers), page_ids, pool_pages};
   Side dst{buf.data(), nullptr, n_pages};
   return pace_kv::launch_page_copy(src, dst, num_layers, n_pages, page_bytes, err_count,
-                                   static_cast<hipStream_t>(stream), nullptr, nullptr,
-                                   pace_kv::StorePolicy::kPack);
+                                   static_cast<hipStream_t>(stream), pace_kv::StorePolicy::kPack);
 }
 
 int pace_kv_unpack(const void* buf, int64_t buf_layer_stride, void* const* dst_layers,

@@ -167,14 +167,12 @@ int promote_inline(pace_kv_promoter* pr, pace_kv_allocator* dst_alloc,
   const char* const* dst_tab = reinterpret_cast<const char* const*>(dst_layers);
   int rc = PACE_KV_OK;
   if (n > 0 && num_layers > 0) {
+    const Side src{src_tab, nullptr, src_pool_pages, src_ids}, dst{dst_tab, nullptr, dst_pool_pages, dst_ids};
     if (buffer == nullptr) {
-      rc = pace_kv::launch_page_copy(Side{src_tab, nullptr, src_pool_pages},
-                                     Side{dst_tab, nullptr, dst_pool_pages}, num_layers, n,
-                                     page_bytes, err_count, stream, src_ids, dst_ids);
+      rc = pace_kv::launch_page_copy(src, dst, num_layers, n, page_bytes, err_count, stream);
     } else {
-      rc = pace_kv::buffered_copy(Side{src_tab, nullptr, src_pool_pages}, Side{dst_tab, nullptr, dst_pool_pages},
-                                  static_cast<char*>(buffer), buffer_layer_stride, buffer_layers, num_layers, n,
-                                  page_bytes, err_count, stream, src_ids, dst_ids);
+      rc = pace_kv::buffered_copy(src, dst, static_cast<char*>(buffer), buffer_layer_stride, buffer_layers, num_layers,
+                                  n, page_bytes, err_count, stream);
     }
   }
   if (rc) {

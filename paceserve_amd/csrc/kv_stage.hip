@@ -41,11 +41,17 @@
 // and 4096-token requests and within 2% either way for 256-1024 and 8192
 // tokens.
 //
-// A call whose layers fit one chunk has nothing to overlap, so all its stages
-// run on the caller's stream: each wait between streams adds latency, 30-36 us
-// per call on 2-8 MiB requests.  Its device-to-host copy is the copy kernel
-// too, which follows a pack on the same stream sooner than a DMA copy does;
-// so is the allocation-free pack's.
+// A call whose layers fit one chunk has nothing to overlap, so it runs on the
+// caller's stream: each wait between streams adds latency, 30-36 us per call
+// on 2-8 MiB requests.  With pinned host memory it needs no device slot
+// either: one kernel per direction copies between the pages and the host
+// (launch_host_leg).  Measured on MI355X against a pack and a copy kernel, and
+// against a DMA copy and an unpack: 2 MiB 59-63 -> 48 us out and 61 -> 44 in,
+// 14 MiB 284 -> 269 and 284 -> 265, 56 MiB 1067 -> 1046 and 1065 -> 1034.  In
+// the pipeline of several chunks it gained nothing: there the link is busy in
+// both directions, and packs and unpacks already hide under its copies.
+// The allocation-free pack copies with the copy kernel, which follows a pack
+// on the same stream sooner than a DMA copy does.
 //
 // Device slots are reused round-robin; before a slot is overwritten, the
 // stream that writes it waits for the event recorded after the last read of
@@ -301,6 +307,11 @@ hipError_t copy_to_host(void* host, const void* dev, int64_t bytes, bool kernel,
   return hipGetLastError();
 }
 
+// Whether launch_host_leg can copy `bytes` of `host` directly.
+bool direct_host(const void* host, int64_t bytes) {
+  return reinterpret_cast<uintptr_t>(host) % 16 == 0 && device_addressable_host(host, bytes);
+}
+
 // pack(chunk c) of the source pool into out slot `slot`, on `stream`.
 int pack_chunk(pace_kv_stager* s, const ChunkPlan& p, int c, const void* const* src_layers,
                int64_t pool_pages, const int32_t* ids, int32_t* err, hipStream_t stream) {
@@ -417,17 +428,20 @@ int pace_kv_pack_to_host(pace_kv_stager* s, const void* const* src_layers, int n
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   const int chunks = p.num_chunks();
   if (chunks == 1) {
-    // One chunk leaves nothing to overlap: the pack and the copy run on
-    // `stream`, without the waits between streams (measured on MI355X: 30-36
-    // us less per call for 2-8 MiB requests, about 1% less at 128 MiB).  The
-    // copy kernel starts sooner after the pack than a DMA copy does (62 against
-    // 73 us for 2 MiB, the same from 32 MiB).
+    // One chunk leaves nothing to overlap, so everything runs on `stream`,
+    // without the waits between streams (measured on MI355X: 30-36 us less per
+    // call for 2-8 MiB requests, about 1% less at 128 MiB).
+    const int64_t bytes = p.num_layers * p.layer_bytes;
+    if (direct_host(host_out, bytes)) {
+      const pace_kv::Side src{reinterpret_cast<const char* const*>(src_layers), page_ids, pool_pages};
+      return pace_kv::launch_host_leg(src, static_cast<char*>(host_out), true, num_layers, n_pages, page_bytes,
+                                      err_count, stream);
+    }
     PACE_HIP(hipStreamWaitEvent(stream, s->out_free[0], 0), "wait out slot");
     PACE_KV_TRY(pack_chunk(s, p, 0, src_layers, pool_pages, page_ids, err_count, stream));
     // out_free follows the pack also when the copy fails to enqueue.
-    const int64_t bytes = p.count(0) * p.layer_bytes;
     const hipError_t d2h =
-        copy_to_host(host_out, s->out_ring, bytes, device_addressable_host(host_out, bytes), stream);
+        hipMemcpyAsync(host_out, s->out_ring, static_cast<size_t>(bytes), hipMemcpyDeviceToHost, stream);
     PACE_HIP(hipEventRecord(s->out_free[0], stream), "record out_free");
     PACE_HIP(d2h, "D2H copy");
     return PACE_KV_OK;
@@ -473,10 +487,15 @@ int pace_kv_unpack_from_host(pace_kv_stager* s, const void* host_in, void* const
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   const int chunks = p.num_chunks();
   if (chunks == 1) {
-    // One chunk: the copy and the unpack run on `stream` (as in the pack).
+    // One chunk: everything runs on `stream` (as in the pack).
+    const int64_t bytes = p.num_layers * p.layer_bytes;
+    if (direct_host(host_in, bytes)) {
+      const pace_kv::Side dst{reinterpret_cast<const char* const*>(dst_layers), page_ids, pool_pages};
+      return pace_kv::launch_host_leg(dst, const_cast<char*>(static_cast<const char*>(host_in)), false, num_layers,
+                                      n_pages, page_bytes, err_count, stream);
+    }
     PACE_HIP(hipStreamWaitEvent(stream, s->in_free[0], 0), "wait in slot");
-    PACE_HIP(hipMemcpyAsync(s->in_ring, host_in, p.count(0) * p.layer_bytes, hipMemcpyHostToDevice, stream),
-             "H2D copy");
+    PACE_HIP(hipMemcpyAsync(s->in_ring, host_in, bytes, hipMemcpyHostToDevice, stream), "H2D copy");
     // in_free follows the copy also when the unpack fails to launch.
     const int rc = unpack_chunk(s, p, 0, dst_layers, pool_pages, page_ids, err_count, stream);
     PACE_HIP(hipEventRecord(s->in_free[0], stream), "record in_free");
@@ -533,21 +552,33 @@ int pace_kv_roundtrip(pace_kv_stager* s, const void* const* src_layers, int64_t 
   PACE_HIP(make_events(s->host_full, regions), "create host events");
   PACE_HIP(make_events(s->host_free, regions), "create host events");
   char* host = static_cast<char*>(host_buf);
-  const bool host_kernel = device_addressable_host(host_buf, regions * chunk_bytes);
+  const bool host_kernel = direct_host(host_buf, regions * chunk_bytes);
   if (chunks == 1) {
-    // One chunk leaves nothing to overlap: its four stages run on the
-    // caller's stream, without the waits between streams.  They follow the
-    // packs and unpacks of earlier calls on this stager (work_done), the last
-    // reads of both slots and the previous call's last read of its host
-    // buffer, and leave the records a later call waits on.
+    // One chunk leaves nothing to overlap: its stages run on the caller's
+    // stream, without the waits between streams.  They follow the packs and
+    // unpacks of earlier calls on this stager (work_done), the last reads of
+    // both slots and the previous call's last read of its host buffer, and
+    // leave the records a later call waits on.
     hipStream_t caller = static_cast<hipStream_t>(stream_);
     const int64_t bytes = p.count(0) * p.layer_bytes;
     PACE_HIP(hipStreamWaitEvent(caller, s->work_done, 0), "wait earlier calls");
-    PACE_HIP(hipStreamWaitEvent(caller, s->out_free[0], 0), "wait out slot");
     PACE_HIP(hipStreamWaitEvent(caller, s->h2d_done, 0), "wait previous round trip");
+    if (host_kernel) {
+      const pace_kv::Side src{reinterpret_cast<const char* const*>(src_layers), src_ids, src_pool_pages};
+      const pace_kv::Side dst{reinterpret_cast<const char* const*>(dst_layers), dst_ids, dst_pool_pages};
+      PACE_KV_TRY(pace_kv::launch_host_leg(src, host, true, num_layers, n_pages, page_bytes, err_count, caller));
+      // The records follow what was enqueued also when the way back fails to launch.
+      const int rc =
+          pace_kv::launch_host_leg(dst, host, false, num_layers, n_pages, page_bytes, err_count, caller);
+      PACE_HIP(hipEventRecord(s->h2d_done, caller), "record h2d_done");
+      PACE_HIP(hipEventRecord(s->work_done, caller), "record work_done");
+      return rc;
+    }
+    PACE_HIP(hipStreamWaitEvent(caller, s->out_free[0], 0), "wait out slot");
     PACE_KV_TRY(pack_chunk(s, p, 0, src_layers, src_pool_pages, src_ids, err_count, caller));
     // out_free follows the pack also when the copy fails to enqueue.
-    const hipError_t d2h = copy_to_host(host, s->out_ring, bytes, host_kernel, caller);
+    const hipError_t d2h =
+        hipMemcpyAsync(host, s->out_ring, static_cast<size_t>(bytes), hipMemcpyDeviceToHost, caller);
     PACE_HIP(hipEventRecord(s->out_free[0], caller), "record out_free");
     PACE_HIP(d2h, "D2H copy");
     PACE_HIP(hipStreamWaitEvent(caller, s->in_free[0], 0), "wait in slot");

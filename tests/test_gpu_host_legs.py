@@ -1,0 +1,77 @@
+"""One-chunk copies between pages and pinned host memory go in one kernel per
+direction: payloads of less than a round of its lanes, exactly one round, one
+vector more and many, pages that fill, miss or straddle a KiB, more layers than
+a launch takes, and page ids outside the pool."""
+import pytest
+import torch
+
+from paceserve_amd.kv_transfer import ops
+
+pytestmark = pytest.mark.gpu
+# A round is 4 workgroups x 256 lanes x 16 vectors out (256 KiB) and 16 x 256 x
+# 8 in (512 KiB).  (layers, pages, page bytes)
+SHAPES = [(1, 1, 32), (3, 5, 160), (1, 16, 16384), (1, 32, 16384), (2, 8193, 32), (4, 33, 1056), (70, 3, 2048),
+          (5, 40, 65536)]
+
+
+def pool(layers, pages, page_bytes, gen, dev):
+    shape = (layers, pages, 2, 1, 1, page_bytes // 2)
+    whole = torch.randint(0, 120, shape, dtype=torch.uint8, generator=gen).to(dev)
+    return whole, list(whole.view(torch.float8_e4m3fn))
+
+
+@pytest.mark.parametrize("bad", [False, True])
+@pytest.mark.parametrize("layers,n,page_bytes", SHAPES)
+def test_out_in_and_round_trip(gpu, layers, n, page_bytes, bad):
+    N = n + 5
+    gen = torch.Generator().manual_seed(n * page_bytes)
+    (src, src_l), (dst, dst_l) = pool(layers, N, page_bytes, gen, gpu), pool(layers, N, page_bytes, gen, gpu)
+    s_ids, d_ids = torch.randperm(N, generator=gen)[:n], torch.randperm(N, generator=gen)[:n]
+    if bad:
+        s_ids[0], s_ids[n - 1], d_ids[n // 2] = -1, N, -2 ** 31
+    s_ok, d_ok = (s_ids >= 0) & (s_ids < N), (d_ids >= 0) & (d_ids < N)
+    ids = [t.to(torch.int32).to(gpu) for t in (s_ids, d_ids)]
+    err = torch.zeros(1, dtype=torch.int32, device=gpu)
+    before = dst.cpu()
+    host = torch.full((layers, n) + tuple(src.shape[2:]), 121, dtype=torch.uint8, pin_memory=True)
+    want = host.clone()
+    want[:, s_ok] = src.cpu()[:, s_ids[s_ok]]
+    want_dst = before.clone()
+    want_dst[:, d_ids[d_ok]] = want[:, d_ok]
+    content = host.view(torch.float8_e4m3fn)
+    with ops.Stager(-(-layers * n * page_bytes // 256) * 256, 2) as st:
+        st.pack_to_host(src_l, ids[0], content, layers, err=err)
+        torch.cuda.synchronize()
+        assert torch.equal(host, want)
+        assert int(err.item()) == layers * int((~s_ok).sum())
+        st.unpack_from_host(content, dst_l, ids[1], layers, err=err)
+        assert torch.equal(dst.cpu(), want_dst)
+        assert int(err.item()) == layers * int((~s_ok).sum() + (~d_ok).sum())
+
+        dst.copy_(before)
+        host.fill_(121)
+        st.roundtrip(src_l, ids[0], dst_l, ids[1], content, layers)
+        torch.cuda.synchronize()
+        assert torch.equal(host, want)
+        assert torch.equal(dst.cpu(), want_dst)
+
+
+def test_host_memory_that_no_kernel_copies(gpu):
+    """Pageable memory, and pinned memory off a 16-byte boundary, still go
+    through the device slots."""
+    layers, n, page_bytes = 3, 7, 1056
+    gen = torch.Generator().manual_seed(1)
+    (src, src_l), (dst, dst_l) = pool(layers, n, page_bytes, gen, gpu), pool(layers, n, page_bytes, gen, gpu)
+    ids = torch.randperm(n, generator=gen)
+    size = layers * n * page_bytes
+    for raw in (torch.empty(size, dtype=torch.uint8), torch.empty(size + 8, dtype=torch.uint8, pin_memory=True)[8:]):
+        host = raw.view(torch.float8_e4m3fn)
+        with ops.Stager(-(-size // 256) * 256, 2) as st:
+            st.pack_to_host(src_l, ids, host, layers)
+            torch.cuda.synchronize()
+            assert torch.equal(raw.view(layers, n, -1), src.cpu()[:, ids].reshape(layers, n, -1))
+            st.unpack_from_host(host, dst_l, ids, layers)
+            assert torch.equal(dst.cpu()[:, ids], src.cpu()[:, ids])
+            dst.zero_()
+            st.roundtrip(src_l, ids, dst_l, ids, host, layers)
+            assert torch.equal(dst.cpu()[:, ids], src.cpu()[:, ids])
