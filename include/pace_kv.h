@@ -65,6 +65,10 @@ const char* pace_kv_last_error(void);
 /* Device-to-device page copies                                              */
 /* ------------------------------------------------------------------------ */
 
+/* Most page ids that a call with ids in host memory takes (the _inline calls
+ * below, pace_kv_channel_send and pace_kv_channel_recv). */
+#define PACE_KV_INLINE_IDS 512
+
 /*
  * PACK (multi-layer gather).
  *   out[l][j] = src_layers[l][page_ids[j]]   for l < num_layers, j < n_pages
@@ -98,6 +102,23 @@ int pace_kv_unpack(const void* buf, int64_t buf_layer_stride,
                    void* const* dst_layers, int num_layers, int64_t pool_pages,
                    const int32_t* page_ids, int64_t n_pages, int64_t page_bytes,
                    int32_t* err_count, void* stream);
+
+/*
+ * PACK and UNPACK with the page ids in host memory (pageable or pinned, at most
+ * PACE_KV_INLINE_IDS of them, else PACE_KV_ERANGE): they are read during the
+ * call and travel in the kernel arguments, so no upload precedes the copy.
+ * Everything else is as above.
+ */
+int pace_kv_pack_inline(const void* const* src_layers, int num_layers,
+                        int64_t pool_pages, const int32_t* host_page_ids,
+                        int64_t n_pages, int64_t page_bytes, void* out,
+                        int64_t out_layer_stride, int32_t* err_count,
+                        void* stream);
+int pace_kv_unpack_inline(const void* buf, int64_t buf_layer_stride,
+                          void* const* dst_layers, int num_layers,
+                          int64_t pool_pages, const int32_t* host_page_ids,
+                          int64_t n_pages, int64_t page_bytes,
+                          int32_t* err_count, void* stream);
 
 /*
  * MOVE (pack and unpack fused, pool to pool on one device, no transfer buffer).
@@ -219,6 +240,24 @@ int pace_kv_unpack_from_host(pace_kv_stager* stager, const void* host_in,
                              int64_t n_pages, int64_t page_bytes,
                              int layers_per_chunk, int32_t* err_count,
                              void* stream);
+
+/*
+ * The two one-way calls with the page ids in host memory, as
+ * pace_kv_pack_inline and pace_kv_unpack_inline take them.
+ */
+int pace_kv_pack_to_host_inline(pace_kv_stager* stager,
+                                const void* const* src_layers, int num_layers,
+                                int64_t pool_pages, const int32_t* host_page_ids,
+                                int64_t n_pages, int64_t page_bytes,
+                                int layers_per_chunk, void* host_out,
+                                int32_t* err_count, void* stream);
+int pace_kv_unpack_from_host_inline(pace_kv_stager* stager, const void* host_in,
+                                    void* const* dst_layers, int num_layers,
+                                    int64_t pool_pages,
+                                    const int32_t* host_page_ids,
+                                    int64_t n_pages, int64_t page_bytes,
+                                    int layers_per_chunk, int32_t* err_count,
+                                    void* stream);
 
 /* Bytes of the device scratch array through which
  * pace_kv_pack_to_host_noalloc stages its chunks (64 MiB per GPU). */

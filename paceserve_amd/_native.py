@@ -19,6 +19,7 @@ LIB_PATH = Path(__file__).resolve().parent / "libpace_kv.so"
 ABI_VERSION = 2
 MAX_LAYERS_PER_LAUNCH = 64
 NOALLOC_SCRATCH_BYTES = 64 << 20
+INLINE_IDS = 512
 
 PACE_KV_OK = 0
 PACE_KV_EINVAL = -1
@@ -35,6 +36,8 @@ SIGNATURES = {
     "pace_kv_abi_version": (c_int, []),
     "pace_kv_last_error": (c_char_p, []),
     "pace_kv_pack": (c_int, [_VP, c_int, c_int64, _VP, c_int64, c_int64, _VP, c_int64, _VP, _VP]),
+    "pace_kv_pack_inline": (c_int, [_VP, c_int, c_int64, _VP, c_int64, c_int64, _VP, c_int64, _VP, _VP]),
+    "pace_kv_unpack_inline": (c_int, [_VP, c_int64, _VP, c_int, c_int64, _VP, c_int64, c_int64, _VP, _VP]),
     "pace_kv_unpack": (c_int, [_VP, c_int64, _VP, c_int, c_int64, _VP, c_int64, c_int64, _VP, _VP]),
     "pace_kv_move": (c_int, [_VP, c_int64, _VP, _VP, c_int64, _VP, c_int, c_int64, c_int64, _VP, _VP]),
     "pace_kv_move_buffered": (
@@ -46,6 +49,10 @@ SIGNATURES = {
     "pace_kv_pack_to_host": (
         c_int, [_VP, _VP, c_int, c_int64, _VP, c_int64, c_int64, c_int, _VP, _VP, _VP]),
     "pace_kv_unpack_from_host": (
+        c_int, [_VP, _VP, _VP, c_int, c_int64, _VP, c_int64, c_int64, c_int, _VP, _VP]),
+    "pace_kv_pack_to_host_inline": (
+        c_int, [_VP, _VP, c_int, c_int64, _VP, c_int64, c_int64, c_int, _VP, _VP, _VP]),
+    "pace_kv_unpack_from_host_inline": (
         c_int, [_VP, _VP, _VP, c_int, c_int64, _VP, c_int64, c_int64, c_int, _VP, _VP]),
     "pace_kv_append": (
         c_int, [_VP, _VP, c_int64, c_int64, _VP, _VP, c_int, _VP, c_int64, _VP, c_int64, _VP, c_int,

@@ -56,8 +56,13 @@ struct Side {
   const int32_t* host_ids = nullptr;
 };
 
-// Most page ids per side that a launch carries in its kernel arguments.
-#define PACE_KV_INLINE_IDS 512
+// The page ids of one side of a call: a device array, or a host array of at
+// most PACE_KV_INLINE_IDS entries that travel in the kernel arguments.
+struct IdList {
+  const int32_t* dev;
+  const int32_t* host;
+  bool null() const { return dev == nullptr && host == nullptr; }
+};
 
 // Store flavour of a copy: both write through the L2 at device scope; kStream
 // also marks the stores nontemporal, while kPack (a pack into a transfer
@@ -95,6 +100,12 @@ int buffered_copy(const Side& src, const Side& dst, char* buffer, int64_t buffer
 // whose id is outside the pool is left as it was, on either side, and counted.
 int launch_host_leg(const Side& pool, char* host, bool to_host, int num_layers, int64_t n_pages, int64_t page_bytes,
                     int32_t* err_count, hipStream_t stream);
+
+// pace_kv_pack and pace_kv_unpack for ids of either kind.
+int pack(const void* const* src_layers, int num_layers, int64_t pool_pages, const IdList& ids, int64_t n_pages,
+         int64_t page_bytes, void* out, int64_t out_layer_stride, int32_t* err_count, hipStream_t stream);
+int unpack(const void* buf, int64_t buf_layer_stride, void* const* dst_layers, int num_layers, int64_t pool_pages,
+           const IdList& ids, int64_t n_pages, int64_t page_bytes, int32_t* err_count, hipStream_t stream);
 
 // Builds the layer table of a contiguous buffer [num_layers][layer_stride].
 void buffer_layers(const void* base, int64_t layer_stride, int num_layers,

@@ -650,6 +650,40 @@ int buffered_copy(const Side& src, const Side& dst, char* buffer, int64_t buffer
   return PACE_KV_OK;
 }
 
+int pack(const void* const* src_layers, int num_layers, int64_t pool_pages, const IdList& ids, int64_t n_pages,
+         int64_t page_bytes, void* out, int64_t out_layer_stride, int32_t* err_count, hipStream_t stream) {
+  if (num_layers < 0) return fail(PACE_KV_EINVAL, "num_layers must be >= 0");
+  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
+  if (ids.null() || out == nullptr) return fail(PACE_KV_EINVAL, "pack: NULL page_ids or out");
+  if (n_pages > 0 && page_bytes > 0 &&
+      (n_pages > INT64_MAX / page_bytes || out_layer_stride < n_pages * page_bytes))
+    return fail(PACE_KV_ERANGE, "pack: out_layer_stride %lld < n_pages*page_bytes",
+                (long long)out_layer_stride);
+  if (out_layer_stride % 16 != 0) return fail(PACE_KV_EINVAL, "pack: out_layer_stride not a multiple of 16");
+  std::vector<const char*> buf(num_layers);
+  buffer_layers(out, out_layer_stride, num_layers, buf.data());
+  const Side src{reinterpret_cast<const char* const*>(src_layers), ids.dev, pool_pages, ids.host};
+  const Side dst{buf.data(), nullptr, n_pages};
+  return launch_page_copy(src, dst, num_layers, n_pages, page_bytes, err_count, stream, StorePolicy::kPack);
+}
+
+int unpack(const void* buf, int64_t buf_layer_stride, void* const* dst_layers, int num_layers, int64_t pool_pages,
+           const IdList& ids, int64_t n_pages, int64_t page_bytes, int32_t* err_count, hipStream_t stream) {
+  if (num_layers < 0) return fail(PACE_KV_EINVAL, "num_layers must be >= 0");
+  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
+  if (ids.null() || buf == nullptr) return fail(PACE_KV_EINVAL, "unpack: NULL page_ids or buf");
+  if (n_pages > 0 && page_bytes > 0 &&
+      (n_pages > INT64_MAX / page_bytes || buf_layer_stride < n_pages * page_bytes))
+    return fail(PACE_KV_ERANGE, "unpack: buf_layer_stride %lld < n_pages*page_bytes",
+                (long long)buf_layer_stride);
+  if (buf_layer_stride % 16 != 0) return fail(PACE_KV_EINVAL, "unpack: buf_layer_stride not a multiple of 16");
+  std::vector<const char*> src_tab(num_layers);
+  buffer_layers(buf, buf_layer_stride, num_layers, src_tab.data());
+  const Side src{src_tab.data(), nullptr, n_pages};
+  const Side dst{reinterpret_cast<const char* const*>(dst_layers), ids.dev, pool_pages, ids.host};
+  return launch_page_copy(src, dst, num_layers, n_pages, page_bytes, err_count, stream);
+}
+
 // Resolves num_layers host or device layer pointers to the addresses the
 // kernel uses, after checking that each lies in a registered allocation of
 // the expected kind (pinned host memory mapped for the device, or device
@@ -731,39 +765,29 @@ const char* pace_kv_last_error(void) { return pace_kv::g_last_error; }
 int pace_kv_pack(const void* const* src_layers, int num_layers, int64_t pool_pages,
                  const int32_t* page_ids, int64_t n_pages, int64_t page_bytes, void* out,
                  int64_t out_layer_stride, int32_t* err_count, void* stream) {
-  if (num_layers < 0) return fail(PACE_KV_EINVAL, "num_layers must be >= 0");
-  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
-  if (page_ids == nullptr || out == nullptr) return fail(PACE_KV_EINVAL, "pack: NULL page_ids or out");
-  if (n_pages > 0 && page_bytes > 0 &&
-      (n_pages > INT64_MAX / page_bytes || out_layer_stride < n_pages * page_bytes))
-    return fail(PACE_KV_ERANGE, "pack: out_layer_stride %lld < n_pages*page_bytes",
-                (long long)out_layer_stride);
-  if (out_layer_stride % 16 != 0) return fail(PACE_KV_EINVAL, "pack: out_layer_stride not a multiple of 16");
-  std::vector<const char*> buf(num_layers);
-  pace_kv::buffer_layers(out, out_layer_stride, num_layers, buf.data());
-  Side src{reinterpret_cast<const char* const*>(src_layers), page_ids, pool_pages};
-  Side dst{buf.data(), nullptr, n_pages};
-  return pace_kv::launch_page_copy(src, dst, num_layers, n_pages, page_bytes, err_count,
-                                   static_cast<hipStream_t>(stream), pace_kv::StorePolicy::kPack);
+  return pace_kv::pack(src_layers, num_layers, pool_pages, {page_ids, nullptr}, n_pages, page_bytes, out,
+                       out_layer_stride, err_count, static_cast<hipStream_t>(stream));
+}
+
+int pace_kv_pack_inline(const void* const* src_layers, int num_layers, int64_t pool_pages,
+                        const int32_t* host_page_ids, int64_t n_pages, int64_t page_bytes, void* out,
+                        int64_t out_layer_stride, int32_t* err_count, void* stream) {
+  return pace_kv::pack(src_layers, num_layers, pool_pages, {nullptr, host_page_ids}, n_pages, page_bytes, out,
+                       out_layer_stride, err_count, static_cast<hipStream_t>(stream));
 }
 
 int pace_kv_unpack(const void* buf, int64_t buf_layer_stride, void* const* dst_layers,
                    int num_layers, int64_t pool_pages, const int32_t* page_ids, int64_t n_pages,
                    int64_t page_bytes, int32_t* err_count, void* stream) {
-  if (num_layers < 0) return fail(PACE_KV_EINVAL, "num_layers must be >= 0");
-  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
-  if (page_ids == nullptr || buf == nullptr) return fail(PACE_KV_EINVAL, "unpack: NULL page_ids or buf");
-  if (n_pages > 0 && page_bytes > 0 &&
-      (n_pages > INT64_MAX / page_bytes || buf_layer_stride < n_pages * page_bytes))
-    return fail(PACE_KV_ERANGE, "unpack: buf_layer_stride %lld < n_pages*page_bytes",
-                (long long)buf_layer_stride);
-  if (buf_layer_stride % 16 != 0) return fail(PACE_KV_EINVAL, "unpack: buf_layer_stride not a multiple of 16");
-  std::vector<const char*> src_tab(num_layers);
-  pace_kv::buffer_layers(buf, buf_layer_stride, num_layers, src_tab.data());
-  Side src{src_tab.data(), nullptr, n_pages};
-  Side dst{reinterpret_cast<const char* const*>(dst_layers), page_ids, pool_pages};
-  return pace_kv::launch_page_copy(src, dst, num_layers, n_pages, page_bytes, err_count,
-                                   static_cast<hipStream_t>(stream));
+  return pace_kv::unpack(buf, buf_layer_stride, dst_layers, num_layers, pool_pages, {page_ids, nullptr}, n_pages,
+                         page_bytes, err_count, static_cast<hipStream_t>(stream));
+}
+
+int pace_kv_unpack_inline(const void* buf, int64_t buf_layer_stride, void* const* dst_layers, int num_layers,
+                          int64_t pool_pages, const int32_t* host_page_ids, int64_t n_pages, int64_t page_bytes,
+                          int32_t* err_count, void* stream) {
+  return pace_kv::unpack(buf, buf_layer_stride, dst_layers, num_layers, pool_pages, {nullptr, host_page_ids}, n_pages,
+                         page_bytes, err_count, static_cast<hipStream_t>(stream));
 }
 
 int pace_kv_swap_out(const void* const* dev_layers, int64_t dev_pool_pages, const int32_t* dev_ids,

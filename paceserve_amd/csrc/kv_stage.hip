@@ -65,6 +65,7 @@
 
 using pace_kv::fail;
 using pace_kv::hip_status;
+using pace_kv::IdList;
 
 // Device staging of pace_kv_pack_to_host_noalloc: one array per GPU, which
 // the runtime places when it loads this code object on that GPU and which
@@ -314,16 +315,16 @@ bool direct_host(const void* host, int64_t bytes) {
 
 // pack(chunk c) of the source pool into out slot `slot`, on `stream`.
 int pack_chunk(pace_kv_stager* s, const ChunkPlan& p, int c, const void* const* src_layers,
-               int64_t pool_pages, const int32_t* ids, int32_t* err, hipStream_t stream) {
+               int64_t pool_pages, const IdList& ids, int32_t* err, hipStream_t stream) {
   char* slot = s->out_ring + (c % s->num_slots) * s->slot_bytes;
-  return pace_kv_pack(src_layers + p.first(c), p.count(c), pool_pages, ids, p.n_pages,
+  return pace_kv::pack(src_layers + p.first(c), p.count(c), pool_pages, ids, p.n_pages,
                       p.page_bytes, slot, p.layer_bytes, err, stream);
 }
 
 int unpack_chunk(pace_kv_stager* s, const ChunkPlan& p, int c, void* const* dst_layers,
-                 int64_t pool_pages, const int32_t* ids, int32_t* err, hipStream_t stream) {
+                 int64_t pool_pages, const IdList& ids, int32_t* err, hipStream_t stream) {
   const char* slot = s->in_ring + (c % s->num_slots) * s->slot_bytes;
-  return pace_kv_unpack(slot, p.layer_bytes, dst_layers + p.first(c), p.count(c), pool_pages, ids,
+  return pace_kv::unpack(slot, p.layer_bytes, dst_layers + p.first(c), p.count(c), pool_pages, ids,
                         p.n_pages, p.page_bytes, err, stream);
 }
 
@@ -364,6 +365,118 @@ struct SideJoin {
     if (hipEventRecord(event, side) == hipSuccess) (void)hipStreamWaitEvent(stream, event, 0);
   }
 };
+
+int pack_to_host(pace_kv_stager* s, const void* const* src_layers, int num_layers, int64_t pool_pages,
+                 const IdList& page_ids, int64_t n_pages, int64_t page_bytes, int layers_per_chunk, void* host_out,
+                 int32_t* err_count, hipStream_t stream) {
+  PACE_KV_TRY(check_stager(s));
+  ChunkPlan p;
+  PACE_KV_TRY(make_plan(s, num_layers, n_pages, page_bytes, layers_per_chunk, &p));
+  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
+  if (host_out == nullptr) return fail(PACE_KV_EINVAL, "pack_to_host: host_out is NULL");
+  const int chunks = p.num_chunks();
+  if (chunks == 1) {
+    // One chunk leaves nothing to overlap, so everything runs on `stream`,
+    // without the waits between streams (measured on MI355X: 30-36 us less per
+    // call for 2-8 MiB requests, about 1% less at 128 MiB).
+    const int64_t bytes = p.num_layers * p.layer_bytes;
+    if (direct_host(host_out, bytes)) {
+      const pace_kv::Side src{reinterpret_cast<const char* const*>(src_layers), page_ids.dev, pool_pages, page_ids.host};
+      return pace_kv::launch_host_leg(src, static_cast<char*>(host_out), true, num_layers, n_pages, page_bytes,
+                                      err_count, stream);
+    }
+    PACE_HIP(hipStreamWaitEvent(stream, s->out_free[0], 0), "wait out slot");
+    PACE_KV_TRY(pack_chunk(s, p, 0, src_layers, pool_pages, page_ids, err_count, stream));
+    // out_free follows the pack also when the copy fails to enqueue.
+    const hipError_t d2h =
+        hipMemcpyAsync(host_out, s->out_ring, static_cast<size_t>(bytes), hipMemcpyDeviceToHost, stream);
+    PACE_HIP(hipEventRecord(s->out_free[0], stream), "record out_free");
+    PACE_HIP(d2h, "D2H copy");
+    return PACE_KV_OK;
+  }
+  SideJoin join{s->d2h, stream, s->d2h_done};
+  // Step i enqueues pack(i + 1), then the copy of chunk i: the copy's
+  // completion record, which holds back whatever follows it when the D2H
+  // stream shares the caller's hardware queue, then only delays pack(i + 2).
+  // pack(i + 1) refills the slot of chunk i + 1 - num_slots, whose copy was
+  // enqueued in an earlier step (num_slots >= 2).
+  for (int i = -1; i < chunks; ++i) {
+    if (i + 1 < chunks) {
+      const int slot = (i + 1) % s->num_slots;
+      PACE_HIP(hipStreamWaitEvent(stream, s->out_free[slot], 0), "wait out slot");
+      PACE_KV_TRY(pack_chunk(s, p, i + 1, src_layers, pool_pages, page_ids, err_count, stream));
+      PACE_HIP(hipEventRecord(s->packed[slot], stream), "record packed");
+    }
+    if (i >= 0) {
+      const int slot = i % s->num_slots;
+      PACE_HIP(hipStreamWaitEvent(s->d2h, s->packed[slot], 0), "wait packed");
+      PACE_HIP(hipMemcpyAsync(static_cast<char*>(host_out) + p.first(i) * p.layer_bytes,
+                              s->out_ring + slot * s->slot_bytes, p.count(i) * p.layer_bytes,
+                              hipMemcpyDeviceToHost, s->d2h),
+               "D2H copy");
+      PACE_HIP(hipEventRecord(s->out_free[slot], s->d2h), "record out_free");
+    }
+  }
+  PACE_HIP(hipEventRecord(s->d2h_done, s->d2h), "record d2h_done");
+  PACE_HIP(hipStreamWaitEvent(stream, s->d2h_done, 0), "join D2H");
+  join.ok = true;
+  return PACE_KV_OK;
+}
+
+int unpack_from_host(pace_kv_stager* s, const void* host_in, void* const* dst_layers, int num_layers,
+                     int64_t pool_pages, const IdList& page_ids, int64_t n_pages, int64_t page_bytes,
+                     int layers_per_chunk, int32_t* err_count, hipStream_t stream) {
+  PACE_KV_TRY(check_stager(s));
+  ChunkPlan p;
+  PACE_KV_TRY(make_plan(s, num_layers, n_pages, page_bytes, layers_per_chunk, &p));
+  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
+  if (host_in == nullptr) return fail(PACE_KV_EINVAL, "unpack_from_host: host_in is NULL");
+  const int chunks = p.num_chunks();
+  if (chunks == 1) {
+    // One chunk: everything runs on `stream` (as in the pack).
+    const int64_t bytes = p.num_layers * p.layer_bytes;
+    if (direct_host(host_in, bytes)) {
+      const pace_kv::Side dst{reinterpret_cast<const char* const*>(dst_layers), page_ids.dev, pool_pages, page_ids.host};
+      return pace_kv::launch_host_leg(dst, const_cast<char*>(static_cast<const char*>(host_in)), false, num_layers,
+                                      n_pages, page_bytes, err_count, stream);
+    }
+    PACE_HIP(hipStreamWaitEvent(stream, s->in_free[0], 0), "wait in slot");
+    PACE_HIP(hipMemcpyAsync(s->in_ring, host_in, bytes, hipMemcpyHostToDevice, stream), "H2D copy");
+    // in_free follows the copy also when the unpack fails to launch.
+    const int rc = unpack_chunk(s, p, 0, dst_layers, pool_pages, page_ids, err_count, stream);
+    PACE_HIP(hipEventRecord(s->in_free[0], stream), "record in_free");
+    return rc;
+  }
+  // The caller's earlier work (e.g. writes of host_in by a kernel) comes first.
+  PACE_HIP(hipEventRecord(s->start, stream), "record start");
+  PACE_HIP(hipStreamWaitEvent(s->h2d, s->start, 0), "wait start");
+  // On success the last unpack, on `stream`, follows every copy.
+  SideJoin join{s->h2d, stream, s->start};
+  // Step i enqueues the copy of chunk i + 1, then unpack(i), whose wait for
+  // chunk i's copy then holds back (on a shared hardware queue) only the copy
+  // of chunk i + 2.  That copy refills the slot of chunk i + 2 - num_slots,
+  // whose unpack was enqueued in an earlier step (num_slots >= 2).
+  for (int i = -1; i < chunks; ++i) {
+    if (i + 1 < chunks) {
+      const int c = i + 1;
+      const int slot = c % s->num_slots;
+      PACE_HIP(hipStreamWaitEvent(s->h2d, s->in_free[slot], 0), "wait in slot");
+      PACE_HIP(hipMemcpyAsync(s->in_ring + slot * s->slot_bytes,
+                              static_cast<const char*>(host_in) + p.first(c) * p.layer_bytes,
+                              p.count(c) * p.layer_bytes, hipMemcpyHostToDevice, s->h2d),
+               "H2D copy");
+      PACE_HIP(hipEventRecord(s->in_ready[slot], s->h2d), "record in_ready");
+    }
+    if (i >= 0) {
+      const int slot = i % s->num_slots;
+      PACE_HIP(hipStreamWaitEvent(stream, s->in_ready[slot], 0), "wait in_ready");
+      PACE_KV_TRY(unpack_chunk(s, p, i, dst_layers, pool_pages, page_ids, err_count, stream));
+      PACE_HIP(hipEventRecord(s->in_free[slot], stream), "record in_free");
+    }
+  }
+  join.ok = true;
+  return PACE_KV_OK;
+}
 
 }  // namespace
 
@@ -419,117 +532,33 @@ int pace_kv_stager_destroy(pace_kv_stager* s) {
 int pace_kv_pack_to_host(pace_kv_stager* s, const void* const* src_layers, int num_layers,
                          int64_t pool_pages, const int32_t* page_ids, int64_t n_pages,
                          int64_t page_bytes, int layers_per_chunk, void* host_out,
-                         int32_t* err_count, void* stream_) {
-  PACE_KV_TRY(check_stager(s));
-  ChunkPlan p;
-  PACE_KV_TRY(make_plan(s, num_layers, n_pages, page_bytes, layers_per_chunk, &p));
-  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
-  if (host_out == nullptr) return fail(PACE_KV_EINVAL, "pack_to_host: host_out is NULL");
-  hipStream_t stream = static_cast<hipStream_t>(stream_);
-  const int chunks = p.num_chunks();
-  if (chunks == 1) {
-    // One chunk leaves nothing to overlap, so everything runs on `stream`,
-    // without the waits between streams (measured on MI355X: 30-36 us less per
-    // call for 2-8 MiB requests, about 1% less at 128 MiB).
-    const int64_t bytes = p.num_layers * p.layer_bytes;
-    if (direct_host(host_out, bytes)) {
-      const pace_kv::Side src{reinterpret_cast<const char* const*>(src_layers), page_ids, pool_pages};
-      return pace_kv::launch_host_leg(src, static_cast<char*>(host_out), true, num_layers, n_pages, page_bytes,
-                                      err_count, stream);
-    }
-    PACE_HIP(hipStreamWaitEvent(stream, s->out_free[0], 0), "wait out slot");
-    PACE_KV_TRY(pack_chunk(s, p, 0, src_layers, pool_pages, page_ids, err_count, stream));
-    // out_free follows the pack also when the copy fails to enqueue.
-    const hipError_t d2h =
-        hipMemcpyAsync(host_out, s->out_ring, static_cast<size_t>(bytes), hipMemcpyDeviceToHost, stream);
-    PACE_HIP(hipEventRecord(s->out_free[0], stream), "record out_free");
-    PACE_HIP(d2h, "D2H copy");
-    return PACE_KV_OK;
-  }
-  SideJoin join{s->d2h, stream, s->d2h_done};
-  // Step i enqueues pack(i + 1), then the copy of chunk i: the copy's
-  // completion record, which holds back whatever follows it when the D2H
-  // stream shares the caller's hardware queue, then only delays pack(i + 2).
-  // pack(i + 1) refills the slot of chunk i + 1 - num_slots, whose copy was
-  // enqueued in an earlier step (num_slots >= 2).
-  for (int i = -1; i < chunks; ++i) {
-    if (i + 1 < chunks) {
-      const int slot = (i + 1) % s->num_slots;
-      PACE_HIP(hipStreamWaitEvent(stream, s->out_free[slot], 0), "wait out slot");
-      PACE_KV_TRY(pack_chunk(s, p, i + 1, src_layers, pool_pages, page_ids, err_count, stream));
-      PACE_HIP(hipEventRecord(s->packed[slot], stream), "record packed");
-    }
-    if (i >= 0) {
-      const int slot = i % s->num_slots;
-      PACE_HIP(hipStreamWaitEvent(s->d2h, s->packed[slot], 0), "wait packed");
-      PACE_HIP(hipMemcpyAsync(static_cast<char*>(host_out) + p.first(i) * p.layer_bytes,
-                              s->out_ring + slot * s->slot_bytes, p.count(i) * p.layer_bytes,
-                              hipMemcpyDeviceToHost, s->d2h),
-               "D2H copy");
-      PACE_HIP(hipEventRecord(s->out_free[slot], s->d2h), "record out_free");
-    }
-  }
-  PACE_HIP(hipEventRecord(s->d2h_done, s->d2h), "record d2h_done");
-  PACE_HIP(hipStreamWaitEvent(stream, s->d2h_done, 0), "join D2H");
-  join.ok = true;
-  return PACE_KV_OK;
+                         int32_t* err_count, void* stream) {
+  return pack_to_host(s, src_layers, num_layers, pool_pages, {page_ids, nullptr}, n_pages, page_bytes,
+                      layers_per_chunk, host_out, err_count, static_cast<hipStream_t>(stream));
+}
+
+int pace_kv_pack_to_host_inline(pace_kv_stager* s, const void* const* src_layers, int num_layers,
+                                int64_t pool_pages, const int32_t* host_page_ids, int64_t n_pages,
+                                int64_t page_bytes, int layers_per_chunk, void* host_out,
+                                int32_t* err_count, void* stream) {
+  return pack_to_host(s, src_layers, num_layers, pool_pages, {nullptr, host_page_ids}, n_pages, page_bytes,
+                      layers_per_chunk, host_out, err_count, static_cast<hipStream_t>(stream));
 }
 
 int pace_kv_unpack_from_host(pace_kv_stager* s, const void* host_in, void* const* dst_layers,
                              int num_layers, int64_t pool_pages, const int32_t* page_ids,
                              int64_t n_pages, int64_t page_bytes, int layers_per_chunk,
-                             int32_t* err_count, void* stream_) {
-  PACE_KV_TRY(check_stager(s));
-  ChunkPlan p;
-  PACE_KV_TRY(make_plan(s, num_layers, n_pages, page_bytes, layers_per_chunk, &p));
-  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
-  if (host_in == nullptr) return fail(PACE_KV_EINVAL, "unpack_from_host: host_in is NULL");
-  hipStream_t stream = static_cast<hipStream_t>(stream_);
-  const int chunks = p.num_chunks();
-  if (chunks == 1) {
-    // One chunk: everything runs on `stream` (as in the pack).
-    const int64_t bytes = p.num_layers * p.layer_bytes;
-    if (direct_host(host_in, bytes)) {
-      const pace_kv::Side dst{reinterpret_cast<const char* const*>(dst_layers), page_ids, pool_pages};
-      return pace_kv::launch_host_leg(dst, const_cast<char*>(static_cast<const char*>(host_in)), false, num_layers,
-                                      n_pages, page_bytes, err_count, stream);
-    }
-    PACE_HIP(hipStreamWaitEvent(stream, s->in_free[0], 0), "wait in slot");
-    PACE_HIP(hipMemcpyAsync(s->in_ring, host_in, bytes, hipMemcpyHostToDevice, stream), "H2D copy");
-    // in_free follows the copy also when the unpack fails to launch.
-    const int rc = unpack_chunk(s, p, 0, dst_layers, pool_pages, page_ids, err_count, stream);
-    PACE_HIP(hipEventRecord(s->in_free[0], stream), "record in_free");
-    return rc;
-  }
-  // The caller's earlier work (e.g. writes of host_in by a kernel) comes first.
-  PACE_HIP(hipEventRecord(s->start, stream), "record start");
-  PACE_HIP(hipStreamWaitEvent(s->h2d, s->start, 0), "wait start");
-  // On success the last unpack, on `stream`, follows every copy.
-  SideJoin join{s->h2d, stream, s->start};
-  // Step i enqueues the copy of chunk i + 1, then unpack(i), whose wait for
-  // chunk i's copy then holds back (on a shared hardware queue) only the copy
-  // of chunk i + 2.  That copy refills the slot of chunk i + 2 - num_slots,
-  // whose unpack was enqueued in an earlier step (num_slots >= 2).
-  for (int i = -1; i < chunks; ++i) {
-    if (i + 1 < chunks) {
-      const int c = i + 1;
-      const int slot = c % s->num_slots;
-      PACE_HIP(hipStreamWaitEvent(s->h2d, s->in_free[slot], 0), "wait in slot");
-      PACE_HIP(hipMemcpyAsync(s->in_ring + slot * s->slot_bytes,
-                              static_cast<const char*>(host_in) + p.first(c) * p.layer_bytes,
-                              p.count(c) * p.layer_bytes, hipMemcpyHostToDevice, s->h2d),
-               "H2D copy");
-      PACE_HIP(hipEventRecord(s->in_ready[slot], s->h2d), "record in_ready");
-    }
-    if (i >= 0) {
-      const int slot = i % s->num_slots;
-      PACE_HIP(hipStreamWaitEvent(stream, s->in_ready[slot], 0), "wait in_ready");
-      PACE_KV_TRY(unpack_chunk(s, p, i, dst_layers, pool_pages, page_ids, err_count, stream));
-      PACE_HIP(hipEventRecord(s->in_free[slot], stream), "record in_free");
-    }
-  }
-  join.ok = true;
-  return PACE_KV_OK;
+                             int32_t* err_count, void* stream) {
+  return unpack_from_host(s, host_in, dst_layers, num_layers, pool_pages, {page_ids, nullptr}, n_pages, page_bytes,
+                          layers_per_chunk, err_count, static_cast<hipStream_t>(stream));
+}
+
+int pace_kv_unpack_from_host_inline(pace_kv_stager* s, const void* host_in, void* const* dst_layers,
+                                    int num_layers, int64_t pool_pages, const int32_t* host_page_ids,
+                                    int64_t n_pages, int64_t page_bytes, int layers_per_chunk,
+                                    int32_t* err_count, void* stream) {
+  return unpack_from_host(s, host_in, dst_layers, num_layers, pool_pages, {nullptr, host_page_ids}, n_pages,
+                          page_bytes, layers_per_chunk, err_count, static_cast<hipStream_t>(stream));
 }
 
 int pace_kv_roundtrip(pace_kv_stager* s, const void* const* src_layers, int64_t src_pool_pages,
@@ -575,7 +604,7 @@ int pace_kv_roundtrip(pace_kv_stager* s, const void* const* src_layers, int64_t 
       return rc;
     }
     PACE_HIP(hipStreamWaitEvent(caller, s->out_free[0], 0), "wait out slot");
-    PACE_KV_TRY(pack_chunk(s, p, 0, src_layers, src_pool_pages, src_ids, err_count, caller));
+    PACE_KV_TRY(pack_chunk(s, p, 0, src_layers, src_pool_pages, {src_ids, nullptr}, err_count, caller));
     // out_free follows the pack also when the copy fails to enqueue.
     const hipError_t d2h =
         hipMemcpyAsync(host, s->out_ring, static_cast<size_t>(bytes), hipMemcpyDeviceToHost, caller);
@@ -585,7 +614,7 @@ int pace_kv_roundtrip(pace_kv_stager* s, const void* const* src_layers, int64_t 
     PACE_HIP(hipMemcpyAsync(s->in_ring, host, bytes, hipMemcpyHostToDevice, caller), "H2D copy");
     PACE_HIP(hipEventRecord(s->h2d_done, caller), "record h2d_done");
     // The records follow the H2D copy also when the unpack fails to launch.
-    const int rc = unpack_chunk(s, p, 0, dst_layers, dst_pool_pages, dst_ids, err_count, caller);
+    const int rc = unpack_chunk(s, p, 0, dst_layers, dst_pool_pages, {dst_ids, nullptr}, err_count, caller);
     PACE_HIP(hipEventRecord(s->in_free[0], caller), "record in_free");
     PACE_HIP(hipEventRecord(s->work_done, caller), "record work_done");
     return rc;
@@ -610,7 +639,7 @@ int pace_kv_roundtrip(pace_kv_stager* s, const void* const* src_layers, int64_t 
   auto pack = [&](int c) -> int {
     const int slot = c % S;
     PACE_HIP(hipStreamWaitEvent(stream, s->out_free[slot], 0), "wait out slot");
-    PACE_KV_TRY(pack_chunk(s, p, c, src_layers, src_pool_pages, src_ids, err_count, stream));
+    PACE_KV_TRY(pack_chunk(s, p, c, src_layers, src_pool_pages, {src_ids, nullptr}, err_count, stream));
     PACE_HIP(hipEventRecord(s->packed[slot], stream), "record packed");
     return PACE_KV_OK;
   };
@@ -651,7 +680,7 @@ int pace_kv_roundtrip(pace_kv_stager* s, const void* const* src_layers, int64_t 
   auto unpack = [&](int c) -> int {
     const int slot = c % S;
     PACE_HIP(hipStreamWaitEvent(stream, s->in_ready[slot], 0), "wait in_ready");
-    PACE_KV_TRY(unpack_chunk(s, p, c, dst_layers, dst_pool_pages, dst_ids, err_count, stream));
+    PACE_KV_TRY(unpack_chunk(s, p, c, dst_layers, dst_pool_pages, {dst_ids, nullptr}, err_count, stream));
     PACE_HIP(hipEventRecord(s->in_free[slot], stream), "record in_free");
     return PACE_KV_OK;
   };

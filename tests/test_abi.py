@@ -129,3 +129,18 @@ def test_noalloc_pack_to_host_rejects_a_short_output(lib):
     assert b"needs 24576 bytes, host_out holds 24575" in lib.pace_kv_last_error()
     text = HEADER.read_text()
     assert "#define PACE_KV_NOALLOC_SCRATCH_BYTES (64 << 20)" in text
+
+
+def test_ids_in_host_memory_are_limited(lib):
+    """The calls whose page ids travel in the kernel arguments take at most
+    PACE_KV_INLINE_IDS of them; refused before any device call."""
+    n, text = _native.INLINE_IDS + 1, HEADER.read_text()
+    assert f"#define PACE_KV_INLINE_IDS {_native.INLINE_IDS}" in text
+    ids = (ctypes.c_int32 * n)()
+    at = ctypes.addressof(ids)
+    assert lib.pace_kv_pack_inline(_layers(1), 1, n, at, n, 64, 0x1000, n * 64, None, None) == _native.PACE_KV_ERANGE
+    assert b"512 pages" in lib.pace_kv_last_error()
+    assert lib.pace_kv_unpack_inline(0x1000, n * 64, _layers(1), 1, n, at, n, 64, None, None) == \
+        _native.PACE_KV_ERANGE
+    assert lib.pace_kv_pack_inline(_layers(1), 1, n, None, 3, 64, 0x1000, n * 64, None, None) == \
+        _native.PACE_KV_EINVAL

@@ -81,3 +81,30 @@ def test_promotion(gpu, page_bytes, n, mode):
     want = before.clone()
     want[:, plan.dst_ids] = src.cpu()[:, s_ids]
     assert torch.equal(dst.cpu(), want)
+
+
+@pytest.mark.parametrize("n", [1, 33, 512, 513])     # up to 512 ids travel in the kernel arguments
+@pytest.mark.parametrize("page_bytes", [32, 480, 1056, 2048, 3072])
+def test_host_ids(gpu, page_bytes, n):
+    """Lists and CPU tensors of page ids, through the device and the host
+    legs, in one chunk and in several."""
+    L, N = 5, n + 5
+    gen = torch.Generator().manual_seed(page_bytes * 2048 + n)
+    (src, src_l), (dst, dst_l) = pool(L, N, page_bytes, gen, gpu), pool(L, N, page_bytes, gen, gpu)
+    s_ids, d_ids = ids_of(n, N, gen, False), ids_of(n, N, gen, False)
+    picked = src.cpu()[:, s_ids]
+    want = dst.cpu()
+    want[:, d_ids] = picked
+    buf = ops.pack(src_l, s_ids)
+    assert torch.equal(buf.view(torch.uint8).cpu(), picked)
+    ops.unpack(buf, dst_l, torch.tensor(d_ids))
+    assert torch.equal(dst.cpu(), want)
+    for k in (L, 2):
+        host = torch.empty(buf.shape, dtype=buf.dtype, pin_memory=True)
+        dst[:, d_ids] = 0
+        with ops.Stager(-(-k * n * page_bytes // 256) * 256, 2) as st:
+            st.pack_to_host(src_l, s_ids, host, k)
+            torch.cuda.synchronize()
+            assert torch.equal(host.view(torch.uint8), picked)
+            st.unpack_from_host(host, dst_l, d_ids, k)
+            assert torch.equal(dst.cpu(), want)

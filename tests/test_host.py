@@ -302,3 +302,23 @@ def test_host_destination_ids_must_be_distinct():
     with pytest.raises(ValueError, match="destination page 7 appears"):
         ops.device_ids(torch.tensor([7, 7]), torch.device("cpu"), distinct=True)
     assert ops.device_ids([], torch.device("cpu"), distinct=True).numel() == 0
+
+
+def test_inline_ids_take_what_uploads_take():
+    """Host ids that travel in the kernel arguments: the same values, or None
+    where the upload path decides (too many, none, not an int32 list)."""
+    from array import array
+
+    import torch
+
+    from paceserve_amd.kv_transfer import ops
+    for ids in ([3, 1, 2], (3, 1, 2), array("i", [3, 1, 2]), torch.tensor([3, 1, 2]), torch.tensor([[3], [1], [2]]),
+                torch.tensor([3.7, 1.2, 2.0]), list(np.array([3, 1, 2]))):
+        assert ops._inline_ids(ids, distinct=True).tolist() == [3, 1, 2]
+    assert ops._inline_ids([-1, 2 ** 31 - 1]).tolist() == [-1, 2 ** 31 - 1]
+    assert len(ops._inline_ids(list(range(512)))) == 512
+    for ids in ([], torch.tensor([]), list(range(513)), torch.arange(513), [2 ** 31], [1.5], iter([1, 2])):
+        assert ops._inline_ids(ids) is None
+    with pytest.raises(ValueError, match="destination page 3 appears more than once"):
+        ops._inline_ids([5, 3, 1, 3], distinct=True)
+    assert ops._inline_ids([5, 3, 1, 3]).tolist() == [5, 3, 1, 3]
