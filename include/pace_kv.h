@@ -382,6 +382,16 @@ int pace_kv_append_indptr(const void* keys, const void* values,
                           int64_t row_bytes, int32_t* err_count, void* stream);
 
 /*
+ * Sequence length of every request (device), the appended tokens included:
+ *   seq_lens[b] = max(kv_indptr[b + 1] - kv_indptr[b] - 1, 0) * page_size + kv_last_page_len[b]
+ * in wrapping 32-bit arithmetic.  Replaces flashinfer.get_seq_lens as called in
+ * paceserve/model_executor/attention/flashinfer_attention_wrapper.py:241.
+ */
+int pace_kv_seq_lens(const int32_t* kv_indptr, const int32_t* kv_last_page_len,
+                     int batch_size, int page_size, int32_t* seq_lens,
+                     void* stream);
+
+/*
  * Request index and sequence position of every appended token (device):
  *   for append_indptr[b] <= i < append_indptr[b+1]:
  *     batch_indices[i] = b,

@@ -266,6 +266,21 @@ __global__ __launch_bounds__(kThreads) void append_kernel(const AppendParams p) 
   store_row_vec(reinterpret_cast<u32x4*>(row + half) + vec, v);
 }
 
+// Sequence length of each request, in 32-bit arithmetic that wraps as torch's
+// does.  Bound by its launch: one instead of the five elementwise ones that
+// tensor arithmetic takes (MI355X: FlashInfer's form of a prefill of 2 x 4095
+// tokens, 4 layers, 194.6 -> 184.4 us).
+__global__ __launch_bounds__(256) void seq_lens_kernel(const int32_t* __restrict__ kv_indptr,
+                                                       const int32_t* __restrict__ last_page_len, uint32_t batch_size,
+                                                       uint32_t page_size, int32_t* __restrict__ out) {
+  const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= batch_size) return;
+  const int32_t before_last = static_cast<int32_t>(static_cast<uint32_t>(kv_indptr[b + 1]) -
+                                                   static_cast<uint32_t>(kv_indptr[b]) - 1u);
+  const uint32_t full = before_last > 0 ? static_cast<uint32_t>(before_last) : 0u;
+  out[b] = static_cast<int32_t>(full * page_size + static_cast<uint32_t>(last_page_len[b]));
+}
+
 // One thread per appended token: finds its request by binary search over
 // append_indptr and derives its position from the request's sequence length.
 __global__ __launch_bounds__(256) void positions_kernel(const int32_t* __restrict__ append_indptr,
@@ -409,6 +424,18 @@ int pace_kv_append_indptr(const void* keys, const void* values, int64_t token_st
   p.err = err_count;
   return pace_kv::launch_append(p, nnz, batch_size, num_pages, num_indices, page_size, token_stride_bytes,
                                 row_bytes, true, static_cast<hipStream_t>(stream));
+}
+
+int pace_kv_seq_lens(const int32_t* kv_indptr, const int32_t* kv_last_page_len, int batch_size, int page_size,
+                     int32_t* seq_lens, void* stream) {
+  if (batch_size < 0) return fail(PACE_KV_EINVAL, "seq_lens: negative size");
+  if (batch_size == 0) return PACE_KV_OK;
+  if (!kv_indptr || !kv_last_page_len || !seq_lens) return fail(PACE_KV_EINVAL, "seq_lens: NULL argument");
+  uint32_t bs = static_cast<uint32_t>(batch_size), ps = static_cast<uint32_t>(page_size);
+  void* args[] = {&kv_indptr, &kv_last_page_len, &bs, &ps, &seq_lens};
+  return hip_status(hipLaunchKernel(reinterpret_cast<const void*>(&pace_kv::seq_lens_kernel), dim3((bs + 255) / 256),
+                                    dim3(256), args, 0, static_cast<hipStream_t>(stream)),
+                    "seq_lens launch");
 }
 
 int pace_kv_batch_indices_positions(const int32_t* append_indptr, const int32_t* seq_lens,

@@ -26,8 +26,36 @@ def _i32(t: torch.Tensor, name: str, device: torch.device) -> torch.Tensor:
     return t.to(torch.int32).contiguous()
 
 
+def _plain_i32(t, dev) -> bool:
+    """Whether t is an ordinary contiguous 1-D int32 tensor on dev: no subclass
+    and not wrapped by vmap or another function transform."""
+    return (type(t) is torch.Tensor and t.dtype is torch.int32 and t.dim() == 1 and t.device == dev
+            and t.is_contiguous() and not torch._C._functorch.is_functorch_wrapped_tensor(t))
+
+
+def _one_launch(kv_indptr, kv_last_page_len, page_size) -> bool:
+    """Whether get_seq_lens is one launch of the library: plain int32 tensors
+    of matching lengths on the current device and no tracing.  Everything else
+    (CPU, other integer types, broadcasting, strides, tracers) is tensor
+    arithmetic."""
+    return (type(page_size) is int and 0 <= page_size < 2 ** 31 and type(kv_indptr) is torch.Tensor
+            and kv_indptr.is_cuda and _plain_i32(kv_indptr, kv_indptr.device)
+            and _plain_i32(kv_last_page_len, kv_indptr.device)
+            and kv_indptr.numel() == kv_last_page_len.numel() + 1 > 1
+            and kv_indptr.device.index == torch.cuda.current_device()
+            and torch._C._len_torch_dispatch_stack() == 0 and not torch.jit.is_tracing()
+            and not torch.compiler.is_compiling())
+
+
 def get_seq_lens(kv_indptr: torch.Tensor, kv_last_page_len: torch.Tensor, page_size: int) -> torch.Tensor:
     """max(pages - 1, 0) * page_size + last_page_len per request (int32)."""
+    if _one_launch(kv_indptr, kv_last_page_len, page_size):
+        dev = kv_indptr.device
+        out = torch.empty(kv_last_page_len.numel(), dtype=torch.int32, device=dev)
+        _native.check(_native.load().pace_kv_seq_lens(
+            kv_indptr.data_ptr(), kv_last_page_len.data_ptr(), out.numel(), page_size, out.data_ptr(),
+            _stream_handle(dev)))
+        return out
     pages = kv_indptr[1:] - kv_indptr[:-1]
     return (torch.clamp(pages - 1, min=0) * page_size + kv_last_page_len).to(torch.int32)
 
