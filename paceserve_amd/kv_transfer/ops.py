@@ -158,8 +158,8 @@ def _inline_ids(ids: IdsLike, distinct: bool = False) -> Optional[array]:
     _native.INLINE_IDS, in a CPU tensor, list, tuple or array), as an int32
     array; None for any others, which device_ids takes or refuses.  An upload
     costs a pinned allocation and a copy ahead of each launch: pack and unpack
-    of 32 pages of 64 KiB, 32 layers, take 40 us without, 52 with, and get_kv_cache and insert_kv_cache of
-    100 tokens 569 and 608."""
+    of 32 pages of 64 KiB, 32 layers, take 40 us without, 52 with, and
+    get_kv_cache and insert_kv_cache of 100 tokens 569 and 608."""
     if isinstance(ids, torch.Tensor):
         if ids.device.type != "cpu" or not 0 < ids.numel() <= _native.INLINE_IDS:
             return None
