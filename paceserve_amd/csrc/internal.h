@@ -93,11 +93,14 @@ int launch_page_copy(const Side& src, const Side& dst, int num_layers,
 int buffered_copy(const Side& src, const Side& dst, char* buffer, int64_t buffer_layer_stride, int buffer_layers,
                   int num_layers, int64_t n_pages, int64_t page_bytes, int32_t* err_count, hipStream_t stream);
 
-// Copies pages between a pool and `host`, pinned memory that the device
-// addresses at this pointer, laid out [num_layers][n_pages][page_bytes]: out of
-// the pool (to_host) or into it, in one launch per PACE_KV_MAX_LAYERS_PER_LAUNCH
-// layers.  The arguments are checked as launch_page_copy checks them; a page
-// whose id is outside the pool is left as it was, on either side, and counted.
+// launch_page_copy between device pages (`pool`, with ids) and pinned memory
+// that the device addresses (`host`: a pool with device ids, or, without ids,
+// [num_layers][n_pages][page_bytes] in one piece), out to the host (to_host) or in
+// from it, with few waves.
+int launch_host_leg(const Side& pool, const Side& host, bool to_host, int num_layers, int64_t n_pages,
+                    int64_t page_bytes, int32_t* err_count, hipStream_t stream);
+
+// The same with the host side laid out [num_layers][n_pages][page_bytes].
 int launch_host_leg(const Side& pool, char* host, bool to_host, int num_layers, int64_t n_pages, int64_t page_bytes,
                     int32_t* err_count, hipStream_t stream);
 

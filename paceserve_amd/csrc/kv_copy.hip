@@ -286,14 +286,24 @@ const void* inline_kernel_of(Kind kind, InlineSides sides) {
 constexpr int kHostThreads = 256;
 constexpr int kOutGroups = 4, kOutUnroll = 16;
 constexpr int kInGroups = 16, kInUnroll = 8;
+// Between two paged pools (swaps) both sides' ids take registers: 8 vectors
+// either way, out from 32 workgroups (12 to 16 are 1-4% slower).  Measured
+// against the page copy's one wave per row, 63 pages of 64 KiB, 32 layers: out
+// 2379 -> 2328 us, in 2412 -> 2326; 7 pages out 270 -> 264, in 290 -> 265; 500
+// pages of 8 KiB out 2362 -> 2307, in 2384 -> 2306; 777 of 1536 B out 689 -> 680,
+// in 696 -> 679; 1000 of 512 B 296 -> 298 and 299 -> 302, where the page copy's
+// end-to-end waves would take 306 and 312.
+constexpr int kPagedOutGroups = 32;
 
 struct HostLegParams {
   char* layers[kMaxLayers];
-  u32x4* host;             // [layers][n_pages][page_vecs]
-  const int32_t* ids;      // device array; unused by the inline kernel
+  char* host[kMaxLayers];  // the host side: pages in order, or chosen by host_ids (PAGED)
+  const int32_t* ids;      // device arrays; unused by the inline kernel
+  const int32_t* host_ids;
   int32_t* err;
   int64_t page_bytes;
-  uint32_t pool_pages;
+  uint32_t pool_pages;     // at least 1, on both sides
+  uint32_t host_pages;
   uint32_t page_vecs;
   uint32_t n_pages;
   uint32_t total_vecs;
@@ -309,73 +319,75 @@ struct HostLegParamsInline {
 // What a lane needs to know of the UNROLL vectors of one round.
 template <int UNROLL>
 struct HostRound {
-  uint32_t k[UNROLL], vec[UNROLL], id[UNROLL];
+  uint32_t vec[UNROLL], id[UNROLL], host_id[UNROLL];
   char* base[UNROLL];
+  char* host[UNROLL];
 };
 
-template <int UNROLL>
+template <int UNROLL, bool PAGED>
 __device__ __forceinline__ void next_round(const HostLegParams& p, const int32_t* ids, uint32_t i, uint32_t stride,
                                            HostRound<UNROLL>* r) {
 #pragma unroll
   for (int u = 0; u < UNROLL; ++u) {
-    r->k[u] = min(i + u * stride, p.total_vecs - 1);
-    const uint32_t at = over(p.by_page, r->k[u]);
-    r->vec[u] = r->k[u] - at * p.page_vecs;
+    const uint32_t k = min(i + u * stride, p.total_vecs - 1);
+    const uint32_t at = over(p.by_page, k);
+    r->vec[u] = k - at * p.page_vecs;
     const uint32_t layer = over(p.by_count, at);
+    const uint32_t j = at - layer * p.n_pages;
     r->base[u] = p.layers[layer];
-    r->id[u] = static_cast<uint32_t>(ids[at - layer * p.n_pages]);
+    r->id[u] = static_cast<uint32_t>(ids[j]);
+    r->host[u] = PAGED ? p.host[layer] : p.host[0];
+    r->host_id[u] = PAGED ? static_cast<uint32_t>(p.host_ids[j]) : at;
   }
 }
 
 // The loads of a round are free of branches, so that all of a lane's are in
 // flight together: a vector past the end repeats the last one's and a page id
-// out of range reads the host side, and neither is stored.  The next round's
-// ids are loaded behind this round's vectors.
-template <bool TO_HOST, int UNROLL>
+// out of range reads page 0, and neither is stored.  The next round's ids are
+// loaded behind this round's vectors.
+template <bool TO_HOST, int UNROLL, bool PAGED>
 __device__ __forceinline__ void host_leg(const HostLegParams& p, const int32_t* ids) {
   const uint32_t stride = gridDim.x * kHostThreads;
   uint32_t i = blockIdx.x * kHostThreads + threadIdx.x;
   HostRound<UNROLL> r;
-  next_round(p, ids, i, stride, &r);
+  next_round<UNROLL, PAGED>(p, ids, i, stride, &r);
   for (; i < p.total_vecs; i += UNROLL * stride) {
-    u32x4* pool[UNROLL];
+    u32x4* to[UNROLL];
     u32x4 v[UNROLL];
+    bool ok[UNROLL], first[UNROLL];
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
-      pool[u] = reinterpret_cast<u32x4*>(r.base[u] + static_cast<int64_t>(r.id[u]) * p.page_bytes) + r.vec[u];
-      const u32x4* from = p.host + r.k[u];
-      if (TO_HOST) {
-        // The compiler must not see what the choice is between: it would put
-        // the address, and the loads it needs, behind a branch per vector.
-        uint64_t in_pool = reinterpret_cast<uint64_t>(pool[u]), on_host = reinterpret_cast<uint64_t>(from);
-        asm("" : "+v"(in_pool), "+v"(on_host));
-        from = reinterpret_cast<const u32x4*>(r.id[u] < p.pool_pages ? in_pool : on_host);
-      }
-      v[u] = __builtin_nontemporal_load(reinterpret_cast<const __attribute__((address_space(1))) u32x4*>(
-          reinterpret_cast<uint64_t>(from)));
+      const bool id_ok = r.id[u] < p.pool_pages, host_ok = !PAGED || r.host_id[u] < p.host_pages;
+      u32x4* const pool =
+          reinterpret_cast<u32x4*>(r.base[u] + static_cast<int64_t>(id_ok ? r.id[u] : 0) * p.page_bytes) + r.vec[u];
+      u32x4* const host =
+          reinterpret_cast<u32x4*>(r.host[u] + static_cast<int64_t>(host_ok ? r.host_id[u] : 0) * p.page_bytes) +
+          r.vec[u];
+      v[u] = __builtin_nontemporal_load(TO_HOST ? pool : host);
+      to[u] = TO_HOST ? host : pool;
+      ok[u] = id_ok && host_ok;
+      first[u] = r.vec[u] == 0;
     }
     __builtin_amdgcn_sched_barrier(0);
-    HostRound<UNROLL> ahead;
-    next_round(p, ids, i + UNROLL * stride, stride, &ahead);
+    next_round<UNROLL, PAGED>(p, ids, i + UNROLL * stride, stride, &r);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
       if (i + u * stride >= p.total_vecs) continue;
-      if (r.id[u] < p.pool_pages) store_vec<false>(v[u], TO_HOST ? p.host + r.k[u] : pool[u]);
-      else if (r.vec[u] == 0 && p.err != nullptr) atomicAdd(p.err, 1);
+      if (ok[u]) store_vec<false>(v[u], to[u]);
+      else if (first[u] && p.err != nullptr) atomicAdd(p.err, 1);
     }
-    r = ahead;
   }
 }
 
-template <bool TO_HOST>
+template <bool TO_HOST, bool PAGED>
 __global__ __launch_bounds__(kHostThreads) void host_leg_kernel(const HostLegParams p) {
-  host_leg<TO_HOST, TO_HOST ? kOutUnroll : kInUnroll>(p, p.ids);
+  host_leg<TO_HOST, TO_HOST && !PAGED ? kOutUnroll : kInUnroll, PAGED>(p, p.ids);
 }
 
 template <bool TO_HOST>
 __global__ __launch_bounds__(kHostThreads) void host_leg_inline_kernel(const HostLegParamsInline p) {
-  host_leg<TO_HOST, TO_HOST ? kOutUnroll : kInUnroll>(p.base, p.ids);
+  host_leg<TO_HOST, TO_HOST ? kOutUnroll : kInUnroll, false>(p.base, p.ids);
 }
 
 const void* pick_kernel(Shape shape, Kind kind) {
@@ -559,21 +571,22 @@ bool disjoint(const char* const* a, int64_t a_bytes, const char* const* b, int64
 
 }  // namespace
 
-int launch_host_leg(const Side& pool, char* host, bool to_host, int num_layers, int64_t n_pages, int64_t page_bytes,
-                    int32_t* err_count, hipStream_t stream) {
-  if (num_layers < 0 || n_pages < 0 || pool.pool_pages < 0) return fail(PACE_KV_EINVAL, "host leg: negative size");
-  if (page_bytes <= 0 || page_bytes % kVecBytes != 0)
-    return fail(PACE_KV_EINVAL, "page_bytes must be a positive multiple of 16 (got %lld)", (long long)page_bytes);
-  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
-  if (host == nullptr || !aligned16(host)) return fail(PACE_KV_EINVAL, "host buffer is NULL or not 16-byte aligned");
-  PACE_KV_TRY(check_layers(pool.layers, num_layers, to_host ? "source" : "destination"));
-  if (pool.ids == nullptr && pool.host_ids == nullptr) return fail(PACE_KV_EINVAL, "host leg: NULL page_ids");
-  if (reinterpret_cast<uintptr_t>(pool.ids) & 3u) return fail(PACE_KV_EINVAL, "page ids are not 4-byte aligned");
-  if (pool.host_ids != nullptr && n_pages > PACE_KV_INLINE_IDS)
-    return fail(PACE_KV_ERANGE, "more than %d pages cannot travel in the kernel arguments", PACE_KV_INLINE_IDS);
+int launch_host_leg(const Side& pool, const Side& host, bool to_host, int num_layers, int64_t n_pages,
+                    int64_t page_bytes, int32_t* err_count, hipStream_t stream) {
   constexpr int64_t kMaxVecs = int64_t(1) << 31;  // of one launch: 32-bit indexes, with room for a round past the end
+  const bool paged = host.ids != nullptr;
   const int64_t page_vecs = page_bytes / kVecBytes;
-  if (n_pages > kMaxVecs / page_vecs) return fail(PACE_KV_ERANGE, "host leg: a layer of more than 32 GiB");
+  // Refusals, empty pools (no page to read in a bad id's place) and layers of
+  // 32 GiB and more are the page copy's.
+  if (num_layers <= 0 || n_pages <= 0 || page_vecs <= 0 || page_bytes % kVecBytes != 0 || pool.pool_pages < 1 ||
+      host.pool_pages < (paged ? 1 : n_pages) || n_pages > kMaxVecs / page_vecs ||
+      (pool.ids == nullptr && pool.host_ids == nullptr) || host.host_ids != nullptr ||
+      (paged && pool.host_ids != nullptr) || (reinterpret_cast<uintptr_t>(pool.ids) & 3u) != 0 ||
+      (reinterpret_cast<uintptr_t>(host.ids) & 3u) != 0 || (pool.host_ids != nullptr && n_pages > PACE_KV_INLINE_IDS))
+    return launch_page_copy(to_host ? pool : host, to_host ? host : pool, num_layers, n_pages, page_bytes, err_count,
+                            stream);
+  PACE_KV_TRY(check_layers((to_host ? pool : host).layers, num_layers, "source"));
+  PACE_KV_TRY(check_layers((to_host ? host : pool).layers, num_layers, "destination"));
   const int64_t fit = kMaxVecs / (n_pages * page_vecs);
   const int step = static_cast<int>(std::min<int64_t>({fit, kMaxLayers, num_layers}));
   for (int l0 = 0; l0 < num_layers; l0 += step) {
@@ -581,33 +594,49 @@ int launch_host_leg(const Side& pool, char* host, bool to_host, int num_layers, 
     HostLegParamsInline q;
     memset(&q.base, 0, sizeof(q.base));
     HostLegParams& p = q.base;
-    for (int l = 0; l < nl; ++l) p.layers[l] = const_cast<char*>(pool.layers[l0 + l]);
-    p.host = reinterpret_cast<u32x4*>(host + l0 * n_pages * page_bytes);
+    for (int l = 0; l < nl; ++l) {
+      p.layers[l] = const_cast<char*>(pool.layers[l0 + l]);
+      p.host[l] = const_cast<char*>(host.layers[l0 + l]);
+    }
     p.ids = pool.ids;
+    p.host_ids = host.ids;
     p.err = err_count;
     p.page_bytes = page_bytes;
     p.pool_pages = static_cast<uint32_t>(std::min<int64_t>(pool.pool_pages, INT32_MAX));
+    p.host_pages = static_cast<uint32_t>(std::min<int64_t>(host.pool_pages, INT32_MAX));
     p.page_vecs = static_cast<uint32_t>(page_vecs);
     p.n_pages = static_cast<uint32_t>(n_pages);
     p.total_vecs = static_cast<uint32_t>(nl * n_pages * page_vecs);
     p.by_page = fast_div(p.page_vecs);
     p.by_count = fast_div(p.n_pages);
-    const int64_t most = (p.total_vecs + kHostThreads - 1) / kHostThreads;
-    const dim3 grid(static_cast<uint32_t>(std::min<int64_t>(to_host ? kOutGroups : kInGroups, most)));
+    const int64_t most = (int64_t(p.total_vecs) + kHostThreads - 1) / kHostThreads;
+    const int groups = !to_host ? kInGroups : paged ? kPagedOutGroups : kOutGroups;
+    const dim3 grid(static_cast<uint32_t>(std::min<int64_t>(groups, most)));
     const void* fn;
-    void* args[] = {&q};
-    if (pool.host_ids != nullptr) {
+    void* args[] = {&p};
+    if (paged) {
+      fn = to_host ? reinterpret_cast<const void*>(&host_leg_kernel<true, true>)
+                   : reinterpret_cast<const void*>(&host_leg_kernel<false, true>);
+    } else if (pool.host_ids == nullptr) {
+      fn = to_host ? reinterpret_cast<const void*>(&host_leg_kernel<true, false>)
+                   : reinterpret_cast<const void*>(&host_leg_kernel<false, false>);
+    } else {
       memcpy(q.ids, pool.host_ids, n_pages * sizeof(int32_t));
+      args[0] = &q;
       fn = to_host ? reinterpret_cast<const void*>(&host_leg_inline_kernel<true>)
                    : reinterpret_cast<const void*>(&host_leg_inline_kernel<false>);
-    } else {
-      fn = to_host ? reinterpret_cast<const void*>(&host_leg_kernel<true>)
-                   : reinterpret_cast<const void*>(&host_leg_kernel<false>);
-      args[0] = &p;
     }
     PACE_KV_TRY(hip_status(hipLaunchKernel(fn, grid, dim3(kHostThreads), args, 0, stream), "host leg launch"));
   }
   return PACE_KV_OK;
+}
+
+int launch_host_leg(const Side& pool, char* host, bool to_host, int num_layers, int64_t n_pages, int64_t page_bytes,
+                    int32_t* err_count, hipStream_t stream) {
+  std::vector<const char*> buf(std::max(num_layers, 0));
+  buffer_layers(host, n_pages * page_bytes, num_layers, buf.data());
+  return launch_host_leg(pool, Side{buf.data(), nullptr, n_pages}, to_host, num_layers, n_pages, page_bytes, err_count,
+                         stream);
 }
 
 int buffered_copy(const Side& src, const Side& dst, char* buffer, int64_t buffer_layer_stride, int buffer_layers,
@@ -746,9 +775,9 @@ int swap_copy(const void* const* src_layers, int64_t src_pool_pages, const int32
   std::vector<const char*> s, d;
   PACE_KV_TRY(resolve_layers(src_layers, num_layers, src_pool_pages * page_bytes, src_host, s, what));
   PACE_KV_TRY(resolve_layers(dst_layers, num_layers, dst_pool_pages * page_bytes, dst_host, d, what));
-  Side src{s.data(), src_ids, src_pool_pages};
-  Side dst{d.data(), dst_ids, dst_pool_pages};
-  return launch_page_copy(src, dst, num_layers, n_pages, page_bytes, err_count, stream);
+  const Side src{s.data(), src_ids, src_pool_pages}, dst{d.data(), dst_ids, dst_pool_pages};
+  return launch_host_leg(dst_host ? src : dst, dst_host ? dst : src, dst_host, num_layers, n_pages, page_bytes,
+                         err_count, stream);
 }
 
 }  // namespace pace_kv

@@ -75,3 +75,34 @@ def test_host_memory_that_no_kernel_copies(gpu):
             dst.zero_()
             st.roundtrip(src_l, ids, dst_l, ids, host, layers)
             assert torch.equal(dst.cpu()[:, ids], src.cpu()[:, ids])
+
+
+@pytest.mark.parametrize("bad", [False, True])
+@pytest.mark.parametrize("layers,n,page_bytes", [(1, 1, 1024), (3, 33, 1056), (70, 5, 2048), (2, 900, 1024), (5, 40, 65536),
+                                                 (3, 50, 1008)])
+def test_swaps(gpu, layers, n, page_bytes, bad):
+    """Pages with ids on both sides; a page whose id is out of range on either
+    is skipped and counted once."""
+    N, M = n + 5, n + 3
+    gen = torch.Generator().manual_seed(n * page_bytes)
+    src, src_l = pool(layers, N, page_bytes, gen, gpu)
+    host = ops.HostPagePool(layers, M, tuple(src.shape[2:]), torch.float8_e4m3fn)
+    d_ids, h_ids = torch.randperm(N, generator=gen)[:n], torch.randperm(M, generator=gen)[:n]
+    if bad:
+        d_ids[0], h_ids[n - 1], h_ids[n // 2], d_ids[n // 2] = -1, M, -2 ** 31, N
+    ok = (d_ids >= 0) & (d_ids < N) & (h_ids >= 0) & (h_ids < M)
+    ids = [t.to(torch.int32).to(gpu) for t in (d_ids, h_ids)]
+    err = torch.zeros(1, dtype=torch.int32, device=gpu)
+    for l, t in enumerate(host.layers):
+        t.view(torch.uint8).fill_(121 + l % 2)
+    want = torch.stack([t.view(torch.uint8) for t in host.layers]).clone()
+    want[:, h_ids[ok]] = src.cpu()[:, d_ids[ok]]
+    ops.swap_out(src_l, ids[0], host, ids[1], err=err)
+    torch.cuda.synchronize()
+    assert torch.equal(torch.stack([t.view(torch.uint8) for t in host.layers]), want)
+    before = torch.randint(0, 120, tuple(src.shape), dtype=torch.uint8, generator=gen)
+    src.copy_(before)
+    ops.swap_in(host, ids[1], src_l, ids[0], err=err)
+    before[:, d_ids[ok]] = want[:, h_ids[ok]]
+    assert torch.equal(src.cpu(), before)
+    assert int(err.item()) == 2 * layers * int((~ok).sum())
