@@ -19,8 +19,9 @@ advanced indexing into a temporary device tensor and copies it to *pageable*
 host memory synchronously, L times; here one kernel per layer chunk packs the
 pages into a device slot while the previous chunk streams to *pinned* host
 memory on a side stream (pace_kv_pack_to_host), and insert is the mirror
-(pace_kv_unpack_from_host).  Device-resident transfer buffers skip the host
-leg (pack_pages / unpack_pages).
+(pace_kv_unpack_from_host).  A request of one chunk needs no slot: one kernel
+copies between its pages and the pinned host memory.  Device-resident transfer
+buffers skip the host leg (pack_pages / unpack_pages).
 """
 from __future__ import annotations
 

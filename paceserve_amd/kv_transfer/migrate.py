@@ -11,11 +11,11 @@ One promote() call:
   3. uploads both id lists (CSR-concatenated over requests) with one pinned
      host-to-device copy;
   4. moves the pages in one of three modes:
-       "buffer": pack into a device transfer buffer, then unpack - the
-                 reference's two-step semantics, with the buffer as the
-                 device-resident KVobj payload; layer-chunked when the
-                 buffer would be large;
-       "fused":  pool-to-pool move, no buffer (half the HBM traffic);
+       "buffer": pack into a device transfer buffer and unpack out of it - the
+                 reference's two-step semantics, in one launch that reads each
+                 page once, with the buffer as the device-resident KVobj
+                 payload; layer-chunked when the buffer would be large;
+       "fused":  pool-to-pool move, no buffer (two thirds of that HBM traffic);
        "pinned": the full device->host->device round trip through pinned
                  memory, overlapped per layer chunk (pace_kv_roundtrip).
 Each request's slice of the transfer buffer, buf[:, indptr[r]:indptr[r+1]],
