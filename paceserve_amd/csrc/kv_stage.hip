@@ -139,10 +139,10 @@ struct pace_kv_stager {
   hipStream_t d2h = nullptr;
   hipStream_t h2d = nullptr;
   hipEvent_t work_start = nullptr;  // the caller's stream at the start of a round trip
-  hipEvent_t work_done = nullptr;   // everything a round trip enqueued
+  hipEvent_t work_done = nullptr;   // everything the last round trip enqueued
   hipEvent_t start = nullptr;
   hipEvent_t d2h_done = nullptr;
-  hipEvent_t h2d_done = nullptr;  // the last round trip's last H2D copy
+  hipEvent_t h2d_done = nullptr;
   // The kernel stream below is the work stream in a round trip and the
   // caller's stream in the one-way legs.
   std::vector<hipEvent_t> packed;    // out slot s filled (kernel stream)
@@ -584,22 +584,19 @@ int pace_kv_roundtrip(pace_kv_stager* s, const void* const* src_layers, int64_t 
   const bool host_kernel = direct_host(host_buf, regions * chunk_bytes);
   if (chunks == 1) {
     // One chunk leaves nothing to overlap: its stages run on the caller's
-    // stream, without the waits between streams.  They follow the packs and
-    // unpacks of earlier calls on this stager (work_done), the last reads of
-    // both slots and the previous call's last read of its host buffer, and
+    // stream, without the waits between streams.  They follow the earlier round
+    // trips on this stager (work_done) and the last reads of both slots, and
     // leave the records a later call waits on.
     hipStream_t caller = static_cast<hipStream_t>(stream_);
     const int64_t bytes = p.count(0) * p.layer_bytes;
     PACE_HIP(hipStreamWaitEvent(caller, s->work_done, 0), "wait earlier calls");
-    PACE_HIP(hipStreamWaitEvent(caller, s->h2d_done, 0), "wait previous round trip");
     if (host_kernel) {
       const pace_kv::Side src{reinterpret_cast<const char* const*>(src_layers), src_ids, src_pool_pages};
       const pace_kv::Side dst{reinterpret_cast<const char* const*>(dst_layers), dst_ids, dst_pool_pages};
       PACE_KV_TRY(pace_kv::launch_host_leg(src, host, true, num_layers, n_pages, page_bytes, err_count, caller));
-      // The records follow what was enqueued also when the way back fails to launch.
+      // The record follows what was enqueued also when the way back fails to launch.
       const int rc =
           pace_kv::launch_host_leg(dst, host, false, num_layers, n_pages, page_bytes, err_count, caller);
-      PACE_HIP(hipEventRecord(s->h2d_done, caller), "record h2d_done");
       PACE_HIP(hipEventRecord(s->work_done, caller), "record work_done");
       return rc;
     }
@@ -612,7 +609,6 @@ int pace_kv_roundtrip(pace_kv_stager* s, const void* const* src_layers, int64_t 
     PACE_HIP(d2h, "D2H copy");
     PACE_HIP(hipStreamWaitEvent(caller, s->in_free[0], 0), "wait in slot");
     PACE_HIP(hipMemcpyAsync(s->in_ring, host, bytes, hipMemcpyHostToDevice, caller), "H2D copy");
-    PACE_HIP(hipEventRecord(s->h2d_done, caller), "record h2d_done");
     // The records follow the H2D copy also when the unpack fails to launch.
     const int rc = unpack_chunk(s, p, 0, dst_layers, dst_pool_pages, {dst_ids, nullptr}, err_count, caller);
     PACE_HIP(hipEventRecord(s->in_free[0], caller), "record in_free");
@@ -628,12 +624,12 @@ int pace_kv_roundtrip(pace_kv_stager* s, const void* const* src_layers, int64_t 
   WorkJoin join{s, caller};
   PACE_HIP(hipEventRecord(s->work_start, caller), "record work_start");
   PACE_HIP(hipStreamWaitEvent(stream, s->work_start, 0), "wait work_start");
+  // Nothing above orders the work stream after a one-chunk call on another
+  // caller's stream, whose destination pages this call may read.  Every copy
+  // follows a pack of this call and so the previous call too, whose regions of
+  // the host buffer may lie differently.
+  PACE_HIP(hipStreamWaitEvent(stream, s->work_done, 0), "wait earlier calls");
   const int S = s->num_slots;
-  // A region's events order its reuse within a call and between calls of one
-  // chunk size; a call with another chunk size (or host buffer) carves other
-  // regions, so its first D2H copy waits for the previous call's last H2D
-  // copy to have read the host buffer.
-  PACE_HIP(hipStreamWaitEvent(s->d2h, s->h2d_done, 0), "wait previous round trip");
   // The stages of chunk c; each wait names an event whose record for the
   // chunk it must follow is the latest one enqueued when the wait is.
   auto pack = [&](int c) -> int {
@@ -698,7 +694,6 @@ int pace_kv_roundtrip(pace_kv_stager* s, const void* const* src_layers, int64_t 
       PACE_KV_TRY(h2d_record(c));
       PACE_KV_TRY(unpack(c));
     }
-    PACE_HIP(hipEventRecord(s->h2d_done, s->h2d), "record h2d_done");
     return join.now();
   }
   // Step i enqueues unpack(i-S) and pack(i+1) on `stream`, then both copy
@@ -729,7 +724,6 @@ int pace_kv_roundtrip(pace_kv_stager* s, const void* const* src_layers, int64_t 
     if (h) PACE_KV_TRY(h2d_record(i - 1));
     if (d) PACE_KV_TRY(d2h_record(i));
   }
-  PACE_HIP(hipEventRecord(s->h2d_done, s->h2d), "record h2d_done");
   // The last unpack is on the work stream: the caller's later work comes
   // after it.
   return join.now();

@@ -106,3 +106,25 @@ def test_swaps(gpu, layers, n, page_bytes, bad):
     before[:, d_ids[ok]] = want[:, h_ids[ok]]
     assert torch.equal(src.cpu(), before)
     assert int(err.item()) == 2 * layers * int((~ok).sum())
+
+
+@pytest.mark.parametrize("second", ["one chunk", "chunks"])
+def test_a_round_trip_reads_what_the_one_before_it_wrote(gpu, second):
+    """A migration chain on two streams, its first call held up: the second
+    call's source pages are the first one's destination."""
+    layers, n, page_bytes = 6, 12, 4096
+    gen = torch.Generator().manual_seed(4)
+    (a, a_l), (b, b_l), (c, c_l) = (pool(layers, n, page_bytes, gen, gpu) for _ in range(3))
+    ids = torch.randperm(n, generator=gen).to(torch.int32).to(gpu)
+    size = layers * n * page_bytes
+    hosts = [torch.empty(size, dtype=torch.uint8, pin_memory=True) for _ in range(2)]
+    x, y = torch.cuda.Stream(gpu), torch.cuda.Stream(gpu)
+    torch.cuda.synchronize()
+    with ops.Stager(size, 3) as st:
+        with torch.cuda.stream(x):
+            torch.cuda._sleep(20_000_000)
+            st.roundtrip(a_l, ids, b_l, ids, hosts[0], layers)
+        with torch.cuda.stream(y):
+            st.roundtrip(b_l, ids, c_l, ids, hosts[1], layers if second == "one chunk" else 2)
+        torch.cuda.synchronize()
+    assert torch.equal(b.cpu(), a.cpu()) and torch.equal(c.cpu(), a.cpu())
