@@ -191,6 +191,12 @@ int pace_kv_swap_in(const void* const* host_layers, int64_t host_pool_pages,
  * priority) and the events that order them against the caller's stream.
  * Each slot holds slot_bytes; a layer chunk of k layers needs
  * k * n_pages * page_bytes <= slot_bytes.
+ * Calls on one stager run their packs and unpacks in call order, whichever
+ * `stream` each names.  The exception is a pack_to_host and an
+ * unpack_from_host, which leave each other alone, so that on two streams they
+ * keep both directions of the link busy: where one of them needs the other's
+ * pages or host buffer, the caller orders their streams.  A call made while
+ * `stream` is captured is ordered by the graph alone.
  */
 typedef struct pace_kv_stager pace_kv_stager;
 
@@ -228,8 +234,8 @@ int pace_kv_pack_to_host(pace_kv_stager* stager,
  * copied host-to-device on the H2D side stream while chunk c-1 is unpacked on
  * `stream`; a call of one chunk runs on `stream`: one kernel scatters host_in's
  * pages when that is pinned memory the device addresses, on a 16-byte
- * boundary, else a copy and an unpack.  When the call returns, `stream` is ordered after every copy it enqueued, also when
- * it fails part-way.
+ * boundary, else a copy and an unpack.  When the call returns, `stream` is
+ * ordered after every copy it enqueued, also when it fails part-way.
  *
  * Replaces the pageable host-to-device copy + scatter loop of
  * KVhelper.insert_kv_cache (paceserve/kv_transfer/kv_utils.py:49-52).
@@ -309,8 +315,7 @@ int pace_kv_pack_to_host_noalloc(const void* const* src_layers, int num_layers,
  * waits for everything the call enqueued, so `stream`'s later work comes
  * after the last unpack (also when the call fails part-way).  The copies
  * overlap however the runtime maps these streams onto its hardware queues.
- * Calls on one stager run their packs and unpacks in call order, whichever
- * `stream` each names.  A call of one chunk has nothing to overlap and runs
+ * A call of one chunk has nothing to overlap and runs
  * its stages on `stream`, after the stager's earlier calls: with pinned memory
  * the device addresses, on a 16-byte boundary, the two kernels of the one-way
  * calls, else pack, two copies and unpack.

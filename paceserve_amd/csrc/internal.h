@@ -96,13 +96,14 @@ int buffered_copy(const Side& src, const Side& dst, char* buffer, int64_t buffer
 // launch_page_copy between device pages (`pool`, with ids) and pinned memory
 // that the device addresses (`host`: a pool with device ids, or, without ids,
 // [num_layers][n_pages][page_bytes] in one piece), out to the host (to_host) or in
-// from it, with few waves.
+// from it, with few waves.  `done`, if given, is recorded behind a copy whose
+// every launch succeeded.
 int launch_host_leg(const Side& pool, const Side& host, bool to_host, int num_layers, int64_t n_pages,
-                    int64_t page_bytes, int32_t* err_count, hipStream_t stream);
+                    int64_t page_bytes, int32_t* err_count, hipStream_t stream, hipEvent_t done = nullptr);
 
 // The same with the host side laid out [num_layers][n_pages][page_bytes].
 int launch_host_leg(const Side& pool, char* host, bool to_host, int num_layers, int64_t n_pages, int64_t page_bytes,
-                    int32_t* err_count, hipStream_t stream);
+                    int32_t* err_count, hipStream_t stream, hipEvent_t done = nullptr);
 
 // pace_kv_pack and pace_kv_unpack for ids of either kind.
 int pack(const void* const* src_layers, int num_layers, int64_t pool_pages, const IdList& ids, int64_t n_pages,

@@ -25,6 +25,7 @@
 // ~6.6 TB/s, against ~5.6-5.9 TB/s for 8-32 KiB per workgroup, persistent
 // grid-stride loops or ids staged in LDS (a persistent loop serialises each
 // trip's loads behind the previous trip's stores on the shared vmcnt counter).
+#include <hip/hip_ext.h>
 #include <stdarg.h>
 #include <stdio.h>
 #include <string.h>
@@ -572,7 +573,7 @@ bool disjoint(const char* const* a, int64_t a_bytes, const char* const* b, int64
 }  // namespace
 
 int launch_host_leg(const Side& pool, const Side& host, bool to_host, int num_layers, int64_t n_pages,
-                    int64_t page_bytes, int32_t* err_count, hipStream_t stream) {
+                    int64_t page_bytes, int32_t* err_count, hipStream_t stream, hipEvent_t done) {
   constexpr int64_t kMaxVecs = int64_t(1) << 31;  // of one launch: 32-bit indexes, with room for a round past the end
   const bool paged = host.ids != nullptr;
   const int64_t page_vecs = page_bytes / kVecBytes;
@@ -582,9 +583,11 @@ int launch_host_leg(const Side& pool, const Side& host, bool to_host, int num_la
       host.pool_pages < (paged ? 1 : n_pages) || n_pages > kMaxVecs / page_vecs ||
       (pool.ids == nullptr && pool.host_ids == nullptr) || host.host_ids != nullptr ||
       (paged && pool.host_ids != nullptr) || (reinterpret_cast<uintptr_t>(pool.ids) & 3u) != 0 ||
-      (reinterpret_cast<uintptr_t>(host.ids) & 3u) != 0 || (pool.host_ids != nullptr && n_pages > PACE_KV_INLINE_IDS))
-    return launch_page_copy(to_host ? pool : host, to_host ? host : pool, num_layers, n_pages, page_bytes, err_count,
-                            stream);
+      (reinterpret_cast<uintptr_t>(host.ids) & 3u) != 0 || (pool.host_ids != nullptr && n_pages > PACE_KV_INLINE_IDS)) {
+    PACE_KV_TRY(launch_page_copy(to_host ? pool : host, to_host ? host : pool, num_layers, n_pages, page_bytes,
+                                 err_count, stream));
+    return done != nullptr ? hip_status(hipEventRecord(done, stream), "host leg record") : PACE_KV_OK;
+  }
   PACE_KV_TRY(check_layers((to_host ? pool : host).layers, num_layers, "source"));
   PACE_KV_TRY(check_layers((to_host ? host : pool).layers, num_layers, "destination"));
   const int64_t fit = kMaxVecs / (n_pages * page_vecs);
@@ -626,17 +629,25 @@ int launch_host_leg(const Side& pool, const Side& host, bool to_host, int num_la
       fn = to_host ? reinterpret_cast<const void*>(&host_leg_inline_kernel<true>)
                    : reinterpret_cast<const void*>(&host_leg_inline_kernel<false>);
     }
-    PACE_KV_TRY(hip_status(hipLaunchKernel(fn, grid, dim3(kHostThreads), args, 0, stream), "host leg launch"));
+    // The launch records the event itself: a record behind it would be a packet
+    // of its own, with a wait around it.  Measured on MI355X, a pair of legs
+    // that each end with a record of the caller's: 4 us longer with the event
+    // here, 9 with a record.
+    if (done != nullptr && l0 + nl == num_layers)
+      PACE_KV_TRY(hip_status(hipExtLaunchKernel(fn, grid, dim3(kHostThreads), args, 0, stream, nullptr, done, 0),
+                             "host leg launch"));
+    else
+      PACE_KV_TRY(hip_status(hipLaunchKernel(fn, grid, dim3(kHostThreads), args, 0, stream), "host leg launch"));
   }
   return PACE_KV_OK;
 }
 
 int launch_host_leg(const Side& pool, char* host, bool to_host, int num_layers, int64_t n_pages, int64_t page_bytes,
-                    int32_t* err_count, hipStream_t stream) {
+                    int32_t* err_count, hipStream_t stream, hipEvent_t done) {
   std::vector<const char*> buf(std::max(num_layers, 0));
   buffer_layers(host, n_pages * page_bytes, num_layers, buf.data());
   return launch_host_leg(pool, Side{buf.data(), nullptr, n_pages}, to_host, num_layers, n_pages, page_bytes, err_count,
-                         stream);
+                         stream, done);
 }
 
 int buffered_copy(const Side& src, const Side& dst, char* buffer, int64_t buffer_layer_stride, int buffer_layers,

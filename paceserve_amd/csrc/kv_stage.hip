@@ -58,6 +58,7 @@
 // that slot, so back-to-back calls on one stager are ordered correctly.
 #include <string.h>
 
+#include <initializer_list>
 #include <mutex>
 #include <vector>
 
@@ -140,6 +141,8 @@ struct pace_kv_stager {
   hipStream_t h2d = nullptr;
   hipEvent_t work_start = nullptr;  // the caller's stream at the start of a round trip
   hipEvent_t work_done = nullptr;   // everything the last round trip enqueued
+  hipEvent_t out_done = nullptr;    // everything the last pack to host enqueued
+  hipEvent_t in_done = nullptr;     // the unpacks of the last unpack from host
   hipEvent_t start = nullptr;
   hipEvent_t d2h_done = nullptr;
   hipEvent_t h2d_done = nullptr;
@@ -176,6 +179,8 @@ void release(pace_kv_stager* s) {
   if (s->work) (void)hipStreamDestroy(s->work);
   if (s->work_start) (void)hipEventDestroy(s->work_start);
   if (s->work_done) (void)hipEventDestroy(s->work_done);
+  if (s->out_done) (void)hipEventDestroy(s->out_done);
+  if (s->in_done) (void)hipEventDestroy(s->in_done);
   if (s->d2h) (void)hipStreamDestroy(s->d2h);
   if (s->h2d) (void)hipStreamDestroy(s->h2d);
   if (s->start) (void)hipEventDestroy(s->start);
@@ -328,6 +333,43 @@ int unpack_chunk(pace_kv_stager* s, const ChunkPlan& p, int c, void* const* dst_
                         p.n_pages, p.page_bytes, err, stream);
 }
 
+// Calls on one stager run in call order, whichever stream each names, but for
+// a pack to host and an unpack from host, which leave each other alone so that
+// both directions of the link can be busy: a call's packs and unpacks follow
+// the events of the earlier calls, and it records its own.  A call that is
+// captured into a graph takes no part in this: the graph's replays have no
+// place in the order of calls, and an event recorded in a capture could not be
+// waited for outside of it.
+bool capturing(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return false;
+}
+
+int follow(hipStream_t stream, std::initializer_list<hipEvent_t> earlier) {
+  if (capturing(stream)) return PACE_KV_OK;
+  for (hipEvent_t e : earlier) PACE_HIP(hipStreamWaitEvent(stream, e, 0), "wait earlier calls");
+  return PACE_KV_OK;
+}
+
+// Records `done` behind a call that returns `rc`, also when it failed
+// part-way; returns the call's status, or else the record's.
+int finish(int rc, hipStream_t stream, hipEvent_t done) {
+  if (capturing(stream)) return rc;
+  const int recorded = hip_status(hipEventRecord(done, stream), "record the call");
+  return rc ? rc : recorded;
+}
+
+// A direct leg of one chunk, `done` recorded by its launch.
+int direct_leg(const pace_kv::Side& pool, void* host, bool to_host, const ChunkPlan& p, int32_t* err,
+               hipStream_t stream, hipEvent_t done) {
+  const bool eager = !capturing(stream);
+  const int rc = pace_kv::launch_host_leg(pool, static_cast<char*>(host), to_host, p.num_layers, p.n_pages,
+                                          p.page_bytes, err, stream, eager ? done : nullptr);
+  return rc && eager ? finish(rc, stream, done) : rc;
+}
+
 // Makes `caller` wait for everything a round trip enqueued: now() on the
 // success path (reporting a failure), where the last unpack on the work
 // stream already follows every copy; the destructor on an early error return
@@ -339,8 +381,9 @@ struct WorkJoin {
   bool joined = false;
   int now() {
     joined = true;
-    PACE_HIP(hipEventRecord(s->work_done, s->work), "record work_done");
-    PACE_HIP(hipStreamWaitEvent(caller, s->work_done, 0), "wait work_done");
+    const hipEvent_t done = capturing(s->work) ? s->work_start : s->work_done;
+    PACE_HIP(hipEventRecord(done, s->work), "record work_done");
+    PACE_HIP(hipStreamWaitEvent(caller, done, 0), "wait work_done");
     return PACE_KV_OK;
   }
   ~WorkJoin() {
@@ -366,25 +409,13 @@ struct SideJoin {
   }
 };
 
-int pack_to_host(pace_kv_stager* s, const void* const* src_layers, int num_layers, int64_t pool_pages,
-                 const IdList& page_ids, int64_t n_pages, int64_t page_bytes, int layers_per_chunk, void* host_out,
-                 int32_t* err_count, hipStream_t stream) {
-  PACE_KV_TRY(check_stager(s));
-  ChunkPlan p;
-  PACE_KV_TRY(make_plan(s, num_layers, n_pages, page_bytes, layers_per_chunk, &p));
-  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
-  if (host_out == nullptr) return fail(PACE_KV_EINVAL, "pack_to_host: host_out is NULL");
+// A pack to host through the out slots; `stream` is ordered after what it
+// enqueued however it returns.
+int pack_through_slots(pace_kv_stager* s, const ChunkPlan& p, const void* const* src_layers, int64_t pool_pages,
+                       const IdList& page_ids, void* host_out, int32_t* err_count, hipStream_t stream) {
   const int chunks = p.num_chunks();
   if (chunks == 1) {
-    // One chunk leaves nothing to overlap, so everything runs on `stream`,
-    // without the waits between streams (measured on MI355X: 30-36 us less per
-    // call for 2-8 MiB requests, about 1% less at 128 MiB).
     const int64_t bytes = p.num_layers * p.layer_bytes;
-    if (direct_host(host_out, bytes)) {
-      const pace_kv::Side src{reinterpret_cast<const char* const*>(src_layers), page_ids.dev, pool_pages, page_ids.host};
-      return pace_kv::launch_host_leg(src, static_cast<char*>(host_out), true, num_layers, n_pages, page_bytes,
-                                      err_count, stream);
-    }
     PACE_HIP(hipStreamWaitEvent(stream, s->out_free[0], 0), "wait out slot");
     PACE_KV_TRY(pack_chunk(s, p, 0, src_layers, pool_pages, page_ids, err_count, stream));
     // out_free follows the pack also when the copy fails to enqueue.
@@ -423,23 +454,35 @@ int pack_to_host(pace_kv_stager* s, const void* const* src_layers, int num_layer
   return PACE_KV_OK;
 }
 
-int unpack_from_host(pace_kv_stager* s, const void* host_in, void* const* dst_layers, int num_layers,
-                     int64_t pool_pages, const IdList& page_ids, int64_t n_pages, int64_t page_bytes,
-                     int layers_per_chunk, int32_t* err_count, hipStream_t stream) {
+int pack_to_host(pace_kv_stager* s, const void* const* src_layers, int num_layers, int64_t pool_pages,
+                 const IdList& page_ids, int64_t n_pages, int64_t page_bytes, int layers_per_chunk, void* host_out,
+                 int32_t* err_count, hipStream_t stream) {
   PACE_KV_TRY(check_stager(s));
   ChunkPlan p;
   PACE_KV_TRY(make_plan(s, num_layers, n_pages, page_bytes, layers_per_chunk, &p));
   if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
-  if (host_in == nullptr) return fail(PACE_KV_EINVAL, "unpack_from_host: host_in is NULL");
+  if (host_out == nullptr) return fail(PACE_KV_EINVAL, "pack_to_host: host_out is NULL");
+  PACE_KV_TRY(follow(stream, {s->out_done, s->work_done}));
+  // One chunk leaves nothing to overlap, so everything runs on `stream`,
+  // without the waits between streams (measured on MI355X: 30-36 us less per
+  // call for 2-8 MiB requests, about 1% less at 128 MiB).
+  if (p.num_chunks() == 1 && direct_host(host_out, p.num_layers * p.layer_bytes)) {
+    const pace_kv::Side src{reinterpret_cast<const char* const*>(src_layers), page_ids.dev, pool_pages, page_ids.host};
+    return direct_leg(src, host_out, true, p, err_count, stream, s->out_done);
+  }
+  return finish(pack_through_slots(s, p, src_layers, pool_pages, page_ids, host_out, err_count, stream), stream,
+                s->out_done);
+}
+
+// An unpack from host through the in slots; `stream` is ordered after what it
+// enqueued however it returns.
+int unpack_through_slots(pace_kv_stager* s, const ChunkPlan& p, const void* host_in, void* const* dst_layers,
+                         int64_t pool_pages, const IdList& page_ids, int32_t* err_count, hipStream_t stream) {
   const int chunks = p.num_chunks();
   if (chunks == 1) {
     // One chunk: everything runs on `stream` (as in the pack).
+    PACE_KV_TRY(follow(stream, {s->in_done, s->work_done}));
     const int64_t bytes = p.num_layers * p.layer_bytes;
-    if (direct_host(host_in, bytes)) {
-      const pace_kv::Side dst{reinterpret_cast<const char* const*>(dst_layers), page_ids.dev, pool_pages, page_ids.host};
-      return pace_kv::launch_host_leg(dst, const_cast<char*>(static_cast<const char*>(host_in)), false, num_layers,
-                                      n_pages, page_bytes, err_count, stream);
-    }
     PACE_HIP(hipStreamWaitEvent(stream, s->in_free[0], 0), "wait in slot");
     PACE_HIP(hipMemcpyAsync(s->in_ring, host_in, bytes, hipMemcpyHostToDevice, stream), "H2D copy");
     // in_free follows the copy also when the unpack fails to launch.
@@ -452,6 +495,8 @@ int unpack_from_host(pace_kv_stager* s, const void* host_in, void* const* dst_la
   PACE_HIP(hipStreamWaitEvent(s->h2d, s->start, 0), "wait start");
   // On success the last unpack, on `stream`, follows every copy.
   SideJoin join{s->h2d, stream, s->start};
+  // The unpacks follow the earlier calls; the copies wait for their slots only.
+  PACE_KV_TRY(follow(stream, {s->in_done, s->work_done}));
   // Step i enqueues the copy of chunk i + 1, then unpack(i), whose wait for
   // chunk i's copy then holds back (on a shared hardware queue) only the copy
   // of chunk i + 2.  That copy refills the slot of chunk i + 2 - num_slots,
@@ -478,6 +523,23 @@ int unpack_from_host(pace_kv_stager* s, const void* host_in, void* const* dst_la
   return PACE_KV_OK;
 }
 
+int unpack_from_host(pace_kv_stager* s, const void* host_in, void* const* dst_layers, int num_layers,
+                     int64_t pool_pages, const IdList& page_ids, int64_t n_pages, int64_t page_bytes,
+                     int layers_per_chunk, int32_t* err_count, hipStream_t stream) {
+  PACE_KV_TRY(check_stager(s));
+  ChunkPlan p;
+  PACE_KV_TRY(make_plan(s, num_layers, n_pages, page_bytes, layers_per_chunk, &p));
+  if (num_layers == 0 || n_pages == 0) return PACE_KV_OK;
+  if (host_in == nullptr) return fail(PACE_KV_EINVAL, "unpack_from_host: host_in is NULL");
+  if (p.num_chunks() == 1 && direct_host(host_in, p.num_layers * p.layer_bytes)) {
+    PACE_KV_TRY(follow(stream, {s->in_done, s->work_done}));
+    const pace_kv::Side dst{reinterpret_cast<const char* const*>(dst_layers), page_ids.dev, pool_pages, page_ids.host};
+    return direct_leg(dst, const_cast<void*>(host_in), false, p, err_count, stream, s->in_done);
+  }
+  return finish(unpack_through_slots(s, p, host_in, dst_layers, pool_pages, page_ids, err_count, stream), stream,
+                s->in_done);
+}
+
 }  // namespace
 
 extern "C" {
@@ -499,6 +561,8 @@ int pace_kv_stager_create(int64_t slot_bytes, int num_slots, pace_kv_stager** ou
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->h2d, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&s->work_start, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&s->work_done, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&s->out_done, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&s->in_done, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&s->start, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&s->d2h_done, hipEventDisableTiming);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&s->h2d_done, hipEventDisableTiming);
@@ -584,36 +648,34 @@ int pace_kv_roundtrip(pace_kv_stager* s, const void* const* src_layers, int64_t 
   const bool host_kernel = direct_host(host_buf, regions * chunk_bytes);
   if (chunks == 1) {
     // One chunk leaves nothing to overlap: its stages run on the caller's
-    // stream, without the waits between streams.  They follow the earlier round
-    // trips on this stager (work_done) and the last reads of both slots, and
-    // leave the records a later call waits on.
+    // stream, without the waits between streams.  They follow the stager's
+    // earlier calls and, where they use them, the last reads of both slots.
     hipStream_t caller = static_cast<hipStream_t>(stream_);
     const int64_t bytes = p.count(0) * p.layer_bytes;
-    PACE_HIP(hipStreamWaitEvent(caller, s->work_done, 0), "wait earlier calls");
+    PACE_KV_TRY(follow(caller, {s->work_done, s->out_done, s->in_done}));
     if (host_kernel) {
       const pace_kv::Side src{reinterpret_cast<const char* const*>(src_layers), src_ids, src_pool_pages};
       const pace_kv::Side dst{reinterpret_cast<const char* const*>(dst_layers), dst_ids, dst_pool_pages};
-      PACE_KV_TRY(pace_kv::launch_host_leg(src, host, true, num_layers, n_pages, page_bytes, err_count, caller));
-      // The record follows what was enqueued also when the way back fails to launch.
-      const int rc =
-          pace_kv::launch_host_leg(dst, host, false, num_layers, n_pages, page_bytes, err_count, caller);
-      PACE_HIP(hipEventRecord(s->work_done, caller), "record work_done");
-      return rc;
+      // The record follows what was enqueued also when the way out fails to launch.
+      const int rc = pace_kv::launch_host_leg(src, host, true, num_layers, n_pages, page_bytes, err_count, caller);
+      return rc ? finish(rc, caller, s->work_done) : direct_leg(dst, host, false, p, err_count, caller, s->work_done);
     }
-    PACE_HIP(hipStreamWaitEvent(caller, s->out_free[0], 0), "wait out slot");
-    PACE_KV_TRY(pack_chunk(s, p, 0, src_layers, src_pool_pages, {src_ids, nullptr}, err_count, caller));
-    // out_free follows the pack also when the copy fails to enqueue.
-    const hipError_t d2h =
-        hipMemcpyAsync(host, s->out_ring, static_cast<size_t>(bytes), hipMemcpyDeviceToHost, caller);
-    PACE_HIP(hipEventRecord(s->out_free[0], caller), "record out_free");
-    PACE_HIP(d2h, "D2H copy");
-    PACE_HIP(hipStreamWaitEvent(caller, s->in_free[0], 0), "wait in slot");
-    PACE_HIP(hipMemcpyAsync(s->in_ring, host, bytes, hipMemcpyHostToDevice, caller), "H2D copy");
-    // The records follow the H2D copy also when the unpack fails to launch.
-    const int rc = unpack_chunk(s, p, 0, dst_layers, dst_pool_pages, {dst_ids, nullptr}, err_count, caller);
-    PACE_HIP(hipEventRecord(s->in_free[0], caller), "record in_free");
-    PACE_HIP(hipEventRecord(s->work_done, caller), "record work_done");
-    return rc;
+    const auto through_slots = [&]() -> int {
+      PACE_HIP(hipStreamWaitEvent(caller, s->out_free[0], 0), "wait out slot");
+      PACE_KV_TRY(pack_chunk(s, p, 0, src_layers, src_pool_pages, {src_ids, nullptr}, err_count, caller));
+      // out_free follows the pack also when the copy fails to enqueue.
+      const hipError_t d2h =
+          hipMemcpyAsync(host, s->out_ring, static_cast<size_t>(bytes), hipMemcpyDeviceToHost, caller);
+      PACE_HIP(hipEventRecord(s->out_free[0], caller), "record out_free");
+      PACE_HIP(d2h, "D2H copy");
+      PACE_HIP(hipStreamWaitEvent(caller, s->in_free[0], 0), "wait in slot");
+      PACE_HIP(hipMemcpyAsync(s->in_ring, host, bytes, hipMemcpyHostToDevice, caller), "H2D copy");
+      // in_free follows the copy also when the unpack fails to launch.
+      const int rc = unpack_chunk(s, p, 0, dst_layers, dst_pool_pages, {dst_ids, nullptr}, err_count, caller);
+      PACE_HIP(hipEventRecord(s->in_free[0], caller), "record in_free");
+      return rc;
+    };
+    return finish(through_slots(), caller, s->work_done);
   }
   // Packs and unpacks run on the stager's work stream, created together with
   // its two copy streams (see the file comment); the work stream starts after
@@ -624,11 +686,11 @@ int pace_kv_roundtrip(pace_kv_stager* s, const void* const* src_layers, int64_t 
   WorkJoin join{s, caller};
   PACE_HIP(hipEventRecord(s->work_start, caller), "record work_start");
   PACE_HIP(hipStreamWaitEvent(stream, s->work_start, 0), "wait work_start");
-  // Nothing above orders the work stream after a one-chunk call on another
-  // caller's stream, whose destination pages this call may read.  Every copy
-  // follows a pack of this call and so the previous call too, whose regions of
-  // the host buffer may lie differently.
-  PACE_HIP(hipStreamWaitEvent(stream, s->work_done, 0), "wait earlier calls");
+  // Nothing above orders the work stream after a call on another caller's
+  // stream, whose destination pages this call may read.  Every copy follows a
+  // pack of this call and so the previous round trip too, whose regions of the
+  // host buffer may lie differently.
+  PACE_KV_TRY(follow(stream, {s->work_done, s->out_done, s->in_done}));
   const int S = s->num_slots;
   // The stages of chunk c; each wait names an event whose record for the
   // chunk it must follow is the latest one enqueued when the wait is.

@@ -118,6 +118,12 @@ hipError_t hipLaunchKernel(const void* fn, dim3, dim3, void**, size_t, hipStream
   add(g_names[fn], s);
   return hipSuccess;
 }
+hipError_t hipExtLaunchKernel(const void* fn, dim3, dim3, void**, size_t, hipStream_t s, hipEvent_t, hipEvent_t stop,
+                              int) {
+  add(g_names[fn], s);
+  if (stop != nullptr) g_events[stop] = g_streams[s];
+  return hipSuccess;
+}
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
   const uintptr_t at = reinterpret_cast<uintptr_t>(p);
   auto it = g_pinned.upper_bound(at);

@@ -44,15 +44,35 @@ def in_order(earlier, later):
     return all(e["op"] in o["after"] for o in pages(later) for e in pages(earlier))
 
 
+KINDS = ["pack", "unpack", "trip"]
+OPPOSITE = {("pack", "unpack"), ("unpack", "pack")}    # leave each other alone
+
+
 @pytest.mark.parametrize("host", ["pinned", "pageable"])
-@pytest.mark.parametrize("second", ["trip:6", "trip:2"])
-@pytest.mark.parametrize("first", ["trip:6", "trip:2"])
-def test_a_round_trip_follows_the_round_trip_before_it(recorder, first, second, host):
-    """Of one chunk (on the caller's stream) or three (on the stager's): every
-    pack and unpack follows those of the call before, and what writes the host
-    buffer follows what read it."""
-    a, b = run(recorder, f"{first}:a:{host}", f"{second}:b:{host}")["calls"]
-    assert in_order(a, b)
-    assert all(e["op"] in o["after"] for o in b for e in a)
+@pytest.mark.parametrize("chunks", [(1, 1), (1, 3), (3, 1), (3, 3)])
+@pytest.mark.parametrize("second", KINDS)
+@pytest.mark.parametrize("first", KINDS)
+def test_a_call_follows_the_call_before_it(recorder, first, second, chunks, host):
+    """Two calls on two streams, of one chunk (on the caller's stream) or three
+    (on the stager's too): what the second does with pages follows what the
+    first does with them, and what writes a host buffer follows what used it,
+    but for a pack to host beside an unpack from host."""
+    k1, k2 = (6 // c for c in chunks)
+    a, b = run(recorder, f"{first}:{k1}:a:{host}", f"{second}:{k2}:b:pinned")["calls"]
+    if (first, second) in OPPOSITE:
+        assert not any(e["op"] in o["after"] for o in b for e in a)
+    else:
+        assert in_order(a, b)
+        if second != "unpack":    # an unpack's copies read the host buffer
+            assert all(e["op"] in o["after"] for o in b for e in a)
     for call in (a, b):
         assert all(o["joined"] for o in call)    # the caller's stream follows everything
+
+
+@pytest.mark.parametrize("call", ["pack:6", "unpack:6", "trip:6"])
+def test_a_captured_call_leaves_the_order_of_calls_alone(recorder, call):
+    """A pinned one-chunk call under capture waits for no event of earlier
+    calls, which belong to no graph, and the calls after it follow those."""
+    first, captured, last = run(recorder, "trip:6:a", "capture:g", f"{call}:g", "end:g", "trip:6:b")["calls"]
+    assert not any(e["op"] in o["after"] for o in captured for e in first)
+    assert in_order(first, last) and not any(e["op"] in o["after"] for o in last for e in captured)

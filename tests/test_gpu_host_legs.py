@@ -5,6 +5,7 @@ a launch takes, and page ids outside the pool."""
 import pytest
 import torch
 
+from paceserve_amd import _native
 from paceserve_amd.kv_transfer import ops
 
 pytestmark = pytest.mark.gpu
@@ -128,3 +129,78 @@ def test_a_round_trip_reads_what_the_one_before_it_wrote(gpu, second):
             st.roundtrip(b_l, ids, c_l, ids, hosts[1], layers if second == "one chunk" else 2)
         torch.cuda.synchronize()
     assert torch.equal(b.cpu(), a.cpu()) and torch.equal(c.cpu(), a.cpu())
+
+
+@pytest.mark.parametrize("first", ["unpack", "roundtrip", "roundtrip in chunks"])
+@pytest.mark.parametrize("second", ["unpack", "roundtrip"])
+def test_calls_into_the_same_pages_land_in_call_order(gpu, first, second):
+    """Two calls on two streams, the first held up: the second's pages stay.
+    The same for two packs into one host buffer."""
+    layers, n, page_bytes = 4, 12, 4096
+    gen = torch.Generator().manual_seed(5)
+    (src, src_l), (dst, dst_l) = pool(layers, n, page_bytes, gen, gpu), pool(layers, n, page_bytes, gen, gpu)
+    other, other_l = pool(layers, n, page_bytes, gen, gpu)
+    ids = torch.arange(n, dtype=torch.int32, device=gpu)
+    size = layers * n * page_bytes
+    hosts = [torch.empty((layers, n) + tuple(src.shape[2:]), dtype=torch.uint8, pin_memory=True) for _ in range(3)]
+    contents = [h.view(torch.float8_e4m3fn) for h in hosts]
+    for host, pages in zip(hosts, (src, other)):
+        host.copy_(pages.cpu())
+    a, b = torch.cuda.Stream(gpu), torch.cuda.Stream(gpu)
+    torch.cuda.synchronize()
+
+    def call(st, kind, i):
+        if kind == "unpack":
+            st.unpack_from_host(contents[i], dst_l, ids, layers)
+        else:
+            st.roundtrip((src_l, other_l)[i], ids, dst_l, ids, contents[i], 1 if "chunks" in kind else layers)
+
+    with ops.Stager(size, 3) as st:
+        with torch.cuda.stream(a):
+            torch.cuda._sleep(20_000_000)
+            call(st, first, 0)
+        with torch.cuda.stream(b):
+            call(st, second, 1)
+        torch.cuda.synchronize()
+        assert torch.equal(dst.cpu(), other.cpu())
+
+        with torch.cuda.stream(a):
+            torch.cuda._sleep(20_000_000)
+            st.pack_to_host(src_l, ids, contents[2], layers)
+        with torch.cuda.stream(b):
+            st.pack_to_host(other_l, ids, contents[2], layers)
+        torch.cuda.synchronize()
+        assert torch.equal(hosts[2], other.cpu())
+
+
+def test_one_chunk_legs_in_a_graph(gpu):
+    """Captured with the library's own calls, replayed among eager calls on
+    the same stager: each replay copies what the pages hold then."""
+    layers, n, page_bytes = 4, 12, 4096
+    gen = torch.Generator().manual_seed(6)
+    (src, src_l), (dst, dst_l) = pool(layers, n, page_bytes, gen, gpu), pool(layers, n, page_bytes, gen, gpu)
+    ids = torch.randperm(n, generator=gen).to(torch.int32).to(gpu)
+    host = torch.empty((layers, n) + tuple(src.shape[2:]), dtype=torch.uint8, pin_memory=True)
+    spare = torch.empty_like(host).pin_memory()
+    sp, dp, lib = ops.as_pool(src_l), ops.as_pool(dst_l), _native.load()
+    with ops.Stager(layers * n * page_bytes, 2) as st:
+        st.pack_to_host(src_l, ids, spare.view(torch.float8_e4m3fn), layers)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            stream = torch.cuda.current_stream().cuda_stream
+            _native.check(lib.pace_kv_pack_to_host(st._handle, sp.table(), layers, n, ids.data_ptr(), n, page_bytes,
+                                                   layers, host.data_ptr(), None, stream))
+            _native.check(lib.pace_kv_unpack_from_host(st._handle, host.data_ptr(), dp.table(), layers, n,
+                                                       ids.data_ptr(), n, page_bytes, layers, None, stream))
+        for i in range(4):
+            src.copy_(torch.randint(0, 120, tuple(src.shape), dtype=torch.uint8, generator=gen))
+            dst.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(dst.cpu(), src.cpu())
+            assert torch.equal(host, src.cpu()[:, ids.cpu().long()])
+            st.pack_to_host(src_l, ids, spare.view(torch.float8_e4m3fn), layers)
+            st.roundtrip(src_l, ids, dst_l, ids, spare, layers)
+            torch.cuda.synchronize()
+            assert torch.equal(spare.reshape(host.shape), host)
