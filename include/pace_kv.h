@@ -202,6 +202,7 @@ typedef struct pace_kv_stager pace_kv_stager;
 
 int pace_kv_stager_create(int64_t slot_bytes, int num_slots,
                           pace_kv_stager** out);
+/* Waits for everything the stager's calls enqueued, then frees it. */
 int pace_kv_stager_destroy(pace_kv_stager* stager);
 
 /*

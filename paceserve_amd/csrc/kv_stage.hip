@@ -585,9 +585,11 @@ int pace_kv_stager_destroy(pace_kv_stager* s) {
   (void)hipStreamSynchronize(s->work);
   hipError_t e1 = hipStreamSynchronize(s->d2h);
   hipError_t e2 = hipStreamSynchronize(s->h2d);
+  // The callers' streams: one-way packs and unpacks, and calls of one chunk.
+  for (hipEvent_t e : {s->out_done, s->in_done, s->work_done}) (void)hipEventSynchronize(e);
   for (hipEvent_t e : s->in_free) (void)hipEventSynchronize(e);
   for (hipEvent_t e : s->packed) (void)hipEventSynchronize(e);
-  for (hipEvent_t e : s->out_free) (void)hipEventSynchronize(e);  // one-chunk copies on the caller's stream
+  for (hipEvent_t e : s->out_free) (void)hipEventSynchronize(e);
   release(s);
   if (e1 != hipSuccess) return hip_status(e1, "stager_destroy (D2H stream)");
   return hip_status(e2, "stager_destroy (H2D stream)");

@@ -76,3 +76,12 @@ def test_a_captured_call_leaves_the_order_of_calls_alone(recorder, call):
     first, captured, last = run(recorder, "trip:6:a", "capture:g", f"{call}:g", "end:g", "trip:6:b")["calls"]
     assert not any(e["op"] in o["after"] for o in captured for e in first)
     assert in_order(first, last) and not any(e["op"] in o["after"] for o in last for e in captured)
+
+
+@pytest.mark.parametrize("host", ["pinned", "pageable"])
+@pytest.mark.parametrize("call", ["pack:6", "unpack:6", "trip:6", "pack:2", "unpack:2", "trip:2"])
+def test_destroy_waits_for_everything_before_it_frees(recorder, call, host):
+    """What every call enqueued has finished when a stager gives its memory
+    back, and with it the host tensors that Stager kept alive."""
+    assert run(recorder, f"{call}:a:{host}")["unwaited"] == 0
+    assert run(recorder, f"{call}:a:{host}", "trip:6:b", f"{call}:c:{host}")["unwaited"] == 0

@@ -204,3 +204,27 @@ def test_one_chunk_legs_in_a_graph(gpu):
             st.roundtrip(src_l, ids, dst_l, ids, spare, layers)
             torch.cuda.synchronize()
             assert torch.equal(spare.reshape(host.shape), host)
+
+
+@pytest.mark.parametrize("kind", ["pack", "unpack", "roundtrip"])
+def test_close_waits_for_one_chunk_calls(gpu, kind):
+    """A closed stager's calls have finished, on a stream that was held up."""
+    layers, n, page_bytes = 4, 12, 4096
+    gen = torch.Generator().manual_seed(7)
+    (src, src_l), (dst, dst_l) = pool(layers, n, page_bytes, gen, gpu), pool(layers, n, page_bytes, gen, gpu)
+    ids = torch.arange(n, dtype=torch.int32, device=gpu)
+    host = torch.empty((layers, n) + tuple(src.shape[2:]), dtype=torch.uint8, pin_memory=True)
+    host.copy_(src.cpu()) if kind == "unpack" else host.fill_(121)
+    content, stream = host.view(torch.float8_e4m3fn), torch.cuda.Stream(gpu)
+    torch.cuda.synchronize()
+    with ops.Stager(layers * n * page_bytes, 2) as st, torch.cuda.stream(stream):
+        torch.cuda._sleep(20_000_000)
+        if kind == "pack":
+            st.pack_to_host(src_l, ids, content, layers)
+        elif kind == "unpack":
+            st.unpack_from_host(content, dst_l, ids, layers)
+        else:
+            st.roundtrip(src_l, ids, dst_l, ids, content, layers)
+        st.close()
+    assert torch.equal(host, src.cpu())
+    assert kind == "pack" or torch.equal(dst.cpu(), src.cpu())
