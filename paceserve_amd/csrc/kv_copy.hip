@@ -577,11 +577,14 @@ int launch_host_leg(const Side& pool, const Side& host, bool to_host, int num_la
   constexpr int64_t kMaxVecs = int64_t(1) << 31;  // of one launch: 32-bit indexes, with room for a round past the end
   const bool paged = host.ids != nullptr;
   const int64_t page_vecs = page_bytes / kVecBytes;
-  // Refusals, empty pools (no page to read in a bad id's place) and layers of
-  // 32 GiB and more are the page copy's.
+  // The page copy would take a side without ids for a contiguous buffer.
+  if (num_layers > 0 && n_pages > 0 && pool.ids == nullptr && pool.host_ids == nullptr)
+    return fail(PACE_KV_EINVAL, "host leg: NULL page ids");
+  // Other refusals, empty pools (no page to read in a bad id's place) and
+  // layers of 32 GiB and more are the page copy's.
   if (num_layers <= 0 || n_pages <= 0 || page_vecs <= 0 || page_bytes % kVecBytes != 0 || pool.pool_pages < 1 ||
       host.pool_pages < (paged ? 1 : n_pages) || n_pages > kMaxVecs / page_vecs ||
-      (pool.ids == nullptr && pool.host_ids == nullptr) || host.host_ids != nullptr ||
+      host.host_ids != nullptr ||
       (paged && pool.host_ids != nullptr) || (reinterpret_cast<uintptr_t>(pool.ids) & 3u) != 0 ||
       (reinterpret_cast<uintptr_t>(host.ids) & 3u) != 0 || (pool.host_ids != nullptr && n_pages > PACE_KV_INLINE_IDS)) {
     PACE_KV_TRY(launch_page_copy(to_host ? pool : host, to_host ? host : pool, num_layers, n_pages, page_bytes,

@@ -4,7 +4,9 @@ JSON, the operations each call enqueued and which earlier ones they follow.
 usage: calls.py RECORDER LIBRARY CALL...
 A CALL is KIND:LAYERS_PER_CHUNK:STREAM[:HOST], with KIND pack, unpack or trip,
 STREAM a letter and HOST pinned (the default) or pageable; "capture:STREAM"
-and "end:STREAM" start and end a stream's capture."""
+and "end:STREAM" start and end a stream's capture.  A KIND of pack-null,
+unpack-null, inline-pack-null, inline-unpack-null, trip-null-src or
+trip-null-dst passes no page ids; its status is printed."""
 import ctypes
 import json
 import sys
@@ -30,7 +32,7 @@ def main(recorder, library, *calls):
     ids = vp(4 * BASE)
     stager = vp()
     assert lib.pace_kv_stager_create(i64(-(-size // 256) * 256), 3, ctypes.byref(stager)) == 0
-    out = []
+    out, status = [], []
     for call in calls:
         kind, *rest = call.split(":")
         if kind in ("capture", "end"):
@@ -39,20 +41,25 @@ def main(recorder, library, *calls):
         k, stream = int(rest[0]), vp(5 * BASE + ord(rest[1]))
         host = vp(pageable if rest[2:] == ["pageable"] else pinned)
         first = rec.rec_count()
-        pool = (layers, L, i64(64), ids, i64(N), i64(PAGE), k)
-        if kind == "pack":
-            rc = lib.pace_kv_pack_to_host(stager, *pool, host, None, stream)
-        elif kind == "unpack":
-            rc = lib.pace_kv_unpack_from_host(stager, host, *pool, None, stream)
+        pool = (layers, L, i64(64), None if "null" in kind else ids, i64(N), i64(PAGE), k)
+        suffix = "_inline" if kind.startswith("inline") else ""
+        if "unpack" in kind:
+            rc = getattr(lib, "pace_kv_unpack_from_host" + suffix)(stager, host, *pool, None, stream)
+        elif "pack" in kind:
+            rc = getattr(lib, "pace_kv_pack_to_host" + suffix)(stager, *pool, host, None, stream)
         else:
-            rc = lib.pace_kv_roundtrip(stager, layers, i64(64), ids, layers, i64(64), ids, L, i64(N), i64(PAGE), k,
+            src, dst = (None if kind == f"trip-null-{side}" else ids for side in ("src", "dst"))
+            rc = lib.pace_kv_roundtrip(stager, layers, i64(64), src, layers, i64(64), dst, L, i64(N), i64(PAGE), k,
                                        host, i64(size), None, stream)
-        assert rc == 0, (call, lib.pace_kv_last_error())
+        if "null" in kind:
+            status.append(rc)
+        else:
+            assert rc == 0, (call, lib.pace_kv_last_error())
         ops = range(first, rec.rec_count())
         out.append([{"op": o, "name": rec.rec_name(o).decode(), "after": [e for e in range(o) if rec.rec_follows(o, e)],
                      "joined": bool(rec.rec_stream_follows(stream, o))} for o in ops])
     assert lib.pace_kv_stager_destroy(stager) == 0
-    print(json.dumps({"calls": out, "unwaited": rec.rec_unwaited_at_free()}))
+    print(json.dumps({"calls": out, "status": status, "unwaited": rec.rec_unwaited_at_free()}))
 
 
 main(*sys.argv[1:])

@@ -33,11 +33,14 @@ def run(recorder, *calls):
     return json.loads(r.stdout)
 
 
-def pages(call):
+def pages_of(call):
     """The operations of a call that read or write pages."""
-    ops = [o for o in call if "page_copy" in o["name"] or "host_leg" in o["name"]]
-    assert ops
-    return ops
+    return [o for o in call if "page_copy" in o["name"] or "host_leg" in o["name"]]
+
+
+def pages(call):
+    assert pages_of(call)
+    return pages_of(call)
 
 
 def in_order(earlier, later):
@@ -85,3 +88,16 @@ def test_destroy_waits_for_everything_before_it_frees(recorder, call, host):
     back, and with it the host tensors that Stager kept alive."""
     assert run(recorder, f"{call}:a:{host}")["unwaited"] == 0
     assert run(recorder, f"{call}:a:{host}", "trip:6:b", f"{call}:c:{host}")["unwaited"] == 0
+
+
+@pytest.mark.parametrize("host", ["pinned", "pageable"])
+@pytest.mark.parametrize("k", [6, 2])
+@pytest.mark.parametrize("kind", ["pack", "unpack", "inline-pack", "inline-unpack", "trip-null-src", "trip-null-dst"])
+def test_missing_page_ids_are_refused(recorder, kind, k, host):
+    """NULL ids are an error of the caller's, not pages 0 to n - 1, however
+    many chunks a call has and whatever its host memory is."""
+    kind = kind if "null" in kind else f"{kind}-null"
+    got = run(recorder, f"{kind}:{k}:a:{host}", f"trip:6:b:{host}")
+    assert got["status"] == [_native.PACE_KV_EINVAL]
+    assert not pages_of(got["calls"][0]) or kind == "trip-null-dst"    # the way out comes first
+    assert all(e["op"] in o["after"] for o in pages(got["calls"][1]) for e in got["calls"][0])

@@ -228,3 +228,19 @@ def test_close_waits_for_one_chunk_calls(gpu, kind):
         st.close()
     assert torch.equal(host, src.cpu())
     assert kind == "pack" or torch.equal(dst.cpu(), src.cpu())
+
+
+@pytest.mark.parametrize("call", ["pack_to_host", "unpack_from_host", "pack_to_host_inline", "unpack_from_host_inline"])
+def test_missing_page_ids_leave_everything_as_it_was(gpu, call):
+    layers, n, page_bytes = 3, 5, 1024
+    gen = torch.Generator().manual_seed(8)
+    src, src_l = pool(layers, n, page_bytes, gen, gpu)
+    before, p, lib = src.cpu(), ops.as_pool(src_l), _native.load()
+    host = torch.full((layers, n, page_bytes), 121, dtype=torch.uint8, pin_memory=True)
+    stream = torch.cuda.current_stream().cuda_stream
+    with ops.Stager(-(-layers * n * page_bytes // 256) * 256, 2) as st:
+        pages = (p.table(), layers, n, None, n, page_bytes, layers)
+        args = (*pages, host.data_ptr()) if call.startswith("pack") else (host.data_ptr(), *pages)
+        assert getattr(lib, "pace_kv_" + call)(st._handle, *args, None, stream) == _native.PACE_KV_EINVAL
+        torch.cuda.synchronize()
+    assert torch.equal(src.cpu(), before) and bool((host == 121).all())
