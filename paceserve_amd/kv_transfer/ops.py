@@ -156,12 +156,17 @@ def device_ids(ids: IdsLike, device: torch.device, distinct: bool = False) -> to
 def _inline_ids(ids: IdsLike, distinct: bool = False) -> Optional[array]:
     """Host page ids that a launch carries in its kernel arguments (at most
     _native.INLINE_IDS, in a CPU tensor, list, tuple or array), as an int32
-    array; None for any others, which device_ids takes or refuses.  An upload
-    costs a pinned allocation and a copy ahead of each launch: pack and unpack
-    of 32 pages of 64 KiB, 32 layers, take 40 us without, 52 with, and
-    get_kv_cache and insert_kv_cache of 100 tokens 569 and 608."""
+    array; None for any others, which device_ids takes or refuses, and for a
+    pinned int32 tensor, which it uploads in stream order: earlier work on the
+    stream may still write the ids, and each replay of a graph reads them
+    again.  An upload costs a pinned allocation and a copy ahead of each
+    launch: pack and unpack of 32 pages of 64 KiB, 32 layers, take 40 us
+    without, 52 with, and get_kv_cache and insert_kv_cache of 100 tokens 569
+    and 608."""
     if isinstance(ids, torch.Tensor):
         if ids.device.type != "cpu" or not 0 < ids.numel() <= _native.INLINE_IDS:
+            return None
+        if ids.dtype is torch.int32 and ids.is_pinned():
             return None
         ids = ids.to(torch.int32).reshape(-1).tolist()
     elif not isinstance(ids, (list, tuple, array)) or not 0 < len(ids) <= _native.INLINE_IDS:

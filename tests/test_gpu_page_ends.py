@@ -108,3 +108,39 @@ def test_host_ids(gpu, page_bytes, n):
             assert torch.equal(host.view(torch.uint8), picked)
             st.unpack_from_host(host, dst_l, d_ids, k)
             assert torch.equal(dst.cpu(), want)
+
+
+def test_pinned_ids_are_read_in_stream_order(gpu):
+    """Pinned ids that earlier work on the stream writes, in a pack and a pack
+    to host, and in a graph whose replays follow the ids' new values."""
+    L, N, n, page_bytes = 3, 40, 7, 1024
+    gen = torch.Generator().manual_seed(11)
+    src, src_l = pool(L, N, page_bytes, gen, gpu)
+    ids = torch.zeros(n, dtype=torch.int32, pin_memory=True)
+    host = torch.empty((L, n) + tuple(src.shape[2:]), dtype=torch.uint8, pin_memory=True)
+    buf = torch.empty(host.shape, dtype=torch.uint8, device=gpu).view(torch.float8_e4m3fn)
+
+    def new_ids():
+        return torch.randperm(N, generator=gen)[:n].to(torch.int32)
+
+    with ops.Stager(L * n * page_bytes, 2) as st:
+        want = new_ids()
+        late = want.to(gpu)
+        torch.cuda.synchronize()
+        torch.cuda._sleep(20_000_000)
+        ids.copy_(late, non_blocking=True)
+        ops.pack(src_l, ids, buf)
+        st.pack_to_host(src_l, ids, host.view(torch.float8_e4m3fn), L)
+        torch.cuda.synchronize()
+    assert torch.equal(buf.view(torch.uint8).cpu(), src.cpu()[:, want.long()])
+    assert torch.equal(host, src.cpu()[:, want.long()])
+
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ops.pack(src_l, ids, buf)
+    for _ in range(4):
+        ids.copy_(new_ids())
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(buf.view(torch.uint8).cpu(), src.cpu()[:, ids.long()])
+        assert torch.equal(ops.pack(src_l, ids.tolist()).view(torch.uint8).cpu(), src.cpu()[:, ids.long()])

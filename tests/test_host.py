@@ -322,3 +322,23 @@ def test_inline_ids_take_what_uploads_take():
     with pytest.raises(ValueError, match="destination page 3 appears more than once"):
         ops._inline_ids([5, 3, 1, 3], distinct=True)
     assert ops._inline_ids([5, 3, 1, 3]).tolist() == [5, 3, 1, 3]
+
+
+def test_pinned_ids_are_left_to_the_stream():
+    """A pinned int32 tensor is uploaded in stream order, since earlier work on
+    the stream may still write it: its values are not read during the call."""
+    import torch
+
+    from paceserve_amd.kv_transfer import ops
+
+    class Pinned(torch.Tensor):
+        def is_pinned(self, device=None):
+            return True
+
+        def tolist(self):
+            raise AssertionError("read during the call")
+
+    ids = torch.tensor([3, 1, 2], dtype=torch.int32)
+    assert ops._inline_ids(ids.as_subclass(Pinned)) is None
+    assert ops._inline_ids(ids.as_subclass(Pinned), distinct=True) is None
+    assert ops._inline_ids(ids).tolist() == [3, 1, 2]
