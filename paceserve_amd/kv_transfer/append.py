@@ -31,25 +31,37 @@ def _i32(t: torch.Tensor, name: str, device: torch.device, index: int = -1) -> t
     return t.to(torch.int32).contiguous()
 
 
+# Private functions of torch: where a release has dropped one, get_seq_lens is
+# tensor arithmetic.
+_wrapped = getattr(getattr(torch._C, "_functorch", None), "is_functorch_wrapped_tensor", None)
+_dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", None)
+_function_modes = getattr(torch._C, "_len_torch_function_stack", None)
+
+
 def _plain_i32(t, dev) -> bool:
     """Whether t is an ordinary contiguous 1-D int32 tensor on dev: no subclass
     and not wrapped by vmap or another function transform."""
     return (type(t) is torch.Tensor and t.dtype is torch.int32 and t.dim() == 1 and t.device == dev
-            and t.is_contiguous() and not torch._C._functorch.is_functorch_wrapped_tensor(t))
+            and t.is_contiguous() and not _wrapped(t))
+
+
+def _unobserved() -> bool:
+    """Whether no mode and no tracer follows tensor operations, as far as torch
+    can tell."""
+    return (not torch.compiler.is_compiling() and None not in (_wrapped, _dispatch_modes, _function_modes)
+            and _dispatch_modes() == 0 and _function_modes() == 0 and not torch.jit.is_tracing())
 
 
 def _one_launch(kv_indptr, kv_last_page_len, page_size) -> bool:
     """Whether get_seq_lens is one launch of the library: plain int32 tensors
-    of matching lengths on the current device and no tracing.  Everything else
-    (CPU, other integer types, broadcasting, strides, tracers) is tensor
-    arithmetic."""
-    return (type(page_size) is int and 0 <= page_size < 2 ** 31 and type(kv_indptr) is torch.Tensor
-            and kv_indptr.is_cuda and _plain_i32(kv_indptr, kv_indptr.device)
+    of matching lengths on the current device, with nothing that follows tensor
+    operations.  Everything else (CPU, other integer types, broadcasting,
+    strides, modes, tracers) is tensor arithmetic."""
+    return (_unobserved() and type(page_size) is int and 0 <= page_size < 2 ** 31
+            and type(kv_indptr) is torch.Tensor and kv_indptr.is_cuda and _plain_i32(kv_indptr, kv_indptr.device)
             and _plain_i32(kv_last_page_len, kv_indptr.device)
             and kv_indptr.numel() == kv_last_page_len.numel() + 1 > 1
-            and kv_indptr.device.index == torch.cuda.current_device()
-            and torch._C._len_torch_dispatch_stack() == 0 and not torch.jit.is_tracing()
-            and not torch.compiler.is_compiling())
+            and kv_indptr.device.index == torch.cuda.current_device())
 
 
 def get_seq_lens(kv_indptr: torch.Tensor, kv_last_page_len: torch.Tensor, page_size: int) -> torch.Tensor:

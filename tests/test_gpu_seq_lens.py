@@ -41,3 +41,18 @@ def test_wraps_as_tensor_arithmetic_does(gpu):
     ip = torch.tensor([0, 2 ** 31 - 1, -2 ** 31, 5], dtype=torch.int32)
     last = torch.tensor([2 ** 31 - 1, 3, -7], dtype=torch.int32)
     assert torch.equal(ap.get_seq_lens(ip.to(gpu), last.to(gpu), 4097).cpu(), ap.get_seq_lens(ip, last, 4097))
+
+
+def test_a_function_mode_sees_the_arithmetic(gpu):
+    seen = []
+
+    class Mode(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    ip, last = (torch.tensor(x, dtype=torch.int32, device=gpu) for x in ([0, 3, 7], [2, 4]))
+    assert ap._one_launch(ip, last, 4)
+    with Mode():
+        got = ap.get_seq_lens(ip, last, 4)
+    assert torch.clamp in seen and got.tolist() == [10, 16]

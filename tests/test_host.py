@@ -342,3 +342,32 @@ def test_pinned_ids_are_left_to_the_stream():
     assert ops._inline_ids(ids.as_subclass(Pinned)) is None
     assert ops._inline_ids(ids.as_subclass(Pinned), distinct=True) is None
     assert ops._inline_ids(ids).tolist() == [3, 1, 2]
+
+
+def test_seq_lens_under_modes_and_without_private_functions(monkeypatch):
+    """get_seq_lens is tensor arithmetic where a mode would see it, and where a
+    torch release lacks one of the private functions that tell."""
+    import torch
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from paceserve_amd.kv_transfer import append as ap
+
+    class Seen(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatched(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert ap._unobserved()
+    for mode in (Seen, Dispatched):
+        with mode():
+            assert not ap._unobserved()
+    for name in ("_wrapped", "_dispatch_modes", "_function_modes"):
+        with monkeypatch.context() as m:
+            m.setattr(ap, name, None)
+            assert not ap._unobserved()
+            got = ap.get_seq_lens(torch.tensor([0, 3, 3]), torch.tensor([2, 0]), 4)
+            assert got.tolist() == [10, 0]
