@@ -350,7 +350,9 @@ int pace_kv_roundtrip(pace_kv_stager* stager,
  * bytes apart (device).  batch_indices, positions (nnz), kv_indptr
  * (batch_size + 1) and kv_indices (num_indices) are device int32 arrays.
  * A token whose request, page slot (outside its request's pages) or page id
- * is out of range is skipped and counted in err_count.
+ * is out of range is skipped and counted in err_count.  A call takes fewer than
+ * 2^24 tokens, one whose row is longer than 16 KiB counting once per 16 KiB of
+ * it (else PACE_KV_ERANGE).
  *
  * Replaces flashinfer.append_paged_kv_cache as called in
  * paceserve/model_executor/attention/flashinfer_attention_wrapper.py:245-255.
@@ -372,7 +374,7 @@ int pace_kv_append(const void* keys, const void* values, int64_t token_stride_by
  * append_indptr, kv_indptr (batch_size + 1 entries), kv_last_page_len
  * (batch_size) and kv_indices are device int32 arrays.  A token outside
  * every request, or whose slot or page is out of range, is skipped and
- * counted in err_count.
+ * counted in err_count.  The limit on nnz is the same.
  *
  * Replaces the three calls the reference makes for each layer
  * (paceserve/model_executor/attention/flashinfer_attention_wrapper.py:

@@ -345,11 +345,11 @@ int launch_append(AppendParams& p, int64_t nnz, int batch_size, int64_t num_page
     return fail(PACE_KV_EINVAL, "append: keys, values and cache must be 16-byte aligned");
   if (num_pages > INT32_MAX) return fail(PACE_KV_ERANGE, "append: too many pages");
   const int64_t row_vecs = row_bytes / kVecBytes;
-  // The most one call takes: 2^24 rows per side, a row longer than 16 KiB
-  // counting once per 16 KiB.
+  // The most one call takes, whatever its launches could: fewer than 2^24 rows
+  // per side, a row longer than 16 KiB counting once per 16 KiB.
   const int64_t pieces = (row_bytes + (16 << 10) - 1) / (16 << 10);
   if (nnz > INT32_MAX || nnz * 2 * pieces >= (int64_t(1) << 25))
-    return fail(PACE_KV_ERANGE, "append: too many tokens for one launch (%lld)", (long long)nnz);
+    return fail(PACE_KV_ERANGE, "append: too many tokens for one call (%lld)", (long long)nnz);
   p.token_stride = token_stride_bytes;
   p.num_indices = num_indices;
   p.row_bytes = row_bytes;

@@ -60,3 +60,38 @@ def test_batches_past_the_limit_are_refused_on_the_host(nnz, row_bytes):
     rc = lib.pace_kv_append(0x1000, 0x1000, row_bytes, nnz, 0x1000, 0x1000, 4, 0x1000, 8, 0x1000, 8, 0x1000, 16,
                             row_bytes, None, None)
     assert rc == _native.PACE_KV_ERANGE and b"too many tokens" in lib.pace_kv_last_error()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("row_bytes", [8192, 8208])    # whole KiB, and rows end to end
+def test_more_rows_than_one_launch_takes(gpu, row_bytes):
+    """A launch takes 2^25 waves; the tokens around the split land in their
+    pages, and all others, of a request without pages, are counted."""
+    first_launch = 2 ** 25 // -(-row_bytes // 1024)
+    nnz, n, P = first_launch + 70, 170, 16
+    print(f"append {nnz} rows of {row_bytes} bytes", flush=True)
+    whole = torch.empty((nnz + 1, 1, row_bytes), dtype=torch.uint8, device=gpu)    # values: one row on from the keys
+    tail = torch.randint(0, 120, (n + 1, 1, row_bytes), dtype=torch.uint8)
+    whole[-n - 1:] = tail.to(gpu)
+    f8 = whole.view(torch.float8_e4m3fn)
+    pages = -(-n // P)
+    NP = pages + 2
+    table = np.random.default_rng(1).permutation(NP)[:pages]
+    args = (i32(table, gpu), i32([0, 0, pages], gpu), i32([0, n - (pages - 1) * P], gpu))
+    want = torch.full((NP, 2, P, 1, row_bytes), 121, dtype=torch.uint8)
+    at, slot = torch.from_numpy(table)[torch.arange(n) // P], torch.arange(n) % P
+    want[at, 0, slot], want[at, 1, slot] = tail[:-1], tail[1:]
+    for form in ("two calls", "fused"):
+        cache = torch.full(want.shape, 121, dtype=torch.uint8, device=gpu)
+        err = torch.zeros(1, dtype=torch.int32, device=gpu)
+        got = cache.view(torch.float8_e4m3fn)
+        if form == "fused":
+            ap.append_paged_kv_cache_indptr(f8[:-1], f8[1:], i32([0, nnz - n, nnz], gpu), got, *args, err=err)
+        else:
+            bi = torch.full((nnz,), -1, dtype=torch.int32, device=gpu)
+            bi[-n:] = 1
+            pos = torch.zeros(nnz, dtype=torch.int32, device=gpu)
+            pos[-n:] = torch.arange(n, dtype=torch.int32, device=gpu)
+            ap.append_paged_kv_cache(f8[:-1], f8[1:], bi, pos, got, *args, err=err)
+        assert torch.equal(cache.cpu(), want), form
+        assert int(err.item()) == nnz - n, form
