@@ -244,3 +244,25 @@ def test_missing_page_ids_leave_everything_as_it_was(gpu, call):
         assert getattr(lib, "pace_kv_" + call)(st._handle, *args, None, stream) == _native.PACE_KV_EINVAL
         torch.cuda.synchronize()
     assert torch.equal(src.cpu(), before) and bool((host == 121).all())
+
+
+def test_more_vectors_than_one_launch_takes(gpu):
+    """A launch takes 2^31 vectors: three layers of 2^30 go in two.  Two pages
+    of each layer are copied, the rest of the 16384 are out of range."""
+    layers, n, page_bytes = 3, 1 << 14, 1 << 20
+    gen = torch.Generator().manual_seed(9)
+    src, src_l = pool(layers, 2, page_bytes, gen, gpu)
+    host = ops.HostPagePool(layers, 2, tuple(src.shape[2:]), torch.float8_e4m3fn)
+    d_ids, h_ids = (torch.full((n,), -1, dtype=torch.int32) for _ in range(2))
+    d_ids[0], d_ids[-1], h_ids[0], h_ids[-1] = 1, 0, 0, 1
+    d_ids, h_ids = d_ids.to(gpu), h_ids.to(gpu)
+    err = torch.zeros(1, dtype=torch.int32, device=gpu)
+    ops.swap_out(src_l, d_ids, host, h_ids, err=err)
+    torch.cuda.synchronize()
+    assert torch.equal(torch.stack([t.view(torch.uint8) for t in host.layers]), src.cpu().flip(1))
+    assert int(err.item()) == layers * (n - 2)
+    before = src.cpu()
+    src.zero_()
+    ops.swap_in(host, h_ids, src_l, d_ids, err=err)
+    assert torch.equal(src.cpu(), before)
+    assert int(err.item()) == 2 * layers * (n - 2)
