@@ -35,6 +35,7 @@ from __future__ import annotations
 import argparse
 import json
 import os
+import re
 import statistics
 import sys
 import time
@@ -239,21 +240,38 @@ def run_device(args, w, dev, src, dst, plan, s_ids, d_ids):
     return res
 
 
+# The enumerators of the page copy's template arguments, in order.
+SHAPES = ("kPow2", "kRows", "kSpanFlat", "kLaneFlat")
+KINDS = ("kStream", "kPack", "kTee")
+
+
+def copy_shape(page_bytes: int, both_indexed: bool) -> str:
+    """How a launch splits its pages over waves: the rule of enum Shape in
+    csrc/kv_copy.hip."""
+    if page_bytes % 1024 == 0:
+        rows = page_bytes // 1024
+        return "kPow2" if rows & (rows - 1) == 0 else "kRows"
+    return "kSpanFlat" if both_indexed and page_bytes >= 512 else "kLaneFlat"
+
+
 def copy_kernel_names(mode: str, page_bytes: int) -> str:
     """The page_copy_kernel instances a step launches (template arguments
-    GUARD = page not a multiple of 1 KiB rows, PACK = the pack's cacheable
-    write-through stores rather than streaming ones, POW2 = a power-of-two
-    number of rows per page)."""
-    guard = "true" if page_bytes % 1024 else "false"
-    rows = -(-page_bytes // 1024)
-    pow2 = "true" if rows & (rows - 1) == 0 else "false"
-
-    def k(pack: str) -> str:
-        return f"page_copy_kernel<{guard}, {pack}, {pow2}>"
-
+    Shape, Kind)."""
     if mode == "fused":
-        return f"{k('false')} (move, streaming write-through stores)"
-    return f"{k('true')} (pack, write-through stores) and {k('false')} (unpack, streaming write-through stores)"
+        return f"page_copy_kernel<{copy_shape(page_bytes, True)}, kStream> (move, streaming write-through stores)"
+    shape = copy_shape(page_bytes, False)
+    return (f"page_copy_kernel<{shape}, kPack> (pack, write-through stores) and "
+            f"page_copy_kernel<{shape}, kStream> (unpack, streaming write-through stores)")
+
+
+def short_kernel_name(name: str) -> str:
+    """A profiler's name of one of the library's kernels without its namespace
+    and arguments, its enumerators by name."""
+    def enumerator(m):
+        return {"Shape": SHAPES, "Kind": KINDS}[m[1]][int(m[2])]
+
+    name = re.sub(r"\((?:pace_kv::)?\(anonymous namespace\)::(Shape|Kind)\)(\d)", enumerator, name)
+    return name.split("(anonymous namespace)::", 1)[-1].split("(")[0]
 
 
 def run_ceiling(w, dev, src, dst, n: int, reps: int = 10) -> dict:
@@ -1104,8 +1122,7 @@ def summarize_pmc(fetch_csv: str, write_csv: str, workload: str) -> dict:
     out = {"workload": workload, "kernel": KERNEL_TAG, "fetch_csv": fetch_csv, "write_csv": write_csv}
     for name, path, counter in (("fetch", fetch_csv, "FETCH_SIZE"), ("write", write_csv, "WRITE_SIZE")):
         by = _per_dispatch(path, counter)
-        names = sorted({k.replace("void pace_kv::(anonymous namespace)::", "").split("(")[0]
-                        for k in by if "page_copy_kernel" in k})
+        names = sorted({short_kernel_name(k) for k in by if "page_copy_kernel" in k})
         if names:
             out["kernel"] = " and ".join(names)
         ours = [v for k, vals in by.items() if "page_copy_kernel" in k for v in vals]
@@ -1146,14 +1163,14 @@ def requests_per_launch(rdreq_csv: str, wrreq_csv: str) -> dict:
 def timed_dispatches(trace_csv: str, bench: dict):
     """The page-copy dispatches of the timed steps in a rocprofv3 kernel
     trace of one bench.py run.  The headline's launches are the page-copy
-    dispatches whose grid covers its batch (64 threads per 1 KiB row of each
-    of its pages; the staging legs that run earlier and the other workloads
+    dispatches whose grid covers its batch (64 threads per 1 KiB of its pages
+    end to end; the staging legs that run earlier and the other workloads
     that run later have other batches); in dispatch order they are the W
     warm-up steps, then the K timed steps, then the launch-timing pass and
     the copy ceiling.  Returns (durations ns, span ns) of the timed ones."""
     cfg = bench["config"]
     page_bytes = cfg["payload_bytes"] // (cfg["layers"] * cfg["pages"])
-    grid_x = -(-page_bytes // 1024) * cfg["pages"] * 64
+    grid_x = -(-page_bytes * cfg["pages"] // 1024) * 64
     rows = [r for r in _rows(trace_csv) if "page_copy_kernel" in r["Kernel_Name"]
             and int(r.get("Grid_Size_X", grid_x)) == grid_x]
     rows.sort(key=lambda r: int(r["Dispatch_Id"]))
@@ -1183,7 +1200,7 @@ def summarize_stats(stats_csv: str, bench_json: str, command: str, trace_csv: st
     for r in ours + others[:4]:
         name = r["Name"]
         if "pace_kv::" in name:
-            short = name.split("(anonymous namespace)::", 1)[-1].split("(")[0]
+            short = short_kernel_name(name)
         else:
             short = "torch normal_ (pool fill)" if "distribution" in name else name[:48]
         out.append(f"| {short} | {r['Calls']} | {float(r['AverageNs']):.0f} | {r['MinNs']} | {r['MaxNs']} | "
@@ -1216,44 +1233,35 @@ def summarize_stats(stats_csv: str, bench_json: str, command: str, trace_csv: st
 def summarize_promote(trace_csv: str, bench_json: str, command: str) -> str:
     """Markdown summary of the promote kernels in a rocprofv3 kernel trace of
     one bench.py run.  pace_kv_promote carries a 4096-token request's page ids
-    in the kernel arguments, so its launches are the run's only
-    page_copy_inline_kernel dispatches: a pack (source ids inline) and an
-    unpack (destination ids inline) per buffer-mode promote, one move (both
-    inline) per fused promote."""
+    in the kernel arguments, so its launches are the run's
+    page_copy_inline_kernel dispatches with ids inline on both sides: one that
+    also fills the buffer per buffer-mode promote, one move per fused promote."""
     bench = _json(bench_json)
     pr = bench["promote_4k"]
-    kinds = {"true, false>": "pack (source ids inline)", "false, true>": "unpack (destination ids inline)",
-             "true, true>": "move (both inline)"}
-    durs = {}
+    kinds = {"kTee, true, true>": "through the buffer", "kStream, true, true>": "move"}
+    durs = {k: [] for k in kinds.values()}
     for r in _rows(trace_csv):
-        name = r["Kernel_Name"]
-        if "page_copy_inline_kernel" not in name:
-            continue
-        tmpl = name.split("page_copy_inline_kernel<", 1)[1].split(">", 1)[0] + ">"
-        kind = next((v for k, v in kinds.items() if tmpl.endswith(k)), tmpl)
-        durs.setdefault(kind, []).append((int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3)
+        name = short_kernel_name(r["Kernel_Name"])
+        kind = next((v for k, v in kinds.items() if name.endswith(k)), None)
+        if kind and name.startswith("page_copy_inline_kernel<"):
+            durs[kind].append((int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3)
     payload = pr["payload_bytes"]
+    moved = {"through the buffer": 3, "move": 2}
     out = ["# promote kernels on llama3-8b-4096tok-bf16 - kernel trace", "",
            "One 4096-token request (256 pages), Llama-3-8B KV, bf16, 2048-page pools; "
            f"payload {payload} B. `pace_kv_promote` plans, allocates and launches in one call.", "",
            "Command (repo root, one MI355X):", "", "```", "export TMPDIR=/tmp", command, "```", "",
-           "| kernel | launches | mean us | p50 us | min us | max us | GB/s (2 x payload / p50) |",
+           "| kernel | launches | mean us | p50 us | min us | max us | bytes moved / p50, GB/s |",
            "|---|---|---|---|---|---|---|"]
-    for kind in ("pack (source ids inline)", "unpack (destination ids inline)", "move (both inline)"):
-        d = sorted(durs.get(kind, []))
-        if not d:
-            continue
-        p50 = statistics.median(d)
-        out.append(f"| {kind} | {len(d)} | {statistics.mean(d):.1f} | {p50:.1f} | {d[0]:.1f} | {d[-1]:.1f} | "
-                   f"{2 * payload / (p50 * 1e-6) / 1e9:.0f} |")
-    pk = statistics.median(durs.get("pack (source ids inline)", [0.0]))
-    up = statistics.median(durs.get("unpack (destination ids inline)", [0.0]))
-    mv = statistics.median(durs.get("move (both inline)", [0.0]))
-    out += ["", f"bench.py in the same run: promote p50 {pr['buffer_native']['p50_us']} us (pack + unpack, "
-            f"{pr['buffer_native']['runs']} runs), of which {pk + up:.1f} us are the two kernels "
-            f"({4 * payload / ((pk + up) * 1e-6) / 1e9:.0f} GB/s of pack+unpack bytes); fused promote p50 "
-            f"{pr['fused_native']['p50_us']} us, of which {mv:.1f} us is the move kernel. The rest is host "
-            f"time (Python, planning, launch) and completion."]
+    p50 = {k: statistics.median(d) if d else 0.0 for k, d in durs.items()}
+    for kind, d in durs.items():
+        if d:
+            out.append(f"| {kind} ({moved[kind]} x payload) | {len(d)} | {statistics.mean(d):.1f} | {p50[kind]:.1f} | "
+                       f"{min(d):.1f} | {max(d):.1f} | {moved[kind] * payload / (p50[kind] * 1e-6) / 1e9:.0f} |")
+    out += ["", f"bench.py in the same run: promote p50 {pr['buffer_native']['p50_us']} us (through the buffer, "
+            f"{pr['buffer_native']['runs']} runs), of which {p50['through the buffer']:.1f} us is the kernel; fused "
+            f"promote p50 {pr['fused_native']['p50_us']} us, of which {p50['move']:.1f} us is the kernel. The rest is "
+            f"host time (Python, planning, launch) and completion."]
     if pr.get("c_caller"):
         c = pr["c_caller"]
         out += ["", f"The same call from C (tests/c_abi/pace_kv_promote_latency, in the same run): buffer p50 "
@@ -1329,7 +1337,7 @@ def summarize_kernel_pmc(kernel: str, command: str, csvs: list) -> str:
             name = r["Kernel_Name"]
             if not any(k in name for k in wanted):
                 continue
-            short = name.split("(anonymous namespace)::", 1)[-1].split("(")[0]
+            short = short_kernel_name(name)
             if short.startswith("__amd_rocclr"):
                 short = short.split("<")[0]
             key = (short, int(r.get("Grid_Size", 0) or 0))

@@ -3,6 +3,7 @@ kernel naming, PMC byte scaling, the timed-dispatch selection from a kernel
 trace, and the one-GPU contract."""
 import csv
 import json
+import re
 import subprocess
 import sys
 from pathlib import Path
@@ -12,8 +13,10 @@ import pytest
 import bench
 
 ROOT = Path(__file__).resolve().parent.parent
-COPY = "void pace_kv::(anonymous namespace)::page_copy_kernel<false, false, true>(pace_kv::(anonymous namespace)::CopyParams)"
-COPY_T = COPY.replace("<false, false, true>", "<false, true, true>")
+# The names as rocprofv3 prints them
+NS = "pace_kv::(anonymous namespace)::"
+COPY = f"void {NS}page_copy_kernel<({NS}Shape)0, ({NS}Kind)0>({NS}CopyParams)"
+COPY_T = COPY.replace("Kind)0", "Kind)1")
 
 
 def write_csv(path, rows):
@@ -26,11 +29,29 @@ def write_csv(path, rows):
 
 def test_copy_kernel_names_follow_the_store_policy():
     names = bench.copy_kernel_names("buffer", 65536)
-    assert "page_copy_kernel<false, true, true> (pack, write-through stores)" in names
-    assert "page_copy_kernel<false, false, true> (unpack" in names
-    # 96 B: one partial row (a power of two); 3 KiB: three rows (not)
-    assert bench.copy_kernel_names("fused", 96).startswith("page_copy_kernel<true, false, true> (move")
-    assert bench.copy_kernel_names("fused", 3072).startswith("page_copy_kernel<false, false, false>")
+    assert "page_copy_kernel<kPow2, kPack> (pack, write-through stores)" in names
+    assert "page_copy_kernel<kPow2, kStream> (unpack" in names
+    # 96 and 1040 B: end to end, by lanes' or the wave's ids; 3 KiB: three rows
+    assert bench.copy_kernel_names("fused", 96).startswith("page_copy_kernel<kLaneFlat, kStream> (move")
+    assert bench.copy_kernel_names("fused", 1040).startswith("page_copy_kernel<kSpanFlat, kStream>")
+    assert bench.copy_kernel_names("buffer", 1040).startswith("page_copy_kernel<kLaneFlat, kPack>")
+    assert bench.copy_kernel_names("fused", 3072).startswith("page_copy_kernel<kRows, kStream>")
+
+
+def test_kernel_names_are_the_library_s():
+    """Every instance that copy_kernel_names names is a kernel of the built
+    library, and the enumerators are the source's, in its order."""
+    src = (ROOT / "paceserve_amd" / "csrc" / "kv_copy.hip").read_text()
+    enums = {name: re.findall(r"(k\w+) = (\d)", body) for name, body in re.findall(r"enum (\w+) \{([^}]*)\}", src)}
+    assert enums["Shape"] == [(n, str(i)) for i, n in enumerate(bench.SHAPES)]
+    assert enums["Kind"] == [(n, str(i)) for i, n in enumerate(bench.KINDS)]
+    assert bench.short_kernel_name(COPY) == "page_copy_kernel<kPow2, kStream>"
+    lib = (ROOT / "paceserve_amd" / "libpace_kv.so").read_bytes()
+    for mode in ("buffer", "fused"):
+        for page_bytes in (96, 512, 1040, 3072, 65536):
+            for shape, kind in re.findall(r"page_copy_kernel<(\w+), (\w+)>", bench.copy_kernel_names(mode, page_bytes)):
+                mangled = f"page_copy_kernelILNS0_5ShapeE{bench.SHAPES.index(shape)}ELNS0_4KindE{bench.KINDS.index(kind)}E"
+                assert mangled.encode() in lib, (mode, page_bytes, shape, kind)
 
 
 def test_summarize_pmc_scales_counters_by_the_calibration_copy(tmp_path):
@@ -52,7 +73,7 @@ def test_summarize_pmc_scales_counters_by_the_calibration_copy(tmp_path):
     assert d["write_bytes_per_launch"] == 2000 * 1024
     assert d["traffic_bytes_per_launch"] == 4000 * 1024
     assert d["fetch_dispatches"] == 2
-    assert d["kernel"] == "page_copy_kernel<false, false, true> and page_copy_kernel<false, true, true>"
+    assert d["kernel"] == "page_copy_kernel<kPow2, kPack> and page_copy_kernel<kPow2, kStream>"
 
 
 def test_summarize_pmc_needs_both_kinds_of_dispatch(tmp_path):
@@ -67,7 +88,7 @@ def test_pmc_markdown_states_algorithmic_bytes_per_layer_chunk(tmp_path):
 
     w = workloads.get("llama3-70b-256req-bf16")
     alg = 2 * 8 * w.n_pages * w.shape.page_bytes          # one launch = one 8-layer chunk
-    t = {"workload": "llama3-70b-256req-bf16", "kernel": "page_copy_kernel<false, false, true>",
+    t = {"workload": "llama3-70b-256req-bf16", "kernel": "page_copy_kernel<kPow2, kStream>",
          "fetch_kib_per_dispatch_raw": 1.0, "fetch_calibration_kib_raw": 2.0, "fetch_scale": 2.0,
          "fetch_bytes_per_launch": alg // 2, "fetch_dispatches": 3, "write_kib_per_dispatch_raw": 1.0,
          "write_calibration_kib_raw": 1.0, "write_scale": 1.0, "write_bytes_per_launch": alg // 2,
@@ -113,12 +134,12 @@ def test_more_than_one_gpu_is_refused():
 
 
 def test_summarize_promote_splits_the_inline_kernels(tmp_path):
-    inline = "void pace_kv::(anonymous namespace)::page_copy_inline_kernel<false, {}, true, {}, {}>(x)"
+    inline = f"void {NS}page_copy_inline_kernel<({NS}Shape)0, ({NS}Kind){{}}, {{}}, {{}}>({NS}CopyParamsInline)"
     rows, t = [], 0
-    for i, (pack, s_in, d_in, dur) in enumerate([("true", "true", "false", 150000),
-                                                  ("false", "false", "true", 152000)] * 3
-                                                 + [("false", "true", "true", 165000)] * 2):
-        rows.append({"Dispatch_Id": i + 1, "Kernel_Name": inline.format(pack, s_in, d_in),
+    # packs and unpacks with host ids run beside the promotions
+    for i, (kind, s_in, d_in, dur) in enumerate([(2, "true", "true", 258000)] * 3 + [(1, "true", "false", 7000),
+                                                 (0, "false", "true", 9000)] + [(0, "true", "true", 165000)] * 2):
+        rows.append({"Dispatch_Id": i + 1, "Kernel_Name": inline.format(kind, s_in, d_in),
                      "Start_Timestamp": t, "End_Timestamp": t + dur})
         t += dur + 1000
     rows.append({"Dispatch_Id": 99, "Kernel_Name": COPY, "Start_Timestamp": 0, "End_Timestamp": 7})
@@ -128,14 +149,13 @@ def test_summarize_promote_splits_the_inline_kernels(tmp_path):
     bj = tmp_path / "b.json"
     bj.write_text(json.dumps(b))
     md = bench.summarize_promote(path, str(bj), "CMD")
-    assert "| pack (source ids inline) | 3 | 150.0 | 150.0 |" in md
-    assert "| unpack (destination ids inline) | 3 | 152.0 | 152.0 |" in md
-    assert "| move (both inline) | 2 | 165.0 | 165.0 |" in md
-    assert "of which 302.0 us are the two kernels" in md and "of which 165.0 us is the move kernel" in md
+    assert "| through the buffer (3 x payload) | 3 | 258.0 | 258.0 |" in md
+    assert "| move (2 x payload) | 2 | 165.0 | 165.0 |" in md
+    assert "of which 258.0 us is the kernel" in md and "of which 165.0 us is the kernel" in md
 
 
 def test_summarize_kernel_pmc_groups_by_kernel_and_grid(tmp_path):
-    app = "void pace_kv::(anonymous namespace)::append_kernel<2, false, false, true>(pace_kv::(anonymous namespace)::AppendParams)"
+    app = f"void {NS}append_kernel<true, true, false>({NS}AppendParams)"
     rows = []
     for i, (grid, val) in enumerate([(2097152, 100.0), (2097152, 300.0), (32768, 7.0)]):
         rows.append({"Dispatch_Id": i + 1, "Kernel_Name": app, "Grid_Size": grid, "Counter_Name": "FETCH_SIZE",
@@ -147,8 +167,8 @@ def test_summarize_kernel_pmc_groups_by_kernel_and_grid(tmp_path):
                                        for r in rows])
     md = bench.summarize_kernel_pmc("append_kernel", "CMD1\nCMD2", [a, b])
     assert "CMD1\nCMD2" in md
-    assert "| append_kernel<2, false, false, true> | 32768 | 1 | 7 | 14 |" in md
-    assert "| append_kernel<2, false, false, true> | 2097152 | 2 | 200 | 400 |" in md
+    assert "| append_kernel<true, true, false> | 32768 | 1 | 7 | 14 |" in md
+    assert "| append_kernel<true, true, false> | 2097152 | 2 | 200 | 400 |" in md
     assert "other" not in md
 
 
