@@ -251,7 +251,7 @@ def copy_shape(page_bytes: int, both_indexed: bool) -> str:
     if page_bytes % 1024 == 0:
         rows = page_bytes // 1024
         return "kPow2" if rows & (rows - 1) == 0 else "kRows"
-    return "kSpanFlat" if both_indexed and page_bytes >= 512 else "kLaneFlat"
+    return "kSpanFlat" if both_indexed and page_bytes >= 336 else "kLaneFlat"
 
 
 def copy_kernel_names(mode: str, page_bytes: int) -> str:

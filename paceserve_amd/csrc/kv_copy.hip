@@ -61,11 +61,11 @@ struct CopyParams {
   uint32_t src_pool_pages;
   uint32_t dst_pool_pages;
   uint32_t page_vecs;      // page_bytes / 16
+  uint32_t n_pages;        // of this launch, per layer
+  FastDiv by_page;         // pages end to end: division by page_vecs
+  uint32_t total_vecs;     // n_pages * page_vecs
   uint32_t rows_per_page;  // page_bytes / kRowBytes (pages of whole rows)
   uint32_t rows_log2;      // log2(rows_per_page) when that is a power of two
-  FastDiv by_page;         // pages end to end: division by page_vecs
-  uint32_t n_pages;        // of this launch, per layer
-  uint32_t total_vecs;     // n_pages * page_vecs
   char* tee;               // Kind::kTee: page j of layer l also goes to tee + l * tee_stride + j * page_bytes
   int64_t tee_stride;
 };
@@ -82,20 +82,24 @@ enum Kind { kStream = 0, kPack = 1, kTee = 2 };
 // and the start of the next: each lane loads its own page's ids (kLaneFlat), or
 // the wave loads the at most kSpan ids per side that its lanes choose from by
 // scalar loads (kSpanFlat, ids on both sides and pages of at least kSpanVecs
-// vectors).
+// vectors: 336 bytes).
 // Measured on MI355X, 32 layers, 150 MiB, against waves that end with a page:
 //   move    160 B 210 -> 103 us, 256 B 132 -> 52, 512 B 67.4 -> 50.3, 1280 B
 //           57 -> 50, 1536 B 53.7 -> 49.8, the same from 2560 B on
 //   pack    160 B 210 -> 60, 512 B 67 -> 46, 1280 B 54.5 -> 46.3, 1536 B and
 //           more the same or up to 2% faster
 //   unpack  160 B 210 -> 85, 512 B 67.5 -> 48.9, 1280 B 56.4 -> 48.8
-// and on 8 MiB in a graph 512 B 5.3 -> 4.0 us; launches of 0.5 to 2 MiB, about
-// 2.1 us, are up to 0.1 us faster or slower (a move of 0.5 MiB 0.15 slower).
+// and on 6 MiB in a graph, 512 B: move 4.3 -> 3.2 us, pack 4.3 -> 3.4, unpack
+// 4.3 -> 3.2.  Below 2.5 MiB, where a launch takes 1.9 to 2.6 us: moves from 10%
+// faster to 4% slower (the same to 512 KiB), unpacks from 15% faster to 5%
+// slower, packs from 10% faster (0.5 to 1 MiB) to 0.25 us or 12% slower: 1.25 to
+// 2 MiB of pages of 640 bytes and more, whose time steps up past 1024 waves
+// where waves that end with a page step past 2048.
 // A move by lanes' own ids is 3-4% slower than by scalar ids (its id loads go
 // ahead of the page's in one chain); a pack or unpack by scalar ids is 4-8%
 // slower at 150 MiB (the contiguous side needs no id).
 enum Shape { kPow2 = 0, kRows = 1, kSpanFlat = 2, kLaneFlat = 3 };
-constexpr int kSpan = 3;
+constexpr int kSpan = 4;
 constexpr int kSpanVecs = kThreads / (kSpan - 1);
 
 // Page ids carried in the kernel arguments (small promotions): no device id
@@ -105,17 +109,6 @@ struct CopyParamsInline {
   int32_t src_ids[PACE_KV_INLINE_IDS];
   int32_t dst_ids[PACE_KV_INLINE_IDS];
 };
-
-// The page id of position j; in kSpanFlat j lies `nth` < kSpan pages after j0,
-// the wave's first, and the ids of all of them are loaded by scalar loads.
-template <Shape SHAPE>
-__device__ __forceinline__ uint32_t page_of(const CopyParams& p, const int32_t* ids, uint32_t j, uint32_t j0,
-                                            uint32_t nth) {
-  if (SHAPE != kSpanFlat) return static_cast<uint32_t>(ids[j]);
-  const uint32_t last = p.n_pages - 1;
-  const int32_t a = ids[j0], b = ids[min(j0 + 1, last)], c = ids[min(j0 + 2, last)];
-  return static_cast<uint32_t>(nth == 0 ? a : nth == 1 ? b : c);
-}
 
 // Stores carry the device-scope bit (sc1): an XCD's L2 is not coherent with
 // the other XCDs', so such a store writes through it to the memory side, and
@@ -177,31 +170,48 @@ __device__ __forceinline__ void copy_row(const CopyParams& p, const int32_t* sid
                                          const int32_t* dids) {
   const uint32_t x = blockIdx.x;
   const uint32_t layer = blockIdx.y;
-  uint32_t j, vec, j0 = 0, nth = 0;
-  if (SHAPE == kLaneFlat) {
+  uint32_t j, vec, sp, dp;
+  bool inside = true;
+  if (SHAPE == kSpanFlat) {
+    // The arguments are all loaded behind one wait, and then the ids behind
+    // another: left to itself the compiler loads each where it is first used,
+    // eight waits in a row, which small launches showed (a move of 256 KiB of
+    // 512-byte pages 2.06 us, now 1.88).  In kLaneFlat the same was up to 4%
+    // faster below 512 KiB and up to 10% slower at 1 MiB.
+    uint32_t g0 = x * kThreads;
+    if (KIND == kTee) asm("" : "+s"(g0) : "s"(p.tee), "s"(p.tee_stride));
+    asm("" : "+s"(g0) : "s"(p.src[layer]), "s"(p.dst[layer]), "s"(p.err), "s"(p.page_bytes), "s"(p.src_pool_pages),
+                        "s"(p.dst_pool_pages), "s"(p.page_vecs), "s"(p.by_page.mul), "s"(p.by_page.shift1),
+                        "s"(p.by_page.shift2), "s"(p.n_pages), "s"(p.total_vecs));
+    inside = g0 + threadIdx.x < p.total_vecs;
+    const uint32_t j0 = over(p.by_page, g0), last = p.n_pages - 1;
+    const uint32_t j1 = min(j0 + 1, last), j2 = min(j0 + 2, last), j3 = min(j0 + 3, last);
+    int32_t s0 = sids[j0], s1 = sids[j1], s2 = sids[j2], s3 = sids[j3];
+    int32_t d0 = dids[j0], d1 = dids[j1], d2 = dids[j2], d3 = dids[j3];
+    asm("" : "+s"(s0), "+s"(s1), "+s"(s2), "+s"(s3), "+s"(d0), "+s"(d1), "+s"(d2), "+s"(d3));
+    vec = g0 - j0 * p.page_vecs + threadIdx.x;
+    const bool past1 = vec >= p.page_vecs, past2 = vec >= 2 * p.page_vecs, past3 = vec >= 3 * p.page_vecs;
+    j = j0 + past1 + past2 + past3;
+    vec -= past3 ? 3 * p.page_vecs : past2 ? 2 * p.page_vecs : past1 ? p.page_vecs : 0;
+    sp = static_cast<uint32_t>(past3 ? s3 : past2 ? s2 : past1 ? s1 : s0);
+    dp = static_cast<uint32_t>(past3 ? d3 : past2 ? d2 : past1 ? d1 : d0);
+  } else if (SHAPE == kLaneFlat) {
     const uint32_t g = x * kThreads + threadIdx.x;
     if (g >= p.total_vecs) return;
     j = over(p.by_page, g);
     vec = g - j * p.page_vecs;
-  } else if (SHAPE == kSpanFlat) {
-    const uint32_t g0 = x * kThreads;
-    if (g0 + threadIdx.x >= p.total_vecs) return;
-    j0 = over(p.by_page, g0);
-    vec = g0 - j0 * p.page_vecs + threadIdx.x;
-    nth = (vec >= p.page_vecs ? 1 : 0) + (vec >= 2 * p.page_vecs ? 1 : 0);
-    j = j0 + nth;
-    vec -= nth * p.page_vecs;
   } else {
     j = SHAPE == kPow2 ? x >> p.rows_log2 : x / p.rows_per_page;
     const uint32_t row = SHAPE == kPow2 ? x & (p.rows_per_page - 1) : x - j * p.rows_per_page;
     vec = row * kThreads + threadIdx.x;
   }
+  if (!inside) return;
   if (SHAPE != kSpanFlat && sids == nullptr) {
     // Contiguous source (unpack): page j of the buffer is always in bounds,
     // so the load is issued before the destination id is known.
     const u32x4 v = __builtin_nontemporal_load(
         reinterpret_cast<const u32x4*>(p.src[layer] + static_cast<int64_t>(j) * p.page_bytes) + vec);
-    const uint32_t dp = dids ? static_cast<uint32_t>(dids[j]) : j;
+    dp = dids ? static_cast<uint32_t>(dids[j]) : j;
     if (dp >= p.dst_pool_pages) {
       if (vec == 0 && p.err != nullptr) atomicAdd(p.err, 1);
       return;
@@ -209,8 +219,10 @@ __device__ __forceinline__ void copy_row(const CopyParams& p, const int32_t* sid
     store_vec<KIND == kPack>(v, reinterpret_cast<u32x4*>(p.dst[layer] + static_cast<int64_t>(dp) * p.page_bytes) + vec);
     return;
   }
-  const uint32_t sp = page_of<SHAPE>(p, sids, j, j0, nth);
-  const uint32_t dp = SHAPE == kSpanFlat || dids ? page_of<SHAPE>(p, dids, j, j0, nth) : j;
+  if (SHAPE != kSpanFlat) {
+    sp = static_cast<uint32_t>(sids[j]);
+    dp = dids ? static_cast<uint32_t>(dids[j]) : j;
+  }
   if (KIND == kTee) {
     tee_row(p, j, layer, vec, sp, dp);
     return;

@@ -31,7 +31,8 @@ def test_copy_kernel_names_follow_the_store_policy():
     names = bench.copy_kernel_names("buffer", 65536)
     assert "page_copy_kernel<kPow2, kPack> (pack, write-through stores)" in names
     assert "page_copy_kernel<kPow2, kStream> (unpack" in names
-    # 96 and 1040 B: end to end, by lanes' or the wave's ids; 3 KiB: three rows
+    # 96, 352 and 1040 B: end to end, by lanes' or the wave's ids; 3 KiB: three rows
+    assert bench.copy_kernel_names("fused", 352).startswith("page_copy_kernel<kSpanFlat, kStream>")
     assert bench.copy_kernel_names("fused", 96).startswith("page_copy_kernel<kLaneFlat, kStream> (move")
     assert bench.copy_kernel_names("fused", 1040).startswith("page_copy_kernel<kSpanFlat, kStream>")
     assert bench.copy_kernel_names("buffer", 1040).startswith("page_copy_kernel<kLaneFlat, kPack>")

@@ -40,7 +40,7 @@ def expect(src, s_ids, dst, d_ids, k):
 
 @pytest.mark.parametrize("bad", [False, True])
 @pytest.mark.parametrize("k", [2, 5, 70])
-@pytest.mark.parametrize("page_bytes", [32, 992, 1024, 1056, 2048, 3072, 5120])
+@pytest.mark.parametrize("page_bytes", [32, 352, 992, 1024, 1056, 2048, 3072, 5120])
 def test_buffer_and_destination_match_pack_then_unpack(gpu, page_bytes, k, bad):
     L, N = (70, 11) if k == 70 else (5, 40)     # 70 layers: more than one launch
     gen = torch.Generator().manual_seed(page_bytes + k)

@@ -1,6 +1,6 @@
 """Pages that are no whole number of 1 KiB rows are copied end to end: pack,
 unpack, move and promotion of pages around the sizes where the split changes
-(32 vectors: 512 bytes) and where a wave holds one, two or many pages, with
+(21 vectors: 336 bytes) and where a wave holds one, two or many pages, with
 page counts that leave a last wave of one vector, part of it or all of it."""
 import pytest
 import torch
@@ -10,7 +10,7 @@ from paceserve_amd.kv_transfer import ops
 from paceserve_amd.kv_transfer.migrate import KVMigrator
 
 pytestmark = pytest.mark.gpu
-PAGE_BYTES = [32, 64, 480, 496, 512, 544, 1008, 1056, 1536, 3104]
+PAGE_BYTES = [32, 64, 320, 352, 480, 496, 512, 544, 1008, 1056, 1536, 3104]
 
 
 def pool(layers, pages, page_bytes, gen, dev):
