@@ -66,9 +66,10 @@ struct IdList {
 
 // Store flavour of a copy: both write through the L2 at device scope; kStream
 // also marks the stores nontemporal, while kPack (a pack into a transfer
-// buffer) leaves them cacheable, so that the unpack reading the rows next
-// finds them in the memory-side cache.
-enum class StorePolicy { kStream, kPack };
+// buffer that an unpack reads next) leaves them cacheable, so that the unpack
+// finds them in the memory-side cache.  kLink is kStream across the host link
+// (ids on both sides, in device memory), where short pages go one to a wave.
+enum class StorePolicy { kStream, kPack, kLink };
 
 // A second destination of a copy with ids on both sides: page j of layer l
 // also goes to base + l * layer_stride + j * page_bytes.

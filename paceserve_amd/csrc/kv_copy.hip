@@ -98,7 +98,12 @@ enum Kind { kStream = 0, kPack = 1, kTee = 2 };
 // A move by lanes' own ids is 3-4% slower than by scalar ids (its id loads go
 // ahead of the page's in one chain); a pack or unpack by scalar ids is 4-8%
 // slower at 150 MiB (the contiguous side needs no id).
-enum Shape { kPow2 = 0, kRows = 1, kSpanFlat = 2, kLaneFlat = 3 };
+// Across the host link what counts is the number of pieces in which pages
+// travel: pages of up to kLinkPageBytes go one to a wave (kOnePage).
+// Measured on MI355X, swaps of 8 MiB against waves end to end: 160 B out 167
+// against 176 us, in 250 against 304; 400 B 159 against 167 and 192 against 234.
+enum Shape { kPow2 = 0, kRows = 1, kSpanFlat = 2, kLaneFlat = 3, kOnePage = 4 };
+constexpr int kLinkPageBytes = 512;
 constexpr int kSpan = 4;
 constexpr int kSpanVecs = kThreads / (kSpan - 1);
 
@@ -200,6 +205,10 @@ __device__ __forceinline__ void copy_row(const CopyParams& p, const int32_t* sid
     if (g >= p.total_vecs) return;
     j = over(p.by_page, g);
     vec = g - j * p.page_vecs;
+  } else if (SHAPE == kOnePage) {
+    j = x;
+    vec = threadIdx.x;
+    if (vec >= p.page_vecs) return;
   } else {
     j = SHAPE == kPow2 ? x >> p.rows_log2 : x / p.rows_per_page;
     const uint32_t row = SHAPE == kPow2 ? x & (p.rows_per_page - 1) : x - j * p.rows_per_page;
@@ -291,6 +300,8 @@ const void* inline_kernel_of(Kind kind, InlineSides sides) {
 // traffic.  Each lane keeps UNROLL vectors in flight and loads the next round's
 // ids behind them.  Measured on MI355X at 14 and 56 MiB, by workgroups of 256:
 //   out, 16 vectors   4: 54.5 and 56.2 GB/s, 6 to 12 within 2% either way
+//                     (short pages 4: 16 MiB of 160 B 341 us, of 400 B 326;
+//                     8: 310 and 309)
 //   in, 8 vectors     8: 33, 16: 55.4 and 56.8, 24 to 64: 54 to 56.5;
 //                     16 vectors the same or slower
 // Beside host-to-device DMA copies 4 workgroups out keep 48.6 GB/s per
@@ -304,8 +315,7 @@ constexpr int kInGroups = 16, kInUnroll = 8;
 // against the page copy's one wave per row, 63 pages of 64 KiB, 32 layers: out
 // 2379 -> 2328 us, in 2412 -> 2326; 7 pages out 270 -> 264, in 290 -> 265; 500
 // pages of 8 KiB out 2362 -> 2307, in 2384 -> 2306; 777 of 1536 B out 689 -> 680,
-// in 696 -> 679; 1000 of 512 B 296 -> 298 and 299 -> 302, where the page copy's
-// end-to-end waves would take 306 and 312.
+// in 696 -> 679.  Short pages and small swaps are the page copy's (swap_copy).
 constexpr int kPagedOutGroups = 32;
 
 struct HostLegParams {
@@ -405,6 +415,7 @@ __global__ __launch_bounds__(kHostThreads) void host_leg_inline_kernel(const Hos
 
 const void* pick_kernel(Shape shape, Kind kind) {
   switch (shape) {
+    case kOnePage: return reinterpret_cast<const void*>(&page_copy_kernel<kOnePage, kStream>);
     case kPow2: return kernel_of<kPow2>(kind);
     case kRows: return kernel_of<kRows>(kind);
     case kSpanFlat:  // a move or a tee
@@ -504,8 +515,11 @@ int launch_page_copy(const Side& src, const Side& dst, int num_layers, int64_t n
   uint32_t rows_log2 = 0;
   while ((int64_t(1) << rows_log2) < rows_per_page) ++rows_log2;
   const bool whole_rows = page_bytes % kRowBytes == 0;
-  const bool span = page_bytes >= kSpanVecs * kVecBytes && src_indexed && dst_indexed && policy == StorePolicy::kStream;
+  const bool span = page_bytes >= kSpanVecs * kVecBytes && src_indexed && dst_indexed && policy != StorePolicy::kPack;
+  const bool one_page =
+      policy == StorePolicy::kLink && page_bytes <= kLinkPageBytes && !inline_ids && tee == nullptr;
   const Shape shape = whole_rows ? ((int64_t(1) << rows_log2) == rows_per_page ? kPow2 : kRows)
+                      : one_page ? kOnePage
                       : span     ? kSpanFlat
                                  : kLaneFlat;
 
@@ -538,7 +552,8 @@ int launch_page_copy(const Side& src, const Side& dst, int num_layers, int64_t n
         p.tee = tee->base + l0 * tee->layer_stride + j0 * page_bytes;
         p.tee_stride = tee->layer_stride;
       }
-      const int64_t groups = whole_rows ? rows_per_page * nj : (nj * p.page_vecs + kThreads - 1) / kThreads;
+      const int64_t groups =
+          whole_rows || one_page ? rows_per_page * nj : (nj * p.page_vecs + kThreads - 1) / kThreads;
       const dim3 grid(static_cast<uint32_t>(groups), static_cast<uint32_t>(nl));
       const Kind kind = tee != nullptr ? kTee : (policy == StorePolicy::kPack ? kPack : kStream);
       if (inline_ids) {
@@ -628,7 +643,9 @@ int launch_host_leg(const Side& pool, const Side& host, bool to_host, int num_la
     p.by_page = fast_div(p.page_vecs);
     p.by_count = fast_div(p.n_pages);
     const int64_t most = (int64_t(p.total_vecs) + kHostThreads - 1) / kHostThreads;
-    const int groups = !to_host ? kInGroups : paged ? kPagedOutGroups : kOutGroups;
+    const int groups = !to_host ? kInGroups
+                       : paged  ? kPagedOutGroups
+                                : (page_bytes < kLinkPageBytes ? 2 : 1) * kOutGroups;
     const dim3 grid(static_cast<uint32_t>(std::min<int64_t>(groups, most)));
     const void* fn;
     void* args[] = {&p};
@@ -802,6 +819,15 @@ int swap_copy(const void* const* src_layers, int64_t src_pool_pages, const int32
   PACE_KV_TRY(resolve_layers(src_layers, num_layers, src_pool_pages * page_bytes, src_host, s, what));
   PACE_KV_TRY(resolve_layers(dst_layers, num_layers, dst_pool_pages * page_bytes, dst_host, d, what));
   const Side src{s.data(), src_ids, src_pool_pages}, dst{d.data(), dst_ids, dst_pool_pages};
+  // The page copy is the faster one for short pages (see enum Shape; 512 B, 8
+  // MiB: out 154 against 156 us by the host leg, in 162 against 158) and for
+  // small swaps, where its waves carry one vector each: measured on MI355X,
+  // pages of 8 KiB, alone, 64 KiB in 19.5 against 20.5 us, 256 KiB out 29.0
+  // against 29.8 and in 30.8 against 30.6, 512 KiB in 37.1 against 35.6, 1 MiB
+  // out 43.7 against 44.4 and in 49.6 against 46.4, 2 MiB out 63.1 against 62.4.
+  const int64_t small_bytes = dst_host ? 2 << 20 : 512 << 10;
+  if (page_bytes < kLinkPageBytes + (dst_host ? 1 : 0) || n_pages <= (small_bytes - 1) / page_bytes / num_layers)
+    return launch_page_copy(src, dst, num_layers, n_pages, page_bytes, err_count, stream, StorePolicy::kLink);
   return launch_host_leg(dst_host ? src : dst, dst_host ? dst : src, dst_host, num_layers, n_pages, page_bytes,
                          err_count, stream);
 }

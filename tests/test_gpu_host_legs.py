@@ -80,10 +80,12 @@ def test_host_memory_that_no_kernel_copies(gpu):
 
 @pytest.mark.parametrize("bad", [False, True])
 @pytest.mark.parametrize("layers,n,page_bytes", [(1, 1, 1024), (3, 33, 1056), (70, 5, 2048), (2, 900, 1024), (5, 40, 65536),
-                                                 (3, 50, 1008)])
+                                                 (3, 50, 1008), (3, 40, 32), (5, 700, 496), (70, 9, 512),
+                                                 (2, 5000, 528), (70, 20, 2048), (1, 8, 65536), (4, 8, 65536)])
 def test_swaps(gpu, layers, n, page_bytes, bad):
     """Pages with ids on both sides; a page whose id is out of range on either
-    is skipped and counted once."""
+    is skipped and counted once.  Pages of up to 512 bytes, small swaps (512
+    KiB in, 2 MiB out) and the rest go by three kernels."""
     N, M = n + 5, n + 3
     gen = torch.Generator().manual_seed(n * page_bytes)
     src, src_l = pool(layers, N, page_bytes, gen, gpu)
