@@ -241,7 +241,7 @@ def run_device(args, w, dev, src, dst, plan, s_ids, d_ids):
 
 
 # The enumerators of the page copy's template arguments, in order.
-SHAPES = ("kPow2", "kRows", "kSpanFlat", "kLaneFlat")
+SHAPES = ("kPow2", "kRows", "kSpanFlat", "kLaneFlat", "kOnePage")
 KINDS = ("kStream", "kPack", "kTee")
 
 
