@@ -30,8 +30,8 @@
 //   2 KiB rows, about 8500 tokens             15.5 us, before 17.0
 //   2 KiB rows, 256 tokens of a decode step   2.4 us, before 2.9
 //   8 KiB rows, 8190 tokens                   46 us, before 50 (the other form)
-// Slower are launches of few tokens with rows that are not whole KiB, which
-// take 3 us: 2-3% at 270 tokens of 256 or 384 bytes.
+// Launches of up to 300 tokens with rows of less than a KiB, 2.1 to 2.3 us, are
+// up to 0.06 us slower than that.
 // Waves that end with a row (idle lanes, scalar indices) never measured
 // faster than rows end to end, not in decode either, and up to 40% slower at
 // 16384 tokens.  Every index is checked: a token whose request, page slot or
@@ -54,6 +54,8 @@ constexpr int64_t kMaxGroupsPerLaunch = int64_t(1) << 25;
 constexpr int64_t kCachedLoadBytes = int64_t(1) << 20;
 // Blocks of 64 append_indptr entries that one round of the search loads.
 constexpr int kSearchBlocks = 4;
+// Most entries that a wave of several requests hands round one by one.
+constexpr uint32_t kHandRound = 8;
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
@@ -168,11 +170,21 @@ __device__ __forceinline__ bool locate(const AppendParams& p, FirstRound f, uint
         if (!UNIFORM) hi += search_count(f.x, t1);
       }
       if (UNIFORM) hi = lo;
-      // A wave of several requests: the entries between its first and its
-      // last token's are loaded once more and counted for each token.  (Counting
-      // the entries still held instead measured the same or 1% slower.)
+      // A wave of several requests: the entries between its first and its last
+      // token's.  A few that the wave still holds are handed round, which spares
+      // a small launch a round of loads (MI355X, 256 tokens of 16 requests, rows
+      // of 160 B 2.56 -> 2.25 us; 1000 of 200, rows of 384 B 2.70 -> 2.40; the
+      // same to 2% from 4096 tokens on); else they are loaded once more and
+      // counted for each token.  (Counting all that are held for each token
+      // measured the same or 1% slower than that.)
       uint32_t count = lo;
-      for (uint32_t base = lo; base < hi; base += kThreads) {
+      const bool held = hi - lo <= kHandRound && p.batch_size <= kSearchBlocks * kThreads;
+      for (uint32_t e = lo; held && e < hi; ++e) {
+        const uint32_t block = e / kThreads;
+        const int32_t x = block == 0 ? f.x[0] : block == 1 ? f.x[1] : block == 2 ? f.x[2] : f.x[3];
+        if (__builtin_amdgcn_readlane(x, e % kThreads) <= t) ++count;
+      }
+      for (uint32_t base = lo; !held && base < hi; base += kThreads) {
         const uint32_t e = base + threadIdx.x;
         const int32_t x = e < hi ? p.append_indptr[e] : INT32_MAX;
         for (int32_t k = t0 + 1; k <= t1; ++k) {
