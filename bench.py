@@ -978,11 +978,11 @@ def run_promote(dev, steps=100, warmup=10, c_caller=True):
         log(f"promote 4096 tok {name}: p50 {out[name]['p50_us']} us ({out[name]['gbs']} GB/s)")
     out["payload_bytes"] = w.payload_bytes
     out["c_caller"] = run_promote_c(w) if c_caller else None
-    # the metric's promote latency: allocation + remap + id upload + pack +
-    # unpack, through the single library call
+    # the metric's promote latency: allocation + remap + ids + the movement
+    # through the transfer buffer, in the single library call
     out["p50_us"] = out["buffer_native"]["p50_us"]
     out["p50_mode"] = ("buffer_native (KVMigrator.promote of list block tables -> pace_kv_promote: plan, ids, "
-                       "pack, unpack)")
+                       "one launch that fills the transfer buffer and the destination pages)")
     return out
 
 

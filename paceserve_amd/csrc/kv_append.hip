@@ -24,12 +24,14 @@
 //
 // Bound by HBM from some 16 MiB up, and below by the launch and by the chain
 // of two to four dependent index loads.  Measured on MI355X per launch in a
-// graph, fused form, against one wave per K or V row (or 16 KiB of it):
-//   256-byte rows, 16384 tokens               4.35 us, before 8.1
-//   384-byte rows, about 8500 tokens          5.2 us, before 8.4
-//   2 KiB rows, about 8500 tokens             15.5 us, before 17.0
-//   2 KiB rows, 256 tokens of a decode step   2.4 us, before 2.9
-//   8 KiB rows, 8190 tokens                   46 us, before 50 (the other form)
+// graph of 32 on the same buffers (up to 64 MiB partly from the memory-side
+// cache), fused form and the other, against one wave per K or V row (or 16 KiB):
+//   256-byte rows, 16384 tokens               3.9, 3.4 us, before 10.7, 8.9
+//   256-byte rows, 32768 tokens               5.3, 4.7 us, before 19.4, 16.0
+//   384-byte rows, 8500 tokens                3.8, 3.3 us, before 6.7, 5.7
+//   2 KiB rows, 8500 tokens                   10.9, 11.3 us, before 12.7, 11.5
+//   2 KiB rows, 256 tokens of a decode step   1.96, 2.28 us, before 2.41, 2.34
+//   8 KiB rows, 8190 tokens                   39.6, 39.3 us, before 40.5, 40.2
 // Launches of up to 300 tokens with rows of less than a KiB, 2.1 to 2.3 us, are
 // up to 0.06 us slower than that.
 // Waves that end with a row (idle lanes, scalar indices) never measured

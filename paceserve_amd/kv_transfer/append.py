@@ -99,8 +99,8 @@ def _append_shape(append_key: torch.Tensor, append_value: torch.Tensor, paged_kv
     """(P, H, D, GPU index) of an append.  One look at each property settles an
     append that is in order; any other gets _check_append's checks, one by
     one, and its message.  A small append takes less time on the GPU than in
-    Python: an eager launch of 16 MiB of 256-byte rows, 4.4 us there, goes from
-    10.7 to 9.3 us."""
+    Python: an eager launch of 32768 tokens with 256-byte rows, 5.3 us there,
+    goes from 10.7 to 9.3 us."""
     if kv_layout == "NHD" and type(paged_kv_cache) is type(append_key) is type(append_value) is torch.Tensor:
         index, shape, rows, stride = (paged_kv_cache.get_device(), paged_kv_cache.shape, append_key.shape,
                                       append_key.stride())

@@ -8,8 +8,9 @@ One promote() call:
      (base_worker.py:255-262), all-or-nothing for the batch;
   2. remaps positionally, dropping a trailing extra destination page (the n vs
      n+1 rule, base_worker.py:264-277);
-  3. uploads both id lists (CSR-concatenated over requests) with one pinned
-     host-to-device copy;
+  3. hands both id lists (CSR-concatenated over requests) to the GPU: up to 512
+     pages travel in the kernel arguments, more with one pinned host-to-device
+     copy;
   4. moves the pages in one of three modes:
        "buffer": pack into a device transfer buffer and unpack out of it - the
                  reference's two-step semantics, in one launch that reads each
