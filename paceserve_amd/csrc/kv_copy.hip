@@ -295,10 +295,10 @@ const void* inline_kernel_of(Kind kind, InlineSides sides) {
 // them.
 //
 // Bound by the link (56-57 GB/s per direction), so what counts is to keep
-// enough of it in flight with few waves: the rest of the chip stays free for
-// whatever other streams run, and more waves slow the other direction's
-// traffic.  Each lane keeps UNROLL vectors in flight and loads the next round's
-// ids behind them.  Measured on MI355X at 14 and 56 MiB, by workgroups of 256:
+// enough of it in flight with few waves: the rest of the chip's CUs stay free
+// for other streams, and more waves slow the other direction's traffic.  Each
+// lane keeps UNROLL vectors in flight and loads the next round's ids behind
+// them.  Measured on MI355X at 14 and 56 MiB, by workgroups of 256:
 //   out, 16 vectors   4: 54.5 and 56.2 GB/s, 6 to 12 within 2% either way
 //                     (short pages 4: 16 MiB of 160 B 341 us, of 400 B 326;
 //                     8: 310 and 309)
@@ -307,6 +307,12 @@ const void* inline_kernel_of(Kind kind, InlineSides sides) {
 // Beside host-to-device DMA copies 4 workgroups out keep 48.6 GB/s per
 // direction, 32 workgroups 44; a read stream by waves beside a write stream
 // falls to 28, so only short copies read the host this way.
+// What other streams run meanwhile is slowed by more than those CUs: 1 GiB HBM
+// copies for 6.05 ms, or bf16 matrix products for 11.3 ms, take 6.9 and 12.7 ms
+// beside two legs out of 56 MiB (the same beside a pack and a copy kernel), 7.6
+// and 12.7 beside two legs in (6.1 and 11.4 beside two DMA copies in, which take
+// 1.065 ms each against 1.035), and 7.4 to 7.7 and 12.7 beside two swaps (8.1
+// and 13.1 to 13.3 by the page copy).
 constexpr int kHostThreads = 256;
 constexpr int kOutGroups = 4, kOutUnroll = 16;
 constexpr int kInGroups = 16, kInUnroll = 8;
