@@ -226,7 +226,8 @@ def run_device(args, w, dev, src, dst, plan, s_ids, d_ids):
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": None,
-            "kernel": copy_kernel_names(args.mode, w.shape.page_bytes),
+            "kernel": copy_kernel_names(args.mode, w.shape.page_bytes,
+                                        int(statistics.mean(bytes_per_launch)) // 2),
             "algorithmic_bytes_per_launch": int(statistics.mean(bytes_per_launch)),
             # page ids read per launch (one int32 per page; not in `achieved`)
             "block_table_bytes_per_launch": 4 * n,
@@ -245,23 +246,23 @@ SHAPES = ("kPow2", "kRows", "kSpanFlat", "kLaneFlat", "kOnePage")
 KINDS = ("kStream", "kPack", "kTee")
 
 
-def copy_shape(page_bytes: int, both_indexed: bool) -> str:
+def copy_shape(page_bytes: int, scalar_ids: bool) -> str:
     """How a launch splits its pages over waves: the rule of enum Shape in
-    csrc/kv_copy.hip."""
+    csrc/kv_copy.hip.  scalar_ids: a move, or a pack of up to 64 MiB."""
     if page_bytes % 1024 == 0:
         rows = page_bytes // 1024
         return "kPow2" if rows & (rows - 1) == 0 else "kRows"
-    return "kSpanFlat" if both_indexed and page_bytes >= 336 else "kLaneFlat"
+    return "kSpanFlat" if scalar_ids and page_bytes >= 336 else "kLaneFlat"
 
 
-def copy_kernel_names(mode: str, page_bytes: int) -> str:
+def copy_kernel_names(mode: str, page_bytes: int, launch_bytes: int) -> str:
     """The page_copy_kernel instances a step launches (template arguments
-    Shape, Kind)."""
+    Shape, Kind); launch_bytes: payload of one launch."""
     if mode == "fused":
         return f"page_copy_kernel<{copy_shape(page_bytes, True)}, kStream> (move, streaming write-through stores)"
-    shape = copy_shape(page_bytes, False)
-    return (f"page_copy_kernel<{shape}, kPack> (pack, write-through stores) and "
-            f"page_copy_kernel<{shape}, kStream> (unpack, streaming write-through stores)")
+    return (f"page_copy_kernel<{copy_shape(page_bytes, launch_bytes <= 64 << 20)}, kPack> (pack, write-through "
+            f"stores) and page_copy_kernel<{copy_shape(page_bytes, False)}, kStream> (unpack, streaming "
+            "write-through stores)")
 
 
 def short_kernel_name(name: str) -> str:

@@ -81,29 +81,29 @@ enum Kind { kStream = 0, kPack = 1, kTee = 2 };
 // lane carries a vector and a wave may hold several pages, or the end of one
 // and the start of the next: each lane loads its own page's ids (kLaneFlat), or
 // the wave loads the at most kSpan ids per side that its lanes choose from by
-// scalar loads (kSpanFlat, ids on both sides and pages of at least kSpanVecs
-// vectors: 336 bytes).
+// scalar loads (kSpanFlat: pages of at least kSpanVecs vectors, 336 bytes, with
+// ids on both sides, or packs of up to kSpanPackBytes a launch).
 // Measured on MI355X, 32 layers, 150 MiB, against waves that end with a page:
 //   move    160 B 210 -> 103 us, 256 B 132 -> 52, 512 B 67.4 -> 50.3, 1280 B
 //           57 -> 50, 1536 B 53.7 -> 49.8, the same from 2560 B on
 //   pack    160 B 210 -> 60, 512 B 67 -> 46, 1280 B 54.5 -> 46.3, 1536 B and
 //           more the same or up to 2% faster
 //   unpack  160 B 210 -> 85, 512 B 67.5 -> 48.9, 1280 B 56.4 -> 48.8
-// and on 6 MiB in a graph, 512 B: move 4.3 -> 3.2 us, pack 4.3 -> 3.4, unpack
-// 4.3 -> 3.2.  Below 2.5 MiB, where a launch takes 1.9 to 2.6 us: moves from 10%
-// faster to 4% slower (the same to 512 KiB), unpacks from 15% faster to 5%
-// slower, packs from 10% faster (0.5 to 1 MiB) to 0.25 us or 12% slower: 1.25 to
-// 2 MiB of pages of 640 bytes and more, whose time steps up past 1024 waves
-// where waves that end with a page step past 2048.
+// and on 6 MiB in a graph, 512 B: move 4.3 -> 3.2 us, pack 4.3 -> 3.3, unpack
+// 4.3 -> 3.2.  Below 2.5 MiB, where a launch takes 1.9 to 2.6 us, moves and packs
+// are from 13% faster to 4% slower, unpacks from 15% faster to 5% slower.
 // A move by lanes' own ids is 3-4% slower than by scalar ids (its id loads go
-// ahead of the page's in one chain); a pack or unpack by scalar ids is 4-8%
-// slower at 150 MiB (the contiguous side needs no id).
+// ahead of the page's in one chain).  A pack by lanes' own ids is slower up to
+// 64 MiB (kSpanPackBytes; 1.75 MiB of 1536 B 2.46 against 2.24 us, 2.24 by waves
+// that end with a page; 48 MiB 3 to 17% and 64 MiB 0 to 10%) and 1 to 5% faster from 96 MiB
+// on; an unpack by scalar ids, its eight waits as below, was 4-8% slower at 150 MiB.
 // Across the host link what counts is the number of pieces in which pages
 // travel: pages of up to kLinkPageBytes go one to a wave (kOnePage).
 // Measured on MI355X, swaps of 8 MiB against waves end to end: 160 B out 167
 // against 176 us, in 250 against 304; 400 B 159 against 167 and 192 against 234.
 enum Shape { kPow2 = 0, kRows = 1, kSpanFlat = 2, kLaneFlat = 3, kOnePage = 4 };
 constexpr int kLinkPageBytes = 512;
+constexpr int64_t kSpanPackBytes = 64 << 20;
 constexpr int kSpan = 4;
 constexpr int kSpanVecs = kThreads / (kSpan - 1);
 
@@ -192,14 +192,19 @@ __device__ __forceinline__ void copy_row(const CopyParams& p, const int32_t* sid
     const uint32_t j0 = over(p.by_page, g0), last = p.n_pages - 1;
     const uint32_t j1 = min(j0 + 1, last), j2 = min(j0 + 2, last), j3 = min(j0 + 3, last);
     int32_t s0 = sids[j0], s1 = sids[j1], s2 = sids[j2], s3 = sids[j3];
-    int32_t d0 = dids[j0], d1 = dids[j1], d2 = dids[j2], d3 = dids[j3];
-    asm("" : "+s"(s0), "+s"(s1), "+s"(s2), "+s"(s3), "+s"(d0), "+s"(d1), "+s"(d2), "+s"(d3));
+    int32_t d0 = 0, d1 = 0, d2 = 0, d3 = 0;
+    if (KIND == kPack) {
+      asm("" : "+s"(s0), "+s"(s1), "+s"(s2), "+s"(s3));
+    } else {
+      d0 = dids[j0], d1 = dids[j1], d2 = dids[j2], d3 = dids[j3];
+      asm("" : "+s"(s0), "+s"(s1), "+s"(s2), "+s"(s3), "+s"(d0), "+s"(d1), "+s"(d2), "+s"(d3));
+    }
     vec = g0 - j0 * p.page_vecs + threadIdx.x;
     const bool past1 = vec >= p.page_vecs, past2 = vec >= 2 * p.page_vecs, past3 = vec >= 3 * p.page_vecs;
     j = j0 + past1 + past2 + past3;
     vec -= past3 ? 3 * p.page_vecs : past2 ? 2 * p.page_vecs : past1 ? p.page_vecs : 0;
     sp = static_cast<uint32_t>(past3 ? s3 : past2 ? s2 : past1 ? s1 : s0);
-    dp = static_cast<uint32_t>(past3 ? d3 : past2 ? d2 : past1 ? d1 : d0);
+    dp = KIND == kPack ? j : static_cast<uint32_t>(past3 ? d3 : past2 ? d2 : past1 ? d1 : d0);
   } else if (SHAPE == kLaneFlat) {
     const uint32_t g = x * kThreads + threadIdx.x;
     if (g >= p.total_vecs) return;
@@ -424,9 +429,7 @@ const void* pick_kernel(Shape shape, Kind kind) {
     case kOnePage: return reinterpret_cast<const void*>(&page_copy_kernel<kOnePage, kStream>);
     case kPow2: return kernel_of<kPow2>(kind);
     case kRows: return kernel_of<kRows>(kind);
-    case kSpanFlat:  // a move or a tee
-      return kind == kTee ? reinterpret_cast<const void*>(&page_copy_kernel<kSpanFlat, kTee>)
-                          : reinterpret_cast<const void*>(&page_copy_kernel<kSpanFlat, kStream>);
+    case kSpanFlat: return kernel_of<kSpanFlat>(kind);  // a move, a tee or a small pack
     default: return kernel_of<kLaneFlat>(kind);
   }
 }
@@ -436,8 +439,11 @@ const void* pick_inline_kernel(Shape shape, Kind kind, InlineSides sides) {
     case kPow2: return inline_kernel_of<kPow2>(kind, sides);
     case kRows: return inline_kernel_of<kRows>(kind, sides);
     case kSpanFlat:
-      return kind == kTee ? reinterpret_cast<const void*>(&page_copy_inline_kernel<kSpanFlat, kTee, true, true>)
-                          : reinterpret_cast<const void*>(&page_copy_inline_kernel<kSpanFlat, kStream, true, true>);
+      switch (kind) {
+        case kPack: return reinterpret_cast<const void*>(&page_copy_inline_kernel<kSpanFlat, kPack, true, false>);
+        case kTee: return reinterpret_cast<const void*>(&page_copy_inline_kernel<kSpanFlat, kTee, true, true>);
+        default: return reinterpret_cast<const void*>(&page_copy_inline_kernel<kSpanFlat, kStream, true, true>);
+      }
     default: return inline_kernel_of<kLaneFlat>(kind, sides);
   }
 }
@@ -521,7 +527,10 @@ int launch_page_copy(const Side& src, const Side& dst, int num_layers, int64_t n
   uint32_t rows_log2 = 0;
   while ((int64_t(1) << rows_log2) < rows_per_page) ++rows_log2;
   const bool whole_rows = page_bytes % kRowBytes == 0;
-  const bool span = page_bytes >= kSpanVecs * kVecBytes && src_indexed && dst_indexed && policy != StorePolicy::kPack;
+  const bool small_pack = policy == StorePolicy::kPack && src_indexed && !dst_indexed &&
+                          n_pages <= kSpanPackBytes / page_bytes / std::min(num_layers, kMaxLayers);
+  const bool span = page_bytes >= kSpanVecs * kVecBytes &&
+                    ((src_indexed && dst_indexed && policy != StorePolicy::kPack) || small_pack);
   const bool one_page =
       policy == StorePolicy::kLink && page_bytes <= kLinkPageBytes && !inline_ids && tee == nullptr;
   const Shape shape = whole_rows ? ((int64_t(1) << rows_log2) == rows_per_page ? kPow2 : kRows)

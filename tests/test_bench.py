@@ -28,15 +28,17 @@ def write_csv(path, rows):
 
 
 def test_copy_kernel_names_follow_the_store_policy():
-    names = bench.copy_kernel_names("buffer", 65536)
+    names = bench.copy_kernel_names("buffer", 65536, 1 << 30)
     assert "page_copy_kernel<kPow2, kPack> (pack, write-through stores)" in names
     assert "page_copy_kernel<kPow2, kStream> (unpack" in names
     # 96, 352 and 1040 B: end to end, by lanes' or the wave's ids; 3 KiB: three rows
-    assert bench.copy_kernel_names("fused", 352).startswith("page_copy_kernel<kSpanFlat, kStream>")
-    assert bench.copy_kernel_names("fused", 96).startswith("page_copy_kernel<kLaneFlat, kStream> (move")
-    assert bench.copy_kernel_names("fused", 1040).startswith("page_copy_kernel<kSpanFlat, kStream>")
-    assert bench.copy_kernel_names("buffer", 1040).startswith("page_copy_kernel<kLaneFlat, kPack>")
-    assert bench.copy_kernel_names("fused", 3072).startswith("page_copy_kernel<kRows, kStream>")
+    assert bench.copy_kernel_names("fused", 352, 1 << 30).startswith("page_copy_kernel<kSpanFlat, kStream>")
+    assert bench.copy_kernel_names("fused", 96, 1 << 30).startswith("page_copy_kernel<kLaneFlat, kStream> (move")
+    assert bench.copy_kernel_names("fused", 1040, 1 << 30).startswith("page_copy_kernel<kSpanFlat, kStream>")
+    large, small = (bench.copy_kernel_names("buffer", 1040, n) for n in (1 << 30, 1 << 20))
+    assert large.startswith("page_copy_kernel<kLaneFlat, kPack>") and "<kLaneFlat, kStream>" in large
+    assert small.startswith("page_copy_kernel<kSpanFlat, kPack>") and "<kLaneFlat, kStream>" in small
+    assert bench.copy_kernel_names("fused", 3072, 1 << 30).startswith("page_copy_kernel<kRows, kStream>")
 
 
 def test_kernel_names_are_the_library_s():
@@ -50,7 +52,8 @@ def test_kernel_names_are_the_library_s():
     lib = (ROOT / "paceserve_amd" / "libpace_kv.so").read_bytes()
     for mode in ("buffer", "fused"):
         for page_bytes in (96, 512, 1040, 3072, 65536):
-            for shape, kind in re.findall(r"page_copy_kernel<(\w+), (\w+)>", bench.copy_kernel_names(mode, page_bytes)):
+            names = bench.copy_kernel_names(mode, page_bytes, 1 << 20) + bench.copy_kernel_names(mode, page_bytes, 1 << 30)
+            for shape, kind in re.findall(r"page_copy_kernel<(\w+), (\w+)>", names):
                 mangled = f"page_copy_kernelILNS0_5ShapeE{bench.SHAPES.index(shape)}ELNS0_4KindE{bench.KINDS.index(kind)}E"
                 assert mangled.encode() in lib, (mode, page_bytes, shape, kind)
 

@@ -68,6 +68,22 @@ def test_pack_unpack_move(gpu, page_bytes, n, bad):
     assert int(err.item()) == L * (n - len(ok))
 
 
+@pytest.mark.parametrize("n", [31775, 31776])        # the last pack by scalar ids, and the first by lanes' own
+def test_packs_around_64_mib(gpu, n):
+    L, page_bytes = 2, 1056
+    gen = torch.Generator().manual_seed(n)
+    src, src_l = pool(L, n + 5, page_bytes, gen, gpu)
+    ids = torch.randperm(n + 5, generator=gen)[:n]
+    ids[0], ids[n - 1] = -1, n + 5
+    buf = torch.zeros((L, n) + tuple(src.shape[2:]), dtype=torch.uint8, device=gpu).view(torch.float8_e4m3fn)
+    err = torch.zeros(1, dtype=torch.int32, device=gpu)
+    ops.pack(src_l, ids.to(torch.int32).to(gpu), buf, err=err)
+    want = torch.zeros((L, n) + tuple(src.shape[2:]), dtype=torch.uint8, device=gpu)
+    want[:, 1:-1] = src[:, ids[1:-1].to(gpu)]
+    assert torch.equal(buf.view(torch.uint8), want)
+    assert int(err.item()) == 2 * L
+
+
 @pytest.mark.parametrize("mode", ["fused", "buffer"])
 @pytest.mark.parametrize("n", [1, 33, 512, 513])     # up to 512 ids travel in the kernel arguments
 @pytest.mark.parametrize("page_bytes", PAGE_BYTES)
